@@ -33,7 +33,7 @@ template <bool BWD, typename In, bool MIX, int NBUF>
 __global__ void states_kernel(Dims, StateArgs);
 template <typename In, bool MIX, bool STORE, int PAIRS>
 __global__ void fwd_factor_kernel(Dims, const In*, const In*, const float*, const float*,
-                                  const float*, const float*, float*, float*, MixerIn, int);
+                                  const float*, const float*, float*, float*, MixerIn, int, int);
 __global__ void factored_solve_kernel(const float*, const float*, float*, long);
 __global__ void decode_step_kernel(float*, float*, const float*, const float*, const float*,
                                    const float*, const float*, const float*, long, int, int, float*,
@@ -284,6 +284,38 @@ int turn_polls() {
   return 1 << 16;
 }
 
+// How many spans of tokens each sub-chunk is split into for the factor
+// kernel (the spans after the first bring the start evidence up to their own
+// first token, stage_evidence).  A pair walks its span two tokens a pass, a
+// chain that few sequences leave most of the chip waiting for (B1 T512 H8:
+// 188 us in one span, 32 in sixteen), while a full chip only pays the extra
+// updates (B16 T1024 H8: 308 us in one, 324 in two).  A finer split is taken
+// where it is estimated at least 5% faster (the estimate's own error: B16
+// T1024 H12 is a tie).  The estimate adds up
+// rounds of pairs, in microseconds as measured for spans of 2 to 32 tokens
+// from 2 to 12,288 sub-chunks: a round takes 6, and with one wave per SIMD (up
+// to two pairs per compute unit) 11.4 a pass and 0.42 a caught-up token, with
+// two waves 18 and 1.
+int factor_spans(long subseqs, int sub) {
+  int best = 1;
+  double best_us = 0.0;
+  for (int nspan = 1; nspan <= 16 && nspan <= sub; nspan *= 2) {
+    const int span = (sub + nspan - 1) / nspan, passes = (span + 1) / 2;
+    const double catchup = (double)(nspan - 1) * span;  // of the last span; half on average
+    const long pairs = (subseqs * nspan + 3) / 4, full = 4L * g_cus, rest = pairs % full;
+    double us = (double)(pairs / full) * (6.0 + 18.0 * passes + 0.5 * catchup);
+    if (rest > full / 2)
+      us += (0.9 + 0.1 * (2.0 * rest / full - 1.0)) * (6.0 + 18.0 * passes + catchup);
+    else if (rest > 0)
+      us += 6.0 + 11.4 * passes + 0.42 * catchup;
+    if (nspan == 1 || us < 0.95 * best_us) {
+      best = nspan;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 bool bad_dims(int B, int T, int H, int P, int chunk, std::string* why) {
   if (B <= 0 || T <= 0 || H <= 0) {
     *why = "B, T and H must be positive";
@@ -422,17 +454,19 @@ int forward_impl(const char* entry, const In* keys, const In* values, const In* 
   if (rc) return rc;
   const int polls = turn_polls();
   rc = launch("fwd_factor", st, [&] {
-    // Four sub-chunk sequences per wave pair; four pairs per block when those
-    // blocks fill the chip in whole rounds (one resident per CU), else two.
-    const unsigned blocks4 = (subseqs + 15) / 16;
+    // Four spans per wave pair; four pairs per block when those blocks fill
+    // the chip in whole rounds (one resident per CU), else two.
+    const int nspan = factor_spans(subseqs, d.sub);
+    const unsigned spans = subseqs * nspan;
+    const unsigned blocks4 = (spans + 15) / 16;
     const int pairs = blocks4 % (unsigned)g_cus == 0 ? 4 : 2;
-    const dim3 grid((subseqs + 4 * pairs - 1) / (4 * pairs)), block(128 * pairs);
+    const dim3 grid((spans + 4 * pairs - 1) / (4 * pairs)), block(128 * pairs);
     const auto kernel = factors ? (pairs == 4 ? m4::fwd_factor_kernel<In, MIX, true, 4>
                                               : m4::fwd_factor_kernel<In, MIX, true, 2>)
                                 : (pairs == 4 ? m4::fwd_factor_kernel<In, MIX, false, 4>
                                               : m4::fwd_factor_kernel<In, MIX, false, 2>);
     hipLaunchKernelGGL(kernel, grid, block, 0, st, d, keys, queries, beta, log_decay, floor,
-                       start_evidence, solved, factors, mix, polls);
+                       start_evidence, solved, factors, mix, polls, nspan);
   });
   if (rc) return rc;
   return launch("fwd_read", st, [&] {

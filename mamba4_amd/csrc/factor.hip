@@ -125,6 +125,112 @@ __device__ __forceinline__ void raise_count(lds_int* count, int v) {
                          __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// Tokens whose inputs stage_evidence loads together.
+constexpr int CATCHUP_GROUP = 4;
+
+// The 16x16 blocks (I, K) of the lower triangle that wave W of a pair stages
+// (five each), as f(i, I, K).
+template <int W, typename F>
+__device__ __forceinline__ void for_staged_blocks(F&& f) {
+  int i = 0;
+#pragma unroll
+  for (int I = 0; I < 4; ++I)
+#pragma unroll
+    for (int K = 0; K <= I; ++K)
+      if (W == (I == 3 || (I == 2 && K == 2))) f(i++, I, K);
+}
+
+__device__ __forceinline__ float row_value(float x, int mu) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 16 * mu));
+}
+
+// Wave W's half of the evidence that its pair's spans start from, to LDS: the
+// sub-chunks' start states times -c, then the rank-one updates of the
+// `catchup` tokens before each span (per 16-lane row; the first is sequence
+// token `first`).  A token's update is the turn's, a product by the decay and
+// one multiply-add, here on the rank-one four-block fp32 MFMA over blocks in
+// the exchanged layout (rows16.hpp), so a token's evidence is the same to the
+// bit however its sub-chunk is split.  Per wave and token 80 multiplies and
+// five MFMAs; on DPP-fed multiply-adds in the row layout (224 instructions)
+// a token took 0.75 us; it takes 0.42.
+template <typename In, bool MIX, int W>
+__device__ __forceinline__ void stage_evidence(f4* evidence, const float* start_s, int slot,
+                                               float c, int sexp, int catchup, int first,
+                                               const Dims& d, const In* keys, const float* beta,
+                                               const float* log_decay, const MixerIn& mix, int b,
+                                               int h) {
+  const int lane = threadIdx.x & 63, a = lane & 15, g = lane >> 4;
+  f16 E[5];
+#pragma unroll
+  for (int mu = 0; mu < 4; ++mu) {
+    const float* s0 = start_s + (long)__builtin_amdgcn_readlane(slot, 16 * mu) * 4096;
+    const float nc = -row_value(c, mu);
+    for_staged_blocks<W>([&](int i, int I, int K) {
+      const f4 v = *reinterpret_cast<const f4*>(s0 + (16 * I + a) * 64 + 16 * K + 4 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) E[i][4 * mu + e] = nc * v[e];
+    });
+  }
+  const int most = wave_max4(catchup);
+  // A group's inputs are in flight while the previous group is applied.  Rows
+  // without a token to catch up read one in bounds and take a zero update.
+  TokenInputs cur[CATCHUP_GROUP], next[CATCHUP_GROUP];
+  bool kzero[CATCHUP_GROUP] = {};
+  auto load = [&](TokenInputs (&in)[CATCHUP_GROUP], int from) {
+#pragma unroll
+    for (int j = 0; j < CATCHUP_GROUP; ++j) {
+      const int t = from + j < catchup ? first + from + j : 0;
+      if constexpr (MIX)
+        load_token_mix(in[j], kzero[j], d, mix, beta, log_decay, b, h, t, a);
+      else
+        load_token(in[j], d, keys, keys, beta, log_decay, b, h, t, a);
+    }
+  };
+  if (most > 0) load(cur, 0);
+  for (int from = 0; from < most; from += CATCHUP_GROUP) {
+    if constexpr (MIX)
+#pragma unroll
+      for (int j = 0; j < CATCHUP_GROUP; ++j) mix_token(cur[j], kzero[j]);
+    load(next, from + CATCHUP_GROUP);
+#pragma unroll
+    for (int j = 0; j < CATCHUP_GROUP; ++j) {
+      const bool in = from + j < catchup;
+      const float lam = in ? expf(cur[j].log_lam) : 1.f;
+      const float cbeta = __builtin_ldexpf(cur[j].beta, 2 * sexp);
+      float k[4], nbk[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        k[m] = in ? cur[j].k[m] : 0.f;
+        nbk[m] = in ? -cbeta * cur[j].k[m] : 0.f;
+      }
+#pragma unroll
+      for (int mu = 0; mu < 4; ++mu) {
+        const float l = row_value(lam, mu);
+        for_staged_blocks<W>([&](int i, int, int) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) E[i][4 * mu + e] *= l;
+        });
+      }
+      for_staged_blocks<W>([&](int i, int I, int K) {
+        E[i] = __builtin_amdgcn_mfma_f32_16x16x1f32(k[K], nbk[I], E[i], 0, 0, 0);
+      });
+    }
+#pragma unroll
+    for (int j = 0; j < CATCHUP_GROUP; ++j) cur[j] = next[j];
+  }
+  for_staged_blocks<W>([&](int i, int I, int K) {
+#pragma unroll
+    for (int mu = 0; mu < 4; ++mu)
+      evidence[slot_quad(I, 4 * K + g) * 64 + 16 * mu + a] =
+          f4{E[i][4 * mu], E[i][4 * mu + 1], E[i][4 * mu + 2], E[i][4 * mu + 3]};
+  });
+}
+
+// A sequence is a span of a sub-chunk's tokens, 1/nspan of it (the launch
+// chooses nspan so that few sub-chunks still fill the chip): its pair first
+// brings the sub-chunk's start evidence to the span's first token
+// (stage_evidence).
+//
 // Two waves share the four sequences of a pair and take alternate tokens:
 // wave w factors tokens base+w for base = 0, 2, 4, ...  The running evidence
 // lives in LDS; each wave in its turn reads it, applies its token's rank-one
@@ -160,21 +266,22 @@ __global__ __launch_bounds__(128 * PAIRS) void fwd_factor_kernel(
     Dims d, const In* __restrict__ keys, const In* __restrict__ queries,
     const float* __restrict__ beta, const float* __restrict__ log_decay,
     const float* __restrict__ floor, const float* __restrict__ start_s,
-    float* __restrict__ solved, float* __restrict__ factors, MixerIn mix, int polls) {
+    float* __restrict__ solved, float* __restrict__ factors, MixerIn mix, int polls, int nspan) {
   const int lane = threadIdx.x & 63, a = lane & 15, mu = lane >> 4;
   const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int pair = wave8 >> 1, wave = wave8 & 1;
   const int BH = d.B * d.H;
-  const long nseq = (long)BH * d.NS;
+  const long nseq = (long)BH * d.NS * nspan;
   long seq = ((long)blockIdx.x * PAIRS + pair) * 4 + mu;
   const bool active = seq < nseq;
   if (!active) seq = nseq - 1;
-  // Sequences are ordered sub-chunk-major, so a wave's four rows share the
-  // sub-chunk index and read neighbouring heads.
-  const int ns = (int)(seq / BH), bh = (int)(seq % BH), b = bh / d.H, h = bh % d.H;
-  const int n = ns / d.rsub, u = ns % d.rsub;
-  const int len = active ? sub_len(d, n, u) : 0;
-  const int t0 = n * d.chunk + sub_first(d, u);
+  // Sequences are ordered sub-chunk-major (then by span), so a wave's four
+  // rows share the span and read neighbouring heads.
+  const int nsp = (int)(seq / BH), bh = (int)(seq % BH), b = bh / d.H, h = bh % d.H;
+  const int ns = nsp / nspan, n = ns / d.rsub, u = ns % d.rsub;
+  const int span = (d.sub + nspan - 1) / nspan, off = (nsp - ns * nspan) * span;
+  const int len = active ? max(min(span, sub_len(d, n, u) - off), 0) : 0;
+  const int t0 = n * d.chunk + sub_first(d, u) + off;
   const int steps = wave_max4(len);
 
   // The running evidence, negated (the factorization's working convention).
@@ -202,24 +309,16 @@ __global__ __launch_bounds__(128 * PAIRS) void fwd_factor_kernel(
   const float c = __builtin_ldexpf(1.f, 2 * sexp);
 #pragma unroll
   for (int m = 0; m < 4; ++m) fl[m] *= c;
-  {
-    // Both waves of the pair stage the start evidence: wave 0 slots 0..2 (24 quads),
-    // wave 1 slot 3 (16 quads).
-    const float* s0 = start_s + ((long)bh * d.NS + ns) * 4096;
-    if (wave == 0) {
-#pragma unroll
-      for (int m = 0; m < 3; ++m)
-#pragma unroll
-        for (int q = 0; q < 4 * m + 4; ++q)
-          evidence[slot_quad(m, q) * 64 + lane] =
-              -c * *reinterpret_cast<const f4*>(s0 + (a + 16 * m) * 64 + 4 * q);
-      if (lane == 0) *turn_count = 0;  // after this lane's quad (0, 3): LDS writes stay in order
-    } else {
-#pragma unroll
-      for (int q = 0; q < 16; ++q)
-        evidence[slot_quad(3, q) * 64 + lane] =
-            -c * *reinterpret_cast<const f4*>(s0 + (a + 48) * 64 + 4 * q);
-    }
+  // Both waves of the pair stage the start evidence, brought to the span's
+  // first token.
+  const int catchup = len > 0 ? off : 0;
+  if (wave == 0) {
+    stage_evidence<In, MIX, 0>(evidence, start_s, bh * d.NS + ns, c, sexp, catchup, t0 - off, d,
+                               keys, beta, log_decay, mix, b, h);
+    if (lane == 0) *turn_count = 0;  // after the wave's quad (0, 3): LDS writes stay in order
+  } else {
+    stage_evidence<In, MIX, 1>(evidence, start_s, bh * d.NS + ns, c, sexp, catchup, t0 - off, d,
+                               keys, beta, log_decay, mix, b, h);
   }
   // Rows past their sequence read token 0 (in bounds; never stored).
   auto token = [&](int tt) { return tt < len ? t0 + tt : 0; };
@@ -246,7 +345,7 @@ __global__ __launch_bounds__(128 * PAIRS) void fwd_factor_kernel(
     const bool valid = tt < len;  // per 16-lane row
     float A[4][64];
     const int seen = wait_turn(turn_count, tt, polls);
-    const bool gave_up = seen < tt || (polls < 0 && tt > 0);
+    const bool gave_up = seen < tt || (polls < 0 && off + tt > 0);
     if (gave_up && lane == 0) raise_count(turn_count, kPoisoned);
     const float lam = gave_up || seen >= kPoisoned ? __builtin_nanf("") : expf(cur.log_lam);
     const float cbeta = __builtin_ldexpf(cur.beta, 2 * sexp);
@@ -258,8 +357,11 @@ __global__ __launch_bounds__(128 * PAIRS) void fwd_factor_kernel(
         f4 sv = evidence[slot_quad(m, q) * 64 + lane];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+          // The product by the decay rounded, then one multiply-add:
+          // stage_evidence's MFMA updates round the same way.
+#pragma clang fp contract(off)
           const int k = 4 * q + e;
-          sv[e] = lam * sv[e] + nbk * bcast16(cur.k[k >> 4], k & 15);
+          sv[e] = __builtin_fmaf(nbk, bcast16(cur.k[k >> 4], k & 15), lam * sv[e]);
           A[m][k] = sv[e];
         }
         if (m != 0 || q != 3 || lane != 0) evidence[slot_quad(m, q) * 64 + lane] = sv;
@@ -326,10 +428,10 @@ __global__ __launch_bounds__(128 * PAIRS) void fwd_factor_kernel(
 #define M4_FWD_FACTOR(IN, MIX, STORE)                                                      \
   template __global__ void fwd_factor_kernel<IN, MIX, STORE, 4>(                           \
       Dims, const IN*, const IN*, const float*, const float*, const float*, const float*, \
-      float*, float*, MixerIn, int);                                                       \
+      float*, float*, MixerIn, int, int);                                                       \
   template __global__ void fwd_factor_kernel<IN, MIX, STORE, 2>(                           \
       Dims, const IN*, const IN*, const float*, const float*, const float*, const float*, \
-      float*, float*, MixerIn, int);
+      float*, float*, MixerIn, int, int);
 M4_FWD_FACTOR(float, false, true)
 M4_FWD_FACTOR(bf16_t, false, true)
 M4_FWD_FACTOR(float, true, true)
