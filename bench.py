@@ -401,8 +401,9 @@ MIXER_KERNELS = {
     "prologue_backward": ["prologue_backward", "head_sums"],
     "epilogue_forward": ["epilogue_forward"],
     "epilogue_backward": ["epilogue_backward", "head_sums"],
-    "order_forward": ["order_local", "order_carry", "order_apply"],
-    "order_backward": ["order_bwd_local", "order_bwd_carry", "order_bwd_apply"],
+    "order_forward": ["order_walk", "order_local", "order_carry", "order_apply"],
+    "order_backward": ["order_bwd_walk", "order_bwd_local", "order_bwd_carry",
+                       "order_bwd_apply"],
 }
 
 

@@ -78,6 +78,9 @@ __global__ void order_bwd_local_kernel(OrderDims, const float*, const float*, fl
 __global__ void order_bwd_carry_kernel(OrderDims, float*, const float*, float*);
 __global__ void order_bwd_apply_kernel(OrderDims, const float*, const float*, const float*,
                                        const float*, const float*, const float*, float*, float*);
+__global__ void order_walk_kernel(OrderDims, const float*, const float*, const float*, float*);
+__global__ void order_bwd_walk_kernel(OrderDims, const float*, const float*, const float*,
+                                      const float*, const float*, float*, float*, float*);
 __global__ void spd_solve_kernel(const float*, const float*, long, int, float*, float*);
 __global__ void spd_backward_kernel(const float*, const float*, const float*, long, int, float*,
                                     float*);
@@ -104,7 +107,7 @@ const char* const kKernelNames[] = {"fwd_stats",      "fwd_scan",  "fwd_states",
                                     "prologue_backward", "epilogue_forward",
                                     "epilogue_backward", "head_sums", "order_local",
                                     "order_carry",    "order_apply", "order_bwd_local",
-                                    "order_bwd_carry", "order_bwd_apply",
+                                    "order_bwd_carry", "order_bwd_apply", "order_walk", "order_bwd_walk",
                                     "m3_walk",        "m3_out",    "m3_walk_bwd", "m3_grad",
                                     "m3_finish",      "m3_bias",   "m3_suffix",
                                     "mixer_finish",   "diag_eigen", "diag_summary",
@@ -1282,6 +1285,30 @@ size_t order_workspace(const m4::OrderDims& d, float** states, float** totals, v
 
 unsigned order_threads(int W) { return (unsigned)(64 * ((W + 63) / 64)); }
 
+// Waves of a one-pass order block: columns of 64 channels times runs of 32
+// tokens, up to sixteen waves, no more runs than the sequence has.
+unsigned order_walk_threads(int T, int W) {
+  const int columns = (W + 63) / 64, runs = (T + 31) / 32, most = 16 / columns;
+  return (unsigned)(64 * columns * (runs < most ? runs : most));
+}
+
+// One block per (b, h) reading each value once, or three passes over chunks.
+// A one-pass block takes about 4.2 us per step of its tokens (512 at W = 64,
+// 256 at 128), one block per compute unit at a time, and at best the time of
+// its traffic; the chunk kernels three launches of about 4 us and 3/2 of the
+// traffic at 4.5 TB/s.  Forward + backward, one pass against three: B16
+// T1000 H12 W128 103 / 152 us, B16 T1024 H8 W64 40 / 56, B1 T512 H1 W64
+// 15 / 35; the other way round B2 T4096 H16 W128 197 / 121, B4 T2048 H8 W64
+// 52 / 41.  Near the line (B4 T4096 H16 W64 114 / 109) three passes are taken
+// unless one is estimated 20% faster.
+bool order_walks(int B, int T, int H, int W) {
+  const double runs = (T + 31) / 32, waves = order_walk_threads(T, W) / 64;
+  const double steps = std::ceil(runs * ((W + 63) / 64) / waves);
+  const double rounds = std::ceil((double)B * H / g_cus);
+  const double traffic = 2.0 * sizeof(float) * B * T * H * W / 4.5e6;  // us
+  return std::fmax(3.0 + 4.2 * steps * rounds, traffic) < 0.8 * (12.0 + 1.5 * traffic);
+}
+
 }  // namespace
 
 size_t m4mr_order_workspace_bytes(int B, int T, int H, int W, int chunk) {
@@ -1305,6 +1332,11 @@ int m4mr_order_forward(const float* values, const float* log_decay, const float*
   if (workspace_bytes < order_workspace(d, &states, &totals, workspace))
     return fail(M4MR_EINVAL, "m4mr_order_forward: workspace too small");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (order_walks(B, T, H, W))
+    return launch("order_walk", st, [&] {
+      hipLaunchKernelGGL(m4::order_walk_kernel, dim3(B * H), dim3(order_walk_threads(T, W)), 0, st,
+                         d, values, log_decay, initial, output);
+    });
   const unsigned chunks = (unsigned)((long)B * H * d.NC), threads = order_threads(W);
   int rc = launch("order_local", st, [&] {
     hipLaunchKernelGGL(m4::order_local_kernel, dim3(chunks), dim3(threads), 0, st, d, values,
@@ -1339,6 +1371,12 @@ int m4mr_order_backward(const float* values, const float* log_decay, const float
   if (workspace_bytes < order_workspace(d, &heads, &totals, workspace))
     return fail(M4MR_EINVAL, "m4mr_order_backward: workspace too small");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (order_walks(B, T, H, W))
+    return launch("order_bwd_walk", st, [&] {
+      hipLaunchKernelGGL(m4::order_bwd_walk_kernel, dim3(B * H), dim3(order_walk_threads(T, W)), 0,
+                         st, d, values, log_decay, initial, output, d_output, d_values,
+                         d_log_decay, d_initial);
+    });
   const unsigned chunks = (unsigned)((long)B * H * d.NC), threads = order_threads(W);
   int rc = launch("order_bwd_local", st, [&] {
     hipLaunchKernelGGL(m4::order_bwd_local_kernel, dim3(chunks), dim3(threads), 0, st, d,

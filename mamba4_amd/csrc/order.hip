@@ -17,6 +17,8 @@
 //             g_t = dout_t + lam_(t+1) g_(t+1): d v_t = (1 - lam_t) g_t,
 //             d log_decay_t = lam_t sum_c g_t,c (h_(t-1),c - v_t,c) (summed
 //             over channels in a fixed order), d initial = lam_0 g_0.
+// Where enough (b, h) fill the chip, or the sequence is short, one kernel each
+// way does the whole scan instead (order_walk, order_bwd_walk below).
 #include "common.hpp"
 
 namespace m4 {
@@ -340,6 +342,210 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     for (int w = 0; w < waves; ++w) sum += part[w][c];
     d_log_decay[order_row(d, o.b, o.t0 + c, o.h)] = gate.lam * sum;
   }
+}
+
+// ---------------------------------------------------------------------
+// The same scan with each value read once: one block per (b, h) holds
+// WALK_TOKENS tokens of every channel in registers per wave, its waves
+// covering consecutive runs of tokens (`groups` of them) times 64-channel
+// columns.  Each step, every wave scans its run from zero, the runs' ends and
+// total decays meet in LDS, and every wave takes its start state from them
+// and scans its registers again, writing the results.  The backward also
+// rebuilds h_(t-1) from the values and the one stored output before its run.
+//
+// Bound by HBM: 2 + 3 passes over the values' size instead of the three-pass
+// kernels' 3 + 5 (B16 T1000 H12 W128: 37 us forward and 66 backward, 5.3 and
+// 4.5 TB/s, against 53 and 99).  It needs a (b, h) per compute unit or so to
+// fill the chip, the three-pass kernels a chunk (order_walks in the host code
+// chooses).  A wave's decays stay in scalar registers for both scans (read
+// again from their lanes the forward took 40 us).  Runs of 32 tokens: the
+// backward's two values per token fill the 128 registers that sixteen waves
+// leave each lane.
+constexpr int WALK_TOKENS = 32;
+constexpr int WALK_MAX_WAVES = 16;
+
+struct WalkWave {
+  int bh, b, h, tg, groups, c, cc, l;
+  bool on;
+
+  __device__ __forceinline__ explicit WalkWave(const OrderDims& d) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), columns = (d.W + 63) >> 6;
+    l = lane_id();
+    bh = blockIdx.x;
+    b = bh / d.H;
+    h = bh % d.H;
+    tg = wave / columns;
+    groups = (int)(blockDim.x >> 6) / columns;
+    c = (wave % columns) * 64 + l;
+    on = c < d.W;
+    cc = min(c, d.W - 1);
+  }
+};
+
+// A run's gates: lane l < WALK_TOKENS holds token l (no decay and no inflow
+// past the run's end, which leaves a scan as it is).
+struct WalkGates {
+  float lg, lam, inflow;
+
+  __device__ __forceinline__ WalkGates(const OrderDims& d, const WalkWave& w, int t0, int len,
+                                       const float* log_decay) {
+    lg = w.l < len ? log_decay[order_row(d, w.b, t0 + w.l, w.h)] : 0.f;
+    lam = expf(lg);
+    inflow = -expm1f(lg);
+  }
+  // The run's decay (every lane receives it).
+  __device__ __forceinline__ float total() const { return expf(group4_sum(row16_sum(lg))); }
+};
+
+__device__ __forceinline__ int run_len(const OrderDims& d, int t0) {
+  return max(min(WALK_TOKENS, d.T - t0), 0);
+}
+
+// Rows t0.. of `rows` at this lane's channel, zeros past the run.
+__device__ __forceinline__ void load_run(float (&x)[WALK_TOKENS], const OrderDims& d,
+                                         const WalkWave& w, int t0, int len, const float* rows) {
+  if (len == WALK_TOKENS) {
+    const float* first = rows + order_row(d, w.b, t0, w.h) * d.W + w.cc;
+    const long stride = (long)d.H * d.W;
+#pragma unroll
+    for (int i = 0; i < WALK_TOKENS; ++i) x[i] = first[i * stride];
+  } else {
+    const long last = max(min(t0 + len, d.T) - 1, 0);
+#pragma unroll
+    for (int i = 0; i < WALK_TOKENS; ++i) {
+      const float v = rows[order_row(d, w.b, (int)min((long)t0 + i, last), w.h) * d.W + w.cc];
+      x[i] = i < len ? v : 0.f;
+    }
+  }
+}
+
+__global__ __launch_bounds__(64 * WALK_MAX_WAVES) void order_walk_kernel(
+    OrderDims d, const float* values, const float* log_decay, const float* initial,
+    float* output) {
+  __shared__ float ends[2][WALK_MAX_WAVES][64];
+  __shared__ float decays[2][WALK_MAX_WAVES];
+  const WalkWave w(d);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int columns = (d.W + 63) >> 6, column = wave % columns;
+  const long stride = (long)d.H * d.W;
+  float carry = initial ? initial[(long)w.bh * d.W + w.cc] : 0.f;
+  int buf = 0;
+  for (int base = 0; base < d.T; base += w.groups * WALK_TOKENS, buf ^= 1) {
+    const int t0 = base + w.tg * WALK_TOKENS, len = run_len(d, t0);
+    float x[WALK_TOKENS];
+    load_run(x, d, w, t0, len, values);
+    const WalkGates gate(d, w, t0, len, log_decay);
+    float lam[WALK_TOKENS], s = 0.f;  // the decays in scalar registers
+#pragma unroll
+    for (int i = 0; i < WALK_TOKENS; ++i) {
+      lam[i] = lane_value(gate.lam, i);
+      x[i] *= lane_value(gate.inflow, i);
+      s = lam[i] * s + x[i];
+    }
+    ends[buf][wave][w.l] = s;
+    decays[buf][wave] = gate.total();  // by every lane: its sum crosses lanes
+    __syncthreads();
+    s = carry;
+    for (int j = 0; j < w.groups; ++j) {
+      if (j == w.tg) s = carry;
+      carry = decays[buf][j * columns] * carry + ends[buf][j * columns + column][w.l];
+    }
+    float* out = output + order_row(d, w.b, t0, w.h) * d.W + w.c;
+    if (len == WALK_TOKENS && w.on) {
+#pragma unroll
+      for (int i = 0; i < WALK_TOKENS; ++i) {
+        s = lam[i] * s + x[i];
+        out[i * stride] = s;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < WALK_TOKENS; ++i) {
+        s = lam[i] * s + x[i];
+        if (i < len && w.on) out[i * stride] = s;
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(64 * WALK_MAX_WAVES) void order_bwd_walk_kernel(
+    OrderDims d, const float* values, const float* log_decay, const float* initial,
+    const float* output, const float* d_output, float* d_values, float* d_log_decay,
+    float* d_initial) {
+  static_assert(WALK_TOKENS == ORDER_HALF, "a run is one butterfly");
+  __shared__ float heads[2][WALK_MAX_WAVES][64];
+  __shared__ float decays[2][WALK_MAX_WAVES];
+  __shared__ float part[2][WALK_MAX_WAVES][WALK_TOKENS];
+  const WalkWave w(d);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int columns = (d.W + 63) >> 6, column = wave % columns;
+  const long stride = (long)d.H * d.W;
+  float carry = 0.f;  // the cotangent reaching the step's last token from later ones
+  int buf = 0;
+  const int span = w.groups * WALK_TOKENS;
+  for (int base = (d.T - 1) / span * span; base >= 0; base -= span, buf ^= 1) {
+    const int t0 = base + w.tg * WALK_TOKENS, len = run_len(d, t0);
+    float dy[WALK_TOKENS], v[WALK_TOKENS];
+    load_run(dy, d, w, t0, len, d_output);
+    load_run(v, d, w, t0, len, values);
+    float h = t0 > 0 ? output[order_row(d, w.b, min(t0, d.T) - 1, w.h) * d.W + w.cc]
+              : initial ? initial[(long)w.bh * d.W + w.cc]
+                        : 0.f;
+    const WalkGates gate(d, w, t0, len, log_decay);
+    float lam[WALK_TOKENS], acc = 0.f;
+#pragma unroll
+    for (int i = WALK_TOKENS - 1; i >= 0; --i) {
+      lam[i] = lane_value(gate.lam, i);
+      acc = lam[i] * (dy[i] + acc);
+    }
+    heads[buf][wave][w.l] = acc;
+    decays[buf][wave] = gate.total();  // by every lane: its sum crosses lanes
+    // v becomes h_(t-1) - v_t.
+#pragma unroll
+    for (int i = 0; i < WALK_TOKENS; ++i) {
+      const float x = v[i];
+      v[i] = h - x;
+      h = lam[i] * h + lane_value(gate.inflow, i) * x;
+    }
+    __syncthreads();
+    acc = carry;
+    for (int j = w.groups - 1; j >= 0; --j) {
+      if (j == w.tg) acc = carry;
+      carry = heads[buf][j * columns + column][w.l] + decays[buf][j * columns] * carry;
+    }
+    float* dv = d_values + order_row(d, w.b, t0, w.h) * d.W + w.c;
+    if (len == WALK_TOKENS && w.on) {
+#pragma unroll
+      for (int i = WALK_TOKENS - 1; i >= 0; --i) {
+        const float gt = dy[i] + acc;
+        dv[i * stride] = lane_value(gate.inflow, i) * gt;
+        v[i] *= gt;
+        acc = lam[i] * gt;
+      }
+    } else {
+#pragma unroll
+      for (int i = WALK_TOKENS - 1; i >= 0; --i) {
+        const float gt = dy[i] + acc;
+        const bool in = i < len && w.on;
+        if (in) dv[i * stride] = lane_value(gate.inflow, i) * gt;
+        v[i] = in ? gt * v[i] : 0.f;
+        acc = lam[i] * gt;
+      }
+    }
+    const float sum = wave_sums32(v);
+    if (columns == 1) {
+      const float mine = __shfl(sum, 2 * (w.l & 31));  // lane l < 32: token l
+      if (w.l < len) d_log_decay[order_row(d, w.b, t0 + w.l, w.h)] = gate.lam * mine;
+    } else {
+      if ((w.l & 1) == 0) part[buf][wave][w.l >> 1] = sum;
+      __syncthreads();
+      if (column == 0 && w.l < len) {
+        float all = 0.f;
+        for (int j = 0; j < columns; ++j) all += part[buf][wave + j][w.l];
+        d_log_decay[order_row(d, w.b, t0 + w.l, w.h)] = gate.lam * all;
+      }
+    }
+  }
+  if (d_initial && w.tg == 0 && w.on) d_initial[(long)w.bh * d.W + w.c] = carry;
 }
 
 }  // namespace m4

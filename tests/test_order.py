@@ -207,6 +207,45 @@ def test_order_scan_matches_oracle(gpu_lib, batch, time, heads, width, chunk, in
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("initial", [False, True])
+@pytest.mark.parametrize(
+    "batch,time,heads,width,walks",
+    # One pass: edges of a 32-token run, of a 512-, 256- and 128-token step,
+    # and of a 64-channel column; three passes: long sequences of few heads.
+    [(2, 31, 2, 64, True), (2, 32, 2, 65, True), (1, 33, 3, 1, True), (3, 512, 2, 64, True),
+     (300, 257, 1, 128, True), (300, 130, 1, 256, True), (300, 513, 1, 63, True),
+     (1, 2500, 2, 64, False), (1, 1500, 2, 130, False)],
+)
+def test_order_routes_match_oracle(gpu_lib, batch, time, heads, width, walks, initial):
+    """Both kernel forms at their edges, each batch row another sequence."""
+    from mamba4_amd import _lib, order_memory_chunked
+    from tests.gpu_helpers import announce, normwise
+
+    values, log_decay, init = _problem(batch, time, heads, width, seed=time, initial=initial)
+    d_out = _loss_weights(values.shape)
+    announce(f"order route B{batch} T{time} H{heads} W{width} init={initial}")
+    v, lg, h0, d = _gpu(values, log_decay, init, d_out)
+    leaves = [t.requires_grad_(True) for t in (v, lg, h0) if t is not None]
+    _lib.profile_reset()
+    _lib.profile_select(None)
+    _lib.profile_enable(True)
+    try:
+        out = order_memory_chunked(v, lg, initial=h0)
+        grads = torch.autograd.grad(out, leaves, d)
+        torch.cuda.synchronize()
+    finally:
+        _lib.profile_enable(False)
+    launches = {n: _lib.profile_read(n)[1] for n in ("order_walk", "order_bwd_walk")}
+    _lib.profile_reset()
+    assert launches == dict.fromkeys(launches, int(walks))
+    want = [oracle.order_memory_chunked(values, log_decay, 64, init)]
+    want += oracle.order_memory_backward(values, log_decay, d_out, init)[:len(leaves)]
+    # float32 rounding of a decaying scan (and of a sum over the channels).
+    for got, ref in zip((out, *grads), want):
+        assert normwise(_host(got), ref) <= 3e-6
+
+
+@pytest.mark.gpu
 def test_order_cached_step_and_decay_form(gpu_lib):
     """The order head's cached decode step (lm/models/mamba4.py:283-287) is
     the scan over one token from the cache; order_memory takes the decays."""
