@@ -533,6 +533,23 @@ int m4mr_order_backward(const float* values, const float* log_decay, const float
                         void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * Up to eight dense arrays copied between widths in one launch: array i's
+ * `outer` matrices of src_rows x src_cols elements (2 or 4 bytes each) to
+ * dst_rows x dst_cols, cut off or padded with the bits `fill`.  A caller's
+ * arrays narrower than the kernels' widths pass through it (the reference
+ * pads to its lane width the same way, lm/kernels/mamba4_fused.py:292-297).
+ */
+typedef struct {
+  const void* src;
+  void* dst;
+  long outer;
+  int src_rows, src_cols, dst_rows, dst_cols;
+  int bytes;
+  unsigned fill;
+} m4mr_resize_array;
+int m4mr_resize(const m4mr_resize_array* arrays, int count, void* stream);
+
+/*
  * Kernel timing with HIP events recorded on the launch stream.  While
  * enabled, every kernel launch is bracketed by a pair of events.
  * m4mr_profile_read() waits for the recorded events and returns the total

@@ -45,6 +45,22 @@ class MixerParams(ctypes.Structure):
     ]
 
 
+class ResizeArray(ctypes.Structure):
+    """m4mr_resize_array (include/mamba4_memread.h)."""
+
+    _fields_ = [
+        ("src", ctypes.c_void_p),
+        ("dst", ctypes.c_void_p),
+        ("outer", ctypes.c_long),
+        ("src_rows", ctypes.c_int),
+        ("src_cols", ctypes.c_int),
+        ("dst_rows", ctypes.c_int),
+        ("dst_cols", ctypes.c_int),
+        ("bytes", ctypes.c_int),
+        ("fill", ctypes.c_uint),
+    ]
+
+
 SIGNATURES = {
     "m4mr_version": (ctypes.c_char_p, []),
     "m4mr_last_error": (ctypes.c_char_p, []),
@@ -95,6 +111,7 @@ SIGNATURES = {
     "m4mr_order_workspace_bytes": (_S, [_I] * 5),
     "m4mr_order_forward": (_I, [_P] * 3 + [_I] * 5 + [_P, _P, _S, _P]),
     "m4mr_order_backward": (_I, [_P] * 5 + [_I] * 5 + [_P] * 4 + [_S, _P]),
+    "m4mr_resize": (_I, [ctypes.POINTER(ResizeArray), _I, _P]),
     "m3s_forward": (_I, [_P] * 9 + [_I] * 6 + [_P] * 4 + [_P]),
     "m3s_backward_workspace_bytes": (_S, [_I] * 6),
     "m3s_backward": (_I, [_P] * 9 + [_I] * 6 + [_P] * 4 + [_P] * 9 + [_P, _S, _P]),

@@ -89,6 +89,7 @@ __global__ void spd_wide_kernel(const float*, const float*, int, float*, float*)
 template <bool LDS>
 __global__ void spd_wide_backward_kernel(const float*, const float*, const float*, int, float*,
                                          float*);
+__global__ void resize_kernel(ResizeJobs);
 __global__ void diag_eigen_kernel(const float*, const float*, const float*, int, int, int, float*);
 __global__ void diag_summary_kernel(const float*, int, const float*, int, float*);
 }  // namespace m4
@@ -111,7 +112,7 @@ const char* const kKernelNames[] = {"fwd_stats",      "fwd_scan",  "fwd_states",
                                     "m3_walk",        "m3_out",    "m3_walk_bwd", "m3_grad",
                                     "m3_finish",      "m3_bias",   "m3_suffix",
                                     "mixer_finish",   "diag_eigen", "diag_summary",
-                                    "spd_wide",       "spd_wide_backward"};
+                                    "spd_wide",       "spd_wide_backward", "resize"};
 
 struct ProfRecord {
   const char* name;
@@ -1391,6 +1392,37 @@ int m4mr_order_backward(const float* values, const float* log_decay, const float
   return launch("order_bwd_apply", st, [&] {
     hipLaunchKernelGGL(m4::order_bwd_apply_kernel, dim3(chunks), dim3(threads), 0, st, d, values,
                        log_decay, initial, output, d_output, heads, d_values, d_log_decay);
+  });
+}
+
+int m4mr_resize(const m4mr_resize_array* arrays, int count, void* stream) {
+  g_error.clear();
+  if (!arrays || count < 1 || count > m4::kResizeJobs)
+    return fail(M4MR_EINVAL, "m4mr_resize: need 1.." + std::to_string(m4::kResizeJobs) + " arrays");
+  m4::ResizeJobs jobs{};
+  long elements = 0;
+  for (int i = 0; i < count; ++i) {
+    const m4mr_resize_array& a = arrays[i];
+    if (a.outer < 0 || a.src_rows < 0 || a.src_cols < 0 || a.dst_rows < 0 || a.dst_cols < 0 ||
+        (a.bytes != 2 && a.bytes != 4))
+      return fail(M4MR_EINVAL, "m4mr_resize: sizes must not be negative, elements 2 or 4 bytes");
+    const double wide = (double)a.dst_rows * a.dst_cols;
+    if (wide > INT_MAX || wide * a.outer > 1e15)
+      return fail(M4MR_EINVAL, "m4mr_resize: array too large");
+    const long n = a.outer * a.dst_rows * a.dst_cols;
+    if (n == 0) continue;
+    if (!a.dst || (!a.src && a.src_rows > 0 && a.src_cols > 0))
+      return fail(M4MR_EINVAL, "m4mr_resize: a required pointer is NULL");
+    jobs.job[jobs.count++] = m4::ResizeJob{a.src,      a.dst,      n,       a.src_rows, a.src_cols,
+                                           a.dst_rows, a.dst_cols, a.bytes, a.fill};
+    elements += n;
+  }
+  if (elements == 0) return M4MR_OK;
+  if ((elements + 255) / 256 > INT_MAX) return fail(M4MR_EINVAL, "m4mr_resize: arrays too large");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return launch("resize", st, [&] {
+    hipLaunchKernelGGL(m4::resize_kernel, dim3((unsigned)((elements + 255) / 256)), dim3(256), 0,
+                       st, jobs);
   });
 }
 

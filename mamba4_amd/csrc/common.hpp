@@ -808,6 +808,22 @@ struct StateArgs {
 
 // Shape of the order head's scan: values [B,T,H,W] in chunks of `chunk`
 // tokens, NC of them.
+// One array of resize_kernel: `outer` matrices src_rows x src_cols to
+// dst_rows x dst_cols of `bytes`-byte elements (4 or 2), cut off or padded with
+// `fill`; `elements` of the destination.
+struct ResizeJob {
+  const void* src;
+  void* dst;
+  long elements;
+  int src_rows, src_cols, dst_rows, dst_cols, bytes;
+  unsigned fill;
+};
+constexpr int kResizeJobs = 8;
+struct ResizeJobs {
+  ResizeJob job[kResizeJobs];
+  int count;
+};
+
 struct OrderDims {
   int B, T, H, W, chunk, NC;
 };

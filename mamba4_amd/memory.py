@@ -123,13 +123,55 @@ def memread_forward(keys, values, queries, beta, log_decay, floor, init_s, init_
     return output, variance, final_s, final_c, solved, factors, start_s, start_c
 
 
+def _resized(*arrays):
+    """Each (contiguous tensor, rows, cols, fill) with its last two axes cut
+    off or padded to rows x cols (rows None: the last axis alone), all in one
+    launch; a tensor that has that shape already, or None, is passed through."""
+    out, jobs = [], []
+    for t, rows, cols, fill in arrays:
+        if t is None or (t.shape[-1] == cols and rows in (None, t.shape[-2])):
+            out.append(t)
+            continue
+        lead = t.shape[:-1] if rows is None else t.shape[:-2]
+        shape = lead + (cols,) if rows is None else lead + (rows, cols)
+        new = torch.empty(shape, dtype=t.dtype, device=t.device)
+        jobs.append(_lib.ResizeArray(
+            _ptr(t), _ptr(new), lead.numel(), 1 if rows is None else t.shape[-2], t.shape[-1],
+            1 if rows is None else rows, cols, t.element_size(), _ONE_BITS if fill else 0))
+        out.append(new)
+    if jobs:
+        _lib.check(_lib.load().m4mr_resize((_lib.ResizeArray * len(jobs))(*jobs), len(jobs),
+                                           _stream()))
+    return out
+
+
+_ONE_BITS = 0x3F800000  # 1.0 in float32
+
+
+def _padded(keys, values, queries, floor, init_s, init_c):
+    """The arrays at the library's widths.  Padded key coordinates form an
+    identity block (zero keys, unit floor): they solve to zero and leave the
+    true coordinates unchanged (lm/kernels/mamba4_fused.py:292-297).  Padded
+    values read nothing."""
+    dim, width = _lib.KEY_DIM, _value_width(values.shape[-1])
+    return _resized((keys, None, dim, 0), (values, None, width, 0), (queries, None, dim, 0),
+                    (floor, None, dim, 1), (init_s, dim, dim, 0), (init_c, width, dim, 0))
+
+
 class _MemoryRead(torch.autograd.Function):
-    """Custom VJP around m4mr_forward / m4mr_backward (D = 64, P = 64 or 128;
+    """Custom VJP around m4mr_forward / m4mr_backward (D <= 64, P <= 128;
     keys, values and queries float32, or all bfloat16 through the _bf16
     entry points)."""
 
     @staticmethod
     def forward(ctx, keys, values, queries, beta, log_decay, floor, init_s, init_c, chunk):
+        # A cotangent that nothing reaches stays None rather than a tensor of
+        # zeros filled for every call.
+        ctx.set_materialize_grads(False)
+        ctx.dims = keys.shape[-1], values.shape[-1]
+        ctx.has_initial = init_s is not None
+        keys, values, queries, floor, init_s, init_c = _padded(keys, values, queries, floor,
+                                                               init_s, init_c)
         output, variance, final_s, final_c, solved, factors, start_s, start_c = memread_forward(
             keys, values, queries, beta, log_decay, floor, init_s, init_c, chunk
         )
@@ -138,15 +180,20 @@ class _MemoryRead(torch.autograd.Function):
             keys, values, queries, beta, log_decay, floor, solved, factors, start_s, start_c
         )
         ctx.chunk = chunk
-        ctx.has_initial = init_s is not None
         return output, variance, final_s, final_c
 
     @staticmethod
     def backward(ctx, d_output, d_variance, d_final_s, d_final_c):
+        dim, value_dim = ctx.dims
         grads = memread_backward(*ctx.saved_tensors, ctx.chunk, d_output, d_variance,
                                  d_final_s, d_final_c)
-        d_init = grads[6:] if ctx.has_initial else (None, None)
-        return (*grads[:6], *d_init, None)
+        d_keys, d_values, d_queries, d_floor, d_init_s, d_init_c = _resized(
+            (grads[0], None, dim, 0), (grads[1], None, value_dim, 0), (grads[2], None, dim, 0),
+            (grads[5], None, dim, 0),
+            (grads[6] if ctx.has_initial else None, dim, dim, 0),
+            (grads[7] if ctx.has_initial else None, value_dim, dim, 0))
+        return (d_keys, d_values, d_queries, grads[3], grads[4], d_floor, d_init_s, d_init_c,
+                None)
 
 
 def memread_backward(keys, values, queries, beta, log_decay, floor, solved, factors, start_s,
@@ -259,6 +306,13 @@ def spd_solve(precision, rhs, backend=None):
     return solution.reshape(batch + (dim,))
 
 
+def _expanded(x, shape, device):
+    """x as a float32 tensor of `shape` (itself where it is one already: an
+    expand of nothing still costs an autograd node each way)."""
+    x = torch.as_tensor(x, dtype=torch.float32, device=device)
+    return x if x.shape == shape else x.expand(shape)
+
+
 def _pad_last(x, width, value=0.0):
     extra = width - x.shape[-1]
     return x if extra == 0 else F.pad(x, (0, extra), value=value)
@@ -300,49 +354,42 @@ def selective_gaussian_memory(
         keys, values, queries = (a.to(torch.float32) for a in (keys, values, queries))
     if dim > _lib.KEY_DIM:
         raise ValueError(f"key widths must be <= {_lib.KEY_DIM}; got {dim}")
-    width = _value_width(value_dim)
+    _value_width(value_dim)  # refuses wider values
     if chunk_size < 1:
         raise ValueError("chunk_size must be positive")
     device = keys.device
     shape = (batch, time, heads)
-    beta = torch.as_tensor(beta, dtype=torch.float32, device=device).expand(shape)
-    log_decay = torch.as_tensor(log_decay, dtype=torch.float32, device=device).expand(shape)
-    floor = torch.as_tensor(floor, dtype=torch.float32, device=device).expand(heads, dim)
+    beta, log_decay = _expanded(beta, shape, device), _expanded(log_decay, shape, device)
+    floor = _expanded(floor, (heads, dim), device)
     _require_device(beta, log_decay, floor)
-    # Padded key coordinates form an identity block (zero keys, unit floor):
-    # they solve to zero and leave the true coordinates unchanged
-    # (lm/kernels/mamba4_fused.py:292-297).  Padded values read nothing.
-    k = _pad_last(keys, _lib.KEY_DIM).contiguous()
-    q = _pad_last(queries, _lib.KEY_DIM).contiguous()
-    v = _pad_last(values, width).contiguous()
-    f = _pad_last(floor, _lib.KEY_DIM, value=1.0).contiguous()
     init_s = init_c = None
     if initial is not None:
         init_s = torch.as_tensor(initial.evidence).to(torch.float32)
         init_c = torch.as_tensor(initial.cross).to(torch.float32)
         _require_device(init_s, init_c)
-        init_s = F.pad(init_s, (0, _lib.KEY_DIM - dim, 0, _lib.KEY_DIM - dim)).contiguous()
-        init_c = F.pad(
-            init_c, (0, _lib.KEY_DIM - dim, 0, width - value_dim)
-        ).contiguous()
+        init_s, init_c = init_s.contiguous(), init_c.contiguous()
     chunk = min(int(chunk_size), _lib.MAX_CHUNK)
-    args = (k, v, q, beta.contiguous(), log_decay.contiguous(), f, init_s, init_c, chunk)
+    k, v, q, f = (t.contiguous() for t in (keys, values, queries, floor))
+    beta, log_decay = beta.contiguous(), log_decay.contiguous()
     differentiable = (keys, values, queries, beta, log_decay, floor, init_s, init_c)
     with torch.cuda.device(device):
         if torch.is_grad_enabled() and any(
             t is not None and t.requires_grad for t in differentiable
         ):
-            output, variance, final_s, final_c = _MemoryRead.apply(*args)
+            output, variance, final_s, final_c = _MemoryRead.apply(
+                k, v, q, beta, log_decay, f, init_s, init_c, chunk)
         else:
             # No gradient: factor and solve without storing the factors, as
             # the reference's primal chunk_solve does
             # (lm/kernels/mamba4_fused.py:323-326).
-            output, variance, final_s, final_c = memread_forward(*args, store_factors=False)[:4]
-    return SelectiveResult(
-        output[..., :value_dim],
-        variance,
-        SelectiveState(final_s[..., :dim, :dim], final_c[..., :value_dim, :dim]),
-    )
+            k, v, q, f, init_s, init_c = _padded(k, v, q, f, init_s, init_c)
+            output, variance, final_s, final_c = memread_forward(
+                k, v, q, beta, log_decay, f, init_s, init_c, chunk, store_factors=False)[:4]
+    if value_dim != output.shape[-1]:
+        output, final_c = output[..., :value_dim], final_c[..., :value_dim, :]
+    if dim != _lib.KEY_DIM:
+        final_s, final_c = final_s[..., :dim, :dim], final_c[..., :dim]
+    return SelectiveResult(output, variance, SelectiveState(final_s, final_c))
 
 
 def selective_decode(state, key, value, query, beta, log_decay, floor, solver=None):
