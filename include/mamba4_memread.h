@@ -375,6 +375,18 @@ int m4mr_decode_step(float* evidence, float* cross,
                      float* output, float* variance, void* stream);
 
 /*
+ * The same step with the new state written to new_evidence [N,D,D] and
+ * new_cross [N,P,D], the old one left as it is (each new array either the
+ * old one itself or apart from both).
+ */
+int m4mr_decode_step_to(const float* evidence, const float* cross,
+                        const float* key, const float* value, const float* query,
+                        const float* beta, const float* log_decay, const float* floor,
+                        long N, int H, int value_dim,
+                        float* new_evidence, float* new_cross,
+                        float* output, float* variance, void* stream);
+
+/*
  * Batched SPD solve: precision_n y_n = rhs_n for N systems of width dim
  * (1 <= dim <= M4MR_SPD_MAX_DIM).  precision [N,dim,dim] row-major, of
  * which only the lower triangle (column <= row) is read; rhs and solution

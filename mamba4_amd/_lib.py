@@ -96,6 +96,7 @@ SIGNATURES = {
     ),
     "m4mr_factored_solve": (_I, [_P, _P, _P, _L, _P]),
     "m4mr_decode_step": (_I, [_P] * 8 + [_L, _I, _I, _P, _P, _P]),
+    "m4mr_decode_step_to": (_I, [_P] * 8 + [_L, _I, _I] + [_P] * 5),
     "m4mr_spd_solve": (_I, [_P, _P, _L, _I, _P, _P, _P]),
     "m4mr_spd_solve_backward": (_I, [_P, _P, _P, _L, _I, _P, _P, _P]),
     "m4mr_spd_factor_floats": (_L, [_I]),

@@ -17,7 +17,8 @@
 // stored factors per wave into registers and run the two substitutions.
 //
 // decode_step_kernel restates selective_decode (lm/kernels/mamba4.py:341-355)
-// for four resident states per wave, updated in place.
+// for four states per wave (or per block of eight, when there are few), in
+// place or to new arrays.
 #include "rows16.hpp"
 
 namespace m4 {
@@ -575,7 +576,9 @@ __global__ __launch_bounds__(64) void spd_backward_kernel(
   }
 }
 
-// One decode step for four (batch*head) states per wave, in place.
+// One decode step for four (batch*head) states per wave, from (evidence,
+// cross) to (new_evidence, new_cross), which may be the same arrays: every
+// element is read by the thread that writes it, before it does.
 //
 // The states stream through coalesced passes: in each, the 16 lanes of DPP
 // row mu sweep whole 256-byte rows of state mu (lane c holds column quad c),
@@ -588,16 +591,18 @@ __global__ __launch_bounds__(64) void spd_backward_kernel(
 // Two waves per SIMD: the value, query and key quad are read again after the
 // factorization rather than held in registers across it.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-decode_step_kernel(float* __restrict__ evidence, float* __restrict__ cross,
-                   const float* __restrict__ key, const float* __restrict__ value,
-                   const float* __restrict__ query, const float* __restrict__ beta,
-                   const float* __restrict__ log_decay, const float* __restrict__ floor, long N,
-                   int H, int NV, float* __restrict__ output, float* __restrict__ variance) {
+decode_step_kernel(const float* evidence, const float* cross, float* new_evidence,
+                   float* new_cross, const float* __restrict__ key,
+                   const float* __restrict__ value, const float* __restrict__ query,
+                   const float* __restrict__ beta, const float* __restrict__ log_decay,
+                   const float* __restrict__ floor, long N, int H, int NV,
+                   float* __restrict__ output, float* __restrict__ variance) {
   const int lane = threadIdx.x, a = lane & 15, mu = lane >> 4;
   long nidx = (long)blockIdx.x * 4 + mu;
   const bool active = nidx < N;
   if (!active) nidx = N - 1;
-  float* S = evidence + nidx * 4096;
+  const float* S = evidence + nidx * 4096;
+  float* new_S = new_evidence + nidx * 4096;
   const int P = 64 * NV;  // value width; the cross state is NV stacked 64x64 tiles
   float kr[4], qr[4], fl[4];
 #pragma unroll
@@ -619,7 +624,8 @@ decode_step_kernel(float* __restrict__ evidence, float* __restrict__ cross,
     // lane that holds it in this row's slot (bcast16 of kr[m]).  All 16
     // loads are issued before the first store (a store between them would
     // leave one load in flight at a time).
-    f4* rows = reinterpret_cast<f4*>(S + 16 * m * 64) + a;
+    const f4* rows = reinterpret_cast<const f4*>(S + 16 * m * 64) + a;
+    f4* new_rows = reinterpret_cast<f4*>(new_S + 16 * m * 64) + a;
     f4 sv[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) sv[r] = __builtin_nontemporal_load(rows + 16 * r);
@@ -631,7 +637,7 @@ decode_step_kernel(float* __restrict__ evidence, float* __restrict__ cross,
     }
     if (active)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) __builtin_nontemporal_store(sv[r], rows + 16 * r);
+      for (int r = 0; r < 16; ++r) __builtin_nontemporal_store(sv[r], new_rows + 16 * r);
     __syncthreads();
     // Into the factorization layout, negated: block column 0 as row a of this
     // slot, blocks (m, K >= 1) exchanged (lane (g, j) takes quad 4K + g of
@@ -665,14 +671,16 @@ decode_step_kernel(float* __restrict__ evidence, float* __restrict__ cross,
   __syncthreads();
   const f4 yq = *reinterpret_cast<const f4*>(&ys[mu][4 * a]);
   for (int v = 0; v < NV; ++v) {
-    float* C = cross + (nidx * NV + v) * 4096;
+    const float* C = cross + (nidx * NV + v) * 4096;
+    float* new_C = new_cross + (nidx * NV + v) * 4096;
     float vr[4], out[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < 4; ++m) vr[m] = value[nidx * P + 64 * v + a + 16 * m];
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       // As for S: the slot's 16 row loads go out together.
-      f4* rows = reinterpret_cast<f4*>(C + 16 * m * 64) + a;
+      const f4* rows = reinterpret_cast<const f4*>(C + 16 * m * 64) + a;
+      f4* new_rows = reinterpret_cast<f4*>(new_C + 16 * m * 64) + a;
       f4 cv[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) cv[r] = __builtin_nontemporal_load(rows + 16 * r);
@@ -687,7 +695,7 @@ decode_step_kernel(float* __restrict__ evidence, float* __restrict__ cross,
       }
       if (active)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) __builtin_nontemporal_store(cv[r], rows + 16 * r);
+        for (int r = 0; r < 16; ++r) __builtin_nontemporal_store(cv[r], new_rows + 16 * r);
     }
 #pragma unroll
     for (int m = 0; m < 4; ++m)
@@ -698,6 +706,125 @@ decode_step_kernel(float* __restrict__ evidence, float* __restrict__ cross,
   for (int m = 0; m < 4; ++m) var += qr[m] * y[m];
   var = sum16(var);
   if (active && a == 0) variance[nidx] = var;
+}
+
+// The same step for few states: eight waves per four states instead of one.
+// decode_step_kernel is a chain there (four slots of S, the factorization,
+// four slots of each value tile, each waiting for its loads): 23 us for 48
+// states of P = 128, 12 waves on the whole chip.  Here waves 0..3 each update
+// one slot of S into LDS and waves 4..7 one slot of every value tile, held in
+// registers while wave 0 factors and solves; 17.5 us.  The two groups of
+// waves branch apart as a whole (a scalar branch, two barriers in each), so
+// the value tiles are not live in the factorization's registers.  Same arithmetic in the
+// same order: the results are the same to the bit.
+__global__ __launch_bounds__(512) void decode_step_wide_kernel(
+    const float* evidence, const float* cross, float* new_evidence, float* new_cross,
+    const float* __restrict__ key, const float* __restrict__ value,
+    const float* __restrict__ query, const float* __restrict__ beta,
+    const float* __restrict__ log_decay, const float* __restrict__ floor, long N, int H, int NV,
+    float* __restrict__ output, float* __restrict__ variance) {
+  const int lane = threadIdx.x & 63, a = lane & 15, mu = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slot = wave & 3;
+  long nidx = (long)blockIdx.x * 4 + mu;
+  const bool active = nidx < N;
+  if (!active) nidx = N - 1;
+  const int P = 64 * NV;
+  const f4 kq = *reinterpret_cast<const f4*>(key + nidx * 64 + 4 * a);
+  const float bt = beta[nidx], lam = expf(log_decay[nidx]);
+  __shared__ f4 stage[4][4 * 16 * 17];  // [slot][state][row][quad], as decode_step_kernel's
+  __shared__ float ys[4][64];
+  if (wave < 4) {
+    f4* mine = stage[slot] + mu * 16 * 17;
+    const float kr = key[nidx * 64 + a + 16 * slot];
+    const f4* rows = reinterpret_cast<const f4*>(evidence + nidx * 4096 + 16 * slot * 64) + a;
+    f4* new_rows = reinterpret_cast<f4*>(new_evidence + nidx * 4096 + 16 * slot * 64) + a;
+    f4 sv[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sv[r] = __builtin_nontemporal_load(rows + 16 * r);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float bk = bt * bcast16(kr, r);
+      sv[r] = lam * sv[r] + bk * kq;
+      mine[r * 17 + a] = sv[r];
+    }
+    if (active)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) __builtin_nontemporal_store(sv[r], new_rows + 16 * r);
+    __syncthreads();
+    if (wave == 0) {
+      float A[4][64], fl[4], qr[4], nw[4], y[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        qr[m] = query[nidx * 64 + a + 16 * m];
+        fl[m] = floor[(nidx % H) * 64 + a + 16 * m];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f4 v = stage[m][(mu * 16 + a) * 17 + q];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) A[m][4 * q + e] = -v[e];
+        }
+#pragma unroll
+        for (int K = 1; K <= m; ++K)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const f4 v = stage[m][(s * 16 + a) * 17 + 4 * K + mu];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) A[m][16 * K + 4 * s + e] = -v[e];
+          }
+      }
+      factor_exchanged<false>(A, fl, qr, nw);
+      backward_rows16(A, nw, y);
+      float var = 0.f;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        ys[mu][a + 16 * m] = y[m];
+        var += query[nidx * 64 + a + 16 * m] * y[m];
+      }
+      var = sum16(var);
+      if (active && a == 0) variance[nidx] = var;
+    }
+    __syncthreads();
+  } else {
+    f4 cv[2][16];  // rows 16 slot.. of each value tile
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      if (v < NV) {
+        const float* C = cross + (nidx * NV + v) * 4096 + 16 * slot * 64;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          cv[v][r] = __builtin_nontemporal_load(reinterpret_cast<const f4*>(C) + a + 16 * r);
+      }
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      if (v < NV) {
+        float* C = new_cross + (nidx * NV + v) * 4096 + 16 * slot * 64;
+        const float vr = value[nidx * P + 64 * v + a + 16 * slot];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float bv = bt * bcast16(vr, r);
+          cv[v][r] = lam * cv[v][r] + bv * kq;
+        }
+        if (active)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            __builtin_nontemporal_store(cv[v][r], reinterpret_cast<f4*>(C) + a + 16 * r);
+      }
+    __syncthreads();
+    __syncthreads();
+    const f4 yq = *reinterpret_cast<const f4*>(&ys[mu][4 * a]);
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      if (v < NV) {
+        float out = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const f4 c = cv[v][r];
+          const float part = sum16(c[0] * yq[0] + c[1] * yq[1] + c[2] * yq[2] + c[3] * yq[3]);
+          out = a == r ? part : out;
+        }
+        if (active) output[nidx * P + 64 * v + a + 16 * slot] = out;
+      }
+  }
 }
 
 }  // namespace m4

@@ -427,31 +427,27 @@ def selective_decode(state, key, value, query, beta, log_decay, floor, solver=No
     if dim > _lib.KEY_DIM:
         raise ValueError(f"key widths must be <= {_lib.KEY_DIM}; got {dim}")
     width = _value_width(value_dim)
-    kd, vd = _lib.KEY_DIM - dim, width - value_dim
-    padded = SelectiveState(
-        F.pad(evidence.to(torch.float32), (0, kd, 0, kd)).contiguous(),
-        F.pad(cross.to(torch.float32), (0, kd, 0, vd)).contiguous(),
-    )
     device = evidence.device
-    floor = torch.as_tensor(floor, dtype=torch.float32, device=device).expand(
-        evidence.shape[1], dim
-    )
-    out = selective_decode_(
-        padded,
-        _pad_last(torch.as_tensor(key, device=device).to(torch.float32), _lib.KEY_DIM),
-        _pad_last(torch.as_tensor(value, device=device).to(torch.float32), width),
-        _pad_last(torch.as_tensor(query, device=device).to(torch.float32), _lib.KEY_DIM),
-        beta,
-        log_decay,
-        _pad_last(floor, _lib.KEY_DIM, value=1.0),
-        solver,
-    )
+    f32 = dict(dtype=torch.float32, device=device)
+    key, value, query = (torch.as_tensor(a).to(**f32).contiguous() for a in (key, value, query))
+    floor = torch.as_tensor(floor, **f32).expand(evidence.shape[1], dim).contiguous()
+    wide = _lib.KEY_DIM
+    with torch.cuda.device(device):
+        old_s, old_c, key, value, query, floor = _resized(
+            (evidence.to(torch.float32).contiguous(), wide, wide, 0),
+            (cross.to(torch.float32).contiguous(), width, wide, 0),
+            (key, None, wide, 0), (value, None, width, 0), (query, None, wide, 0),
+            (floor, None, wide, 1))
+    # The kernel reads the states 16 bytes at a time.
+    old_s, old_c = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (old_s, old_c))
+    new = SelectiveState(torch.empty(old_s.shape, **f32), torch.empty(old_c.shape, **f32))
+    out = _decode_step(SelectiveState(old_s, old_c), new, key, value, query, beta, log_decay, floor)
+    if (dim, value_dim) == (wide, width):
+        return out
     return SelectiveResult(
         out.output[..., :value_dim],
         out.variance,
-        SelectiveState(
-            out.state.evidence[..., :dim, :dim], out.state.cross[..., :value_dim, :dim]
-        ),
+        SelectiveState(new.evidence[..., :dim, :dim], new.cross[..., :value_dim, :dim]),
     )
 
 
@@ -461,32 +457,40 @@ def selective_decode_(state, key, value, query, beta, log_decay, floor, solver=N
     Needs float32 contiguous state tensors with D = 64 and P = 64 or 128.
     """
     _check_solver(solver)
-    lib = _lib.load()
     evidence, cross = state.evidence, state.cross
     _require_device(evidence, cross)
-    batch, heads, dim, _ = evidence.shape
-    value_dim = cross.shape[-2]
+    dim, value_dim = evidence.shape[-1], cross.shape[-2]
     if dim != _lib.KEY_DIM or value_dim not in (_lib.VALUE_DIM, _lib.MAX_VALUE_DIM):
         raise ValueError("the in-place decode needs D = 64 and P = 64 or 128 states")
     if evidence.dtype != torch.float32 or not evidence.is_contiguous() or not cross.is_contiguous():
         raise ValueError("the in-place decode needs contiguous float32 states")
-    device = evidence.device
-    f32 = dict(dtype=torch.float32, device=device)
+    f32 = dict(dtype=torch.float32, device=evidence.device)
     key, value, query = (torch.as_tensor(a).to(**f32).contiguous() for a in (key, value, query))
+    floor = torch.as_tensor(floor, **f32).expand(evidence.shape[1], dim).contiguous()
+    return _decode_step(state, state, key, value, query, beta, log_decay, floor)
+
+
+def _decode_step(old, new, key, value, query, beta, log_decay, floor):
+    """m4mr_decode_step_to from the state `old` to `new` (which may be the
+    same) at the library's widths."""
+    lib = _lib.load()
+    batch, heads = old.evidence.shape[:2]
+    width = old.cross.shape[-2]
+    device = old.evidence.device
+    f32 = dict(dtype=torch.float32, device=device)
     beta = torch.as_tensor(beta, **f32).expand(batch, heads).contiguous()
     log_decay = torch.as_tensor(log_decay, **f32).expand(batch, heads).contiguous()
-    floor = torch.as_tensor(floor, **f32).expand(heads, dim).contiguous()
-    output = torch.empty((batch, heads, value_dim), **f32)
+    output = torch.empty((batch, heads, width), **f32)
     variance = torch.empty((batch, heads), **f32)
     with torch.cuda.device(device):
         _lib.check(
-            lib.m4mr_decode_step(
-                _ptr(evidence), _ptr(cross), _ptr(key), _ptr(value), _ptr(query),
-                _ptr(beta), _ptr(log_decay), _ptr(floor), batch * heads, heads, value_dim,
-                _ptr(output), _ptr(variance), _stream(),
+            lib.m4mr_decode_step_to(
+                _ptr(old.evidence), _ptr(old.cross), _ptr(key), _ptr(value), _ptr(query),
+                _ptr(beta), _ptr(log_decay), _ptr(floor), batch * heads, heads, width,
+                _ptr(new.evidence), _ptr(new.cross), _ptr(output), _ptr(variance), _stream(),
             )
         )
-    return SelectiveResult(output, variance, state)
+    return SelectiveResult(output, variance, new)
 
 
 DIAGNOSTIC_KEYS = (
