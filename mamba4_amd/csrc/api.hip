@@ -1094,12 +1094,12 @@ int m4mr_diagnostics(const float* evidence, const float* cross, const float* flo
     return fail(M4MR_EINVAL, "m4mr_diagnostics: a required pointer is NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
   int rc = launch("diag_eigen", st, [&] {
-    hipLaunchKernelGGL(m4::diag_eigen_kernel, dim3((unsigned)(B * H)), dim3(64), 0, st, evidence,
+    hipLaunchKernelGGL(m4::diag_eigen_kernel, dim3((unsigned)(B * H)), dim3(256), 0, st, evidence,
                        cross, floor, H, D, P, per_state);
   });
   if (rc) return rc;
   return launch("diag_summary", st, [&] {
-    hipLaunchKernelGGL(m4::diag_summary_kernel, dim3(1), dim3(256), 0, st, per_state, B * H,
+    hipLaunchKernelGGL(m4::diag_summary_kernel, dim3(1), dim3(1024), 0, st, per_state, B * H,
                        floor, H * D, summary);
   });
 }

@@ -1,22 +1,23 @@
 // Spectral and finiteness probes of the final selective precision: restates
 // selective_diagnostics (lm/kernels/mamba4.py:358-376).
 //
-// diag_eigen_kernel: one 64-lane wave per (batch, head) state.  The
-// symmetrised precision (E + E^T) / 2 + diag(floor) goes to LDS in float64
-// (exact for float32 inputs) and a cyclic Jacobi iteration diagonalises it:
-// each round rotates n/2 disjoint index pairs (the round-robin "circle"
-// ordering, so a sweep of n - 1 rounds meets every pair once), lane k
-// computing pair k's rotation, then every lane applying all of the round's
-// rotations to its column (rows p, q) and then to its row (columns p, q),
-// and lane k finally setting a_pp - t a_pq, a_qq + t a_pq and a zero a_pq
-// (Rutishauser's form, which keeps the diagonal from collecting the
-// rotations' rounding).  Sweeps stop once the off-diagonal mass is below
-// 2^-100 of the diagonal's (or after kMaxSweeps, so every state ends); the
-// extreme diagonal entries are the extreme eigenvalues, rounded to float32.
-// In float32 the same iteration lands 1e-7 to 2e-6 of the largest
-// eigenvalue off float64 eigvalsh on 64-wide states; in float64 the
-// result is float64 eigvalsh's to within the final rounding.  This is a
-// monitoring probe, off every hot path.
+// diag_eigen_kernel: one 256-thread block per (batch, head) state, float64
+// throughout (exact for the float32 inputs).  The symmetrised precision
+// (E + E^T) / 2 + diag(floor) is brought to tridiagonal form by Householder
+// reflections, and the two extreme eigenvalues are found by multisection on
+// the Sturm counts of the tridiagonal (Barth, Martin and Wilkinson,
+// Numerische Mathematik 9 (1967) 386-393): 64 shifts a round, one per lane,
+// so a round narrows the interval 65 times and ten reach float64.  Both steps
+// are backward stable, as eigvalsh's own; the extremes are then rounded to
+// float32.
+//
+// Thread (r, w) holds columns 16w..16w+15 of row r in registers.  A
+// reflection takes a product of the matrix with the vector (16 multiply-adds
+// a thread, the four waves' parts meeting in LDS) and a rank-two update (32),
+// two barriers in all.  Bound by that chain of 62 reflections.  A cyclic
+// Jacobi iteration, every eigenvalue by up to forty sweeps of 63 rounds of
+// four barriers on one wave, took 4,557 us for 192 states of 64; this takes
+// 124.
 // The same pass takes the state's finiteness and the cross statistics'
 // largest magnitude.
 //
@@ -24,8 +25,6 @@
 #include "common.hpp"
 
 namespace m4 {
-
-constexpr int kMaxSweeps = 40;
 
 __device__ __forceinline__ float wave_min(float x) {
 #pragma unroll
@@ -37,22 +36,60 @@ __device__ __forceinline__ float wave_max(float x) {
   for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o));
   return x;
 }
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-  return x;
+// x at the lane of this lane's 16-lane row that the DPP pattern selects.
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double x) {
+  const uint2 u = __builtin_bit_cast(uint2, x);
+  return __builtin_bit_cast(
+      double, uint2{(unsigned)__builtin_amdgcn_update_dpp(0, (int)u.x, CTRL, 0xf, 0xf, true),
+                    (unsigned)__builtin_amdgcn_update_dpp(0, (int)u.y, CTRL, 0xf, 0xf, true)});
 }
 
-// Pair k of round r of the circle ordering of m (even) indices: index 0
-// stays, 1..m-1 turn one place per round.
-__device__ __forceinline__ void circle_pair(int k, int r, int m, int& p, int& q) {
-  const int ring = m - 1;
-  if (k == 0) {
-    p = 0;
-    q = r % ring + 1;
-  } else {
-    p = (r + k) % ring + 1;
-    q = (r - k + ring) % ring + 1;
+// Sum over the wave's 64 lanes, the same total in every lane.
+__device__ __forceinline__ double wave_sum(double x) {
+  x += dpp64<0xB1>(x);   // quad_perm [1,0,3,2]
+  x += dpp64<0x4E>(x);   // quad_perm [2,3,0,1]
+  x += dpp64<0x141>(x);  // row_half_mirror
+  x += dpp64<0x140>(x);  // row_mirror
+  uint2 u = __builtin_bit_cast(uint2, x);
+  auto lo = __builtin_amdgcn_permlane16_swap(u.x, u.x, false, false);
+  auto hi = __builtin_amdgcn_permlane16_swap(u.y, u.y, false, false);
+  x = __builtin_bit_cast(double, uint2{lo[0], hi[0]}) +
+      __builtin_bit_cast(double, uint2{lo[1], hi[1]});
+  u = __builtin_bit_cast(uint2, x);
+  lo = __builtin_amdgcn_permlane32_swap(u.x, u.x, false, false);
+  hi = __builtin_amdgcn_permlane32_swap(u.y, u.y, false, false);
+  return __builtin_bit_cast(double, uint2{lo[0], hi[0]}) +
+         __builtin_bit_cast(double, uint2{lo[1], hi[1]});
+}
+
+// x at lane `lane` (the same for the whole wave).
+__device__ __forceinline__ double lane_double(double x, int lane) {
+  const uint2 u = __builtin_bit_cast(uint2, x);
+  return __builtin_bit_cast(double, uint2{(unsigned)__builtin_amdgcn_readlane((int)u.x, lane),
+                                          (unsigned)__builtin_amdgcn_readlane((int)u.y, lane)});
+}
+
+// 1 / q to float64 rounding or so: the hardware's estimate and two Newton
+// steps (q neither zero nor subnormal).
+__device__ __forceinline__ double reciprocal(double q) {
+  double r = __builtin_amdgcn_rcp(q);
+  r = __builtin_fma(__builtin_fma(-q, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-q, r, 1.0), r, r);
+}
+
+// Eigenvalues below x of the tridiagonal with diagonal d and squared
+// off-diagonal e2 (e2[i] between i and i + 1), n rows: the negative pivots of
+// T - x (a pivot under `tiny` counts as -tiny).
+__device__ __forceinline__ int sturm_count(const double* d, const double* e2, int n, double x,
+                                           double tiny) {
+  int count = 0;
+  double q = d[0] - x;
+  for (int i = 0;; ++i) {
+    if (fabs(q) < tiny) q = -tiny;
+    count += q < 0.0;
+    if (i + 1 == n) return count;
+    q = (d[i + 1] - x) - e2[i] * reciprocal(q);
   }
 }
 
@@ -60,142 +97,156 @@ __device__ __forceinline__ void circle_pair(int k, int r, int m, int& p, int& q)
 // precision has a non-finite entry, as eigvalsh gives), 1 if every entry of
 // the state (evidence and cross) is finite else 0, max |cross| (NaN if a
 // cross entry is NaN, as jnp.max gives).
-__global__ __launch_bounds__(64) void diag_eigen_kernel(const float* __restrict__ evidence,
-                                                        const float* __restrict__ cross,
-                                                        const float* __restrict__ floor, int H,
-                                                        int D, int P, float* __restrict__ per_state) {
-  __shared__ double a[64][65];
-  __shared__ double rc[32], rs[32], rt[32];
-  const int bh = blockIdx.x, h = bh % H, lane = threadIdx.x;
+__global__ __launch_bounds__(256) void diag_eigen_kernel(const float* __restrict__ evidence,
+                                                         const float* __restrict__ cross,
+                                                         const float* __restrict__ floor, int H,
+                                                         int D, int P,
+                                                         float* __restrict__ per_state) {
+  __shared__ double column[2][64];  // the next column to reduce (double buffered)
+  __shared__ double part[4][64];
+  __shared__ double diagonal[64], off2[64];
+  __shared__ double wave_squares[4];
+  __shared__ float extreme[2], wave_max_cross[4];
+  const int bh = blockIdx.x, h = bh % H, r = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float* E = evidence + (long)bh * D * D;
   bool finite = true, prec_finite = true, cross_nan = false;
-  if (lane < D) {
-    const float fl = floor[h * D + lane];
-    prec_finite = isfinite(fl);
-    for (int j = 0; j < D; ++j) {
-      const float x = E[lane * D + j], y = E[j * D + lane];
+  double a[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int c = 16 * w + j;
+    a[j] = 0.0;
+    if (r < D && c < D) {
+      const float x = E[r * D + c], y = E[c * D + r];
       finite = finite && isfinite(x);
-      a[lane][j] = 0.5 * ((double)x + (double)y) + (j == lane ? (double)fl : 0.0);
+      a[j] = 0.5 * ((double)x + (double)y);
+      if (c == r) {
+        const float fl = floor[h * D + r];
+        prec_finite = isfinite(fl);
+        a[j] += (double)fl;
+      }
     }
   }
   prec_finite = prec_finite && finite;
   float cmax = 0.f;
   const float* C = cross + (long)bh * P * D;
-  for (long i = lane; i < (long)P * D; i += 64) {
+  for (long i = threadIdx.x; i < (long)P * D; i += 256) {
     const float v = C[i];
     finite = finite && isfinite(v);
     cross_nan = cross_nan || isnan(v);
     cmax = fmaxf(cmax, fabsf(v));
   }
-  // Uniform over the wave from here on.
-  prec_finite = wave_min(prec_finite ? 1.f : 0.f) > 0.f;
-  __syncthreads();
-  const int m = D + (D & 1);  // an odd width pairs its last index with a dummy
-  for (int sweep = 0; sweep < kMaxSweeps && D > 1 && prec_finite; ++sweep) {
-    double off = 0.0, dia = 0.0;
-    if (lane < D)
-      for (int j = 0; j < D; ++j) {
-        const double v = a[lane][j];
-        if (j == lane)
-          dia += v * v;
-        else
-          off += v * v;
-      }
-    off = wave_sum(off);
-    dia = wave_sum(dia);
-    // Uniform over the wave (kMaxSweeps bounds the loop regardless).
-    if (!(off > 0x1p-100 * dia)) break;
-    for (int r = 0; r < m - 1; ++r) {
-      double app = 0.0, aqq = 0.0, apq0 = 0.0;
-      if (lane < m / 2) {
-        int p, q;
-        circle_pair(lane, r, m, p, q);
-        double c = 1.0, s = 0.0, t = 0.0;
-        if (p < D && q < D) {
-          app = a[p][p];
-          aqq = a[q][q];
-          apq0 = a[p][q];
-          if (apq0 != 0.0) {
-            const double tau = (aqq - app) / (2.0 * apq0);
-            // t = tan of the angle that zeroes a_pq (the smaller root);
-            // 1 / (2 tau) once tau^2 would overflow.
-            t = fabs(tau) < 1e150 ? copysign(1.0, tau) / (fabs(tau) + sqrt(1.0 + tau * tau))
-                                  : 0.5 / tau;
-            c = 1.0 / sqrt(1.0 + t * t);
-            s = t * c;
-          }
-        }
-        rc[lane] = c;
-        rs[lane] = s;
-        rt[lane] = t;
-      }
-      __syncthreads();
-      // Rows p, q of this lane's column (A <- J^T A), then columns p, q of
-      // its row (A <- A J): the round's pairs are disjoint, so their
-      // rotations commute.
-      if (lane < D)
-        for (int k = 0; k < m / 2; ++k) {
-          int p, q;
-          circle_pair(k, r, m, p, q);
-          if (p < D && q < D) {
-            const double c = rc[k], s = rs[k], x = a[p][lane], y = a[q][lane];
-            a[p][lane] = c * x - s * y;
-            a[q][lane] = s * x + c * y;
-          }
-        }
-      __syncthreads();
-      if (lane < D)
-        for (int k = 0; k < m / 2; ++k) {
-          int p, q;
-          circle_pair(k, r, m, p, q);
-          if (p < D && q < D) {
-            const double c = rc[k], s = rs[k], x = a[lane][p], y = a[lane][q];
-            a[lane][p] = c * x - s * y;
-            a[lane][q] = s * x + c * y;
-          }
-        }
-      __syncthreads();
-      // The pair's own entries, from the values the round started with
-      // (only this pair's rotation touches a_pp, a_qq and a_pq).
-      if (lane < m / 2) {
-        int p, q;
-        circle_pair(lane, r, m, p, q);
-        if (p < D && q < D && rt[lane] != 0.0) {
-          a[p][p] = app - rt[lane] * apq0;
-          a[q][q] = aqq + rt[lane] * apq0;
-          a[p][q] = 0.0;
-          a[q][p] = 0.0;
+  cmax = wave_max(cmax);
+  if (r == 0) wave_max_cross[w] = cmax;
+  double squares = 0.0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) squares = __builtin_fma(a[j], a[j], squares);
+  squares = wave_sum(squares);
+  if (r == 0) wave_squares[w] = squares;
+  if (w == 0) column[0][r] = a[0];
+  // Uniform over the block from here on.
+  const bool any_bad_precision = __syncthreads_or(!prec_finite);
+  const bool any_bad = __syncthreads_or(!finite);
+  const bool any_cross_nan = __syncthreads_or(cross_nan);
+
+  // Column k at step k is final up to row k; its entries below are reflected
+  // onto row k + 1.  Rows and columns up to k hold stale values afterwards
+  // that nothing reads.
+  if (!any_bad_precision) {
+    // A column with less than 2^-70 of the matrix's norm below its first
+    // entry is reduced already: what is left of a rank-deficient matrix
+    // would otherwise shrink by 2^-53 a step until its squares underflow.
+    const double negligible =
+        0x1p-140 * (wave_squares[0] + wave_squares[1] + wave_squares[2] + wave_squares[3]);
+    for (int k = 0; k < D; ++k) {
+      const double x = column[k & 1][r];
+      if (w == 0 && r == k) diagonal[k] = x;
+      if (k + 1 == D) break;
+      const double below = r > k + 1 && r < D ? x : 0.0;
+      const double tail = wave_sum(below * below), head = lane_double(x, k + 1);
+      double off = head;
+      if (tail > negligible) {  // the same in every thread: uniform
+        const double norm = sqrt(head * head + tail);
+        off = head > 0.0 ? -norm : norm;
+        const double v = r == k + 1 ? head - off : below;
+        // 2 / v^T v = 1 / (norm (norm + |head|)).
+        const double beta = 1.0 / (norm * (norm + fabs(head)));
+        double p = 0.0;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) p = __builtin_fma(a[j], lane_double(v, 16 * w + j), p);
+        part[w][r] = p;
+        __syncthreads();
+        p = r > k && r < D ? beta * (part[0][r] + part[1][r] + part[2][r] + part[3][r]) : 0.0;
+        const double u = p - 0.5 * beta * wave_sum(p * v) * v;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          a[j] = __builtin_fma(-v, lane_double(u, 16 * w + j), a[j]);
+          a[j] = __builtin_fma(-u, lane_double(v, 16 * w + j), a[j]);
         }
       }
+      if (w == 0 && r == 0) off2[k] = off * off;
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (16 * w + j == k + 1) column[(k + 1) & 1][r] = a[j];
       __syncthreads();
     }
+    __syncthreads();
+
+    // Wave 0 finds the smallest eigenvalue (the least x with a count of 1),
+    // wave 1 the largest (with a count of D), between Gershgorin's bounds.
+    if (w < 2) {
+      const double d = r < D ? diagonal[r] : 0.0;
+      const double left = r > 0 && r < D ? sqrt(off2[r - 1]) : 0.0;
+      const double right = r + 1 < D ? sqrt(off2[r]) : 0.0;
+      double lo = r < D ? d - left - right : INFINITY, hi = r < D ? d + left + right : -INFINITY;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, o));
+        hi = fmax(hi, __shfl_xor(hi, o));
+      }
+      const double size = fmax(fabs(lo), fabs(hi));
+      const double tiny = fmax(size * 0x1p-80, 0x1p-960);
+      lo -= size * 0x1p-48 + tiny;
+      hi += size * 0x1p-48 + tiny;
+      const int want = w == 0 ? 1 : D;
+      for (int round = 0; round < 14; ++round) {
+        if (hi - lo <= 0x1p-52 * fmax(fabs(lo), fabs(hi))) break;  // uniform
+        const double step = (hi - lo) * (1.0 / 65.0), x = lo + step * (r + 1);
+        const unsigned long long at = __ballot(sturm_count(diagonal, off2, D, x, tiny) >= want);
+        // The counts grow with the shift (up to rounding): the first lane
+        // that reaches the count bounds the eigenvalue from above.
+        const int first = at ? __builtin_ctzll(at) : 64;
+        hi = first < 64 ? lane_double(x, first) : hi;
+        lo = first > 0 ? lane_double(x, first - 1) : lo;
+      }
+      if (r == 0) extreme[w] = (float)(0.5 * lo + 0.5 * hi);
+    }
+    __syncthreads();
   }
-  const float ev = lane < D ? (float)a[lane][lane] : 0.f;
-  const float lo = wave_min(lane < D ? ev : INFINITY), hi = wave_max(lane < D ? ev : -INFINITY);
-  // A NaN eigenvalue reads as NaN in both extremes (fminf / fmaxf drop it).
-  const bool nan_ev = !prec_finite || wave_max(isnan(ev) ? 1.f : 0.f) > 0.f;
-  const bool all_finite = wave_min(finite ? 1.f : 0.f) > 0.f;
-  const bool any_cross_nan = wave_max(cross_nan ? 1.f : 0.f) > 0.f;
-  cmax = wave_max(cmax);
-  if (lane == 0) {
-    per_state[4 * bh + 0] = nan_ev ? NAN : lo;
-    per_state[4 * bh + 1] = nan_ev ? NAN : hi;
-    per_state[4 * bh + 2] = all_finite ? 1.f : 0.f;
-    per_state[4 * bh + 3] = any_cross_nan ? NAN : cmax;
+  if (threadIdx.x == 0) {
+    per_state[4 * bh + 0] = any_bad_precision ? NAN : extreme[0];
+    per_state[4 * bh + 1] = any_bad_precision ? NAN : extreme[1];
+    per_state[4 * bh + 2] = any_bad ? 0.f : 1.f;
+    per_state[4 * bh + 3] =
+        any_cross_nan ? NAN
+                      : fmaxf(fmaxf(wave_max_cross[0], wave_max_cross[1]),
+                              fmaxf(wave_max_cross[2], wave_max_cross[3]));
   }
 }
 
 // summary[0..6] = min eigenvalue, max eigenvalue, max condition (per state,
 // max / max(min, 1e-30)), all finite (1 / 0), max |cross|, min floor, max
-// floor (lm/kernels/mamba4.py:368-376).  One 256-thread block.
-__global__ __launch_bounds__(256) void diag_summary_kernel(const float* __restrict__ per_state,
+// floor (lm/kernels/mamba4.py:368-376).  One block of sixteen waves: a chain of
+// loads per thread (16 us with four waves at 192 states of 64, 5.8 with sixteen).
+constexpr int kSummaryThreads = 1024;
+__global__ __launch_bounds__(kSummaryThreads) void diag_summary_kernel(const float* __restrict__ per_state,
                                                            int states, const float* __restrict__ floor,
                                                            int floors, float* __restrict__ summary) {
-  __shared__ float part[7][8];
+  __shared__ float part[7][kSummaryThreads / 64];
   float lo = INFINITY, hi = -INFINITY, cond = -INFINITY, fin = 1.f, cm = 0.f;
   float flo = INFINITY, fhi = -INFINITY;
   bool nan_ev = false, nan_cross = false, nan_floor = false;
-  for (int i = threadIdx.x; i < states; i += 256) {
+  for (int i = threadIdx.x; i < states; i += kSummaryThreads) {
     const float a = per_state[4 * i], b = per_state[4 * i + 1];
     nan_ev = nan_ev || isnan(a) || isnan(b);
     nan_cross = nan_cross || isnan(per_state[4 * i + 3]);
@@ -205,7 +256,8 @@ __global__ __launch_bounds__(256) void diag_summary_kernel(const float* __restri
     fin = fminf(fin, per_state[4 * i + 2]);
     cm = fmaxf(cm, per_state[4 * i + 3]);
   }
-  for (int i = threadIdx.x; i < floors; i += 256) {
+  #pragma unroll 4
+  for (int i = threadIdx.x; i < floors; i += kSummaryThreads) {
     const float f = floor[i];
     nan_floor = nan_floor || isnan(f);
     flo = fminf(flo, f);
@@ -225,7 +277,7 @@ __global__ __launch_bounds__(256) void diag_summary_kernel(const float* __restri
     const int k = threadIdx.x;
     const bool is_min = k == 0 || k == 3 || k == 5;
     float v = part[k][0];
-    for (int j = 1; j < 4; ++j) v = is_min ? fminf(v, part[k][j]) : fmaxf(v, part[k][j]);
+    for (int j = 1; j < kSummaryThreads / 64; ++j) v = is_min ? fminf(v, part[k][j]) : fmaxf(v, part[k][j]);
     // The reference's jnp.min / jnp.max propagate NaN; fminf / fmaxf drop
     // it, so it is put back where the reference would have it.
     if ((k <= 2 && any_ev) || (k == 4 && any_cross) || (k >= 5 && any_floor)) v = NAN;

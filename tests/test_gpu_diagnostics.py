@@ -98,6 +98,41 @@ def test_diagnostics_symmetrise_broadcast_and_flag_non_finite(gpu_lib):
     assert np.isfinite(got["cross_max_abs"])
 
 
+@pytest.mark.parametrize("dim", [1, 2, 3, 16, 17, 33, 64])
+def test_diagnostics_of_degenerate_spectra(gpu_lib, dim):
+    """Matrices whose tridiagonal decouples or repeats eigenvalues, and one
+    that is indefinite: the extremes are eigvalsh's to float32 rounding (and
+    float64 rounding of the largest eigenvalue)."""
+    rng = np.random.default_rng(dim)
+    dense = rng.normal(size=(dim, dim))
+    blocks = np.zeros((dim, dim))
+    half = (dim + 1) // 2
+    blocks[:half, :half] = dense[:half, :half] @ dense[:half, :half].T
+    vector = rng.normal(size=dim)
+    cases = [
+        np.zeros((dim, dim)),
+        np.eye(dim) * 3.0,
+        np.diag(np.logspace(-8, 3, dim)),
+        blocks,                                    # half of it zero
+        np.outer(vector, vector),                  # rank one
+        dense + dense.T,                           # indefinite
+        np.diag(rng.normal(size=dim)) * 1e30,      # squares past float32
+        np.ones((dim, dim)) * 1e-30,
+    ]
+    floor = np.zeros(dim, np.float32)
+    cross = np.ones((1, 1, 2, dim), np.float32)
+    for i, matrix in enumerate(cases):
+        evidence = matrix.astype(np.float32)
+        announce(f"selective_diagnostics degenerate case {i} D={dim}")
+        got = _diagnose(evidence[None, None], cross, floor)
+        exact = evidence.astype(np.float64)
+        want = np.linalg.eigvalsh(0.5 * (exact + exact.T))
+        size = np.abs(want).max()
+        for key, ref in (("precision_min_eigenvalue", want[0]),
+                         ("precision_max_eigenvalue", want[-1])):
+            assert abs(got[key] - ref) <= 1.2e-7 * abs(ref) + 1e-13 * size, (i, key, got[key], ref)
+
+
 def test_diagnostics_rejects_wide_states(gpu_lib):
     from mamba4_amd import SelectiveState, selective_diagnostics
 
