@@ -317,6 +317,24 @@ int m4mr_backward_bf16(const uint16_t* keys, const uint16_t* values, const uint1
                        void* stream);
 
 /*
+ * The same with the key, value and query gradients rounded to bfloat16 (to
+ * nearest, ties to even) as they are stored: a bfloat16 model's gradients
+ * without a float32 copy of them.
+ */
+int m4mr_backward_bf16_to_bf16(const uint16_t* keys, const uint16_t* values, const uint16_t* queries,
+                       const float* beta, const float* log_decay, const float* floor,
+                       int B, int T, int H, int value_dim, int chunk,
+                       const float* solved, const float* factors,
+                       const float* start_evidence, const float* start_cross,
+                       const float* d_output, const float* d_variance,
+                       const float* d_final_evidence, const float* d_final_cross,
+                       uint16_t* d_keys, uint16_t* d_values, uint16_t* d_queries,
+                       float* d_beta, float* d_log_decay, float* d_floor,
+                       float* d_init_evidence, float* d_init_cross,
+                       void* workspace, size_t workspace_bytes,
+                       void* stream);
+
+/*
  * m4mr_backward that allocates nothing and takes no workspace.  No
  * counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under HIP graph capture, serving and training loops

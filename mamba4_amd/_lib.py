@@ -90,6 +90,10 @@ SIGNATURES = {
         _I,
         [_P] * 6 + [_I] * 5 + [_P] * 4 + [_P] * 4 + [_P] * 8 + [_P, _S, _P],
     ),
+    "m4mr_backward_bf16_to_bf16": (
+        _I,
+        [_P] * 6 + [_I] * 5 + [_P] * 4 + [_P] * 4 + [_P] * 8 + [_P, _S, _P],
+    ),
     "m4mr_backward_noalloc": (
         _I,
         [_P] * 6 + [_I] * 5 + [_P] * 4 + [_P] * 4 + [_P] * 8 + [_P],

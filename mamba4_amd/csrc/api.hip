@@ -49,11 +49,11 @@ template <typename In, bool MIX, bool GATE, int NV>
 __global__ void bwd_dy_kernel(Dims, const In*, const In*, const In*, const float*,
                               const float*, const float*, const float*, const float*, float*,
                               MixerIn, MixerGrad);
-template <typename In, bool MIX, bool GATE, int NV>
+template <typename In, bool MIX, bool GATE, int NV, typename Out>
 __global__ void bwd_grads_kernel(Dims, const In*, const In*, const float*, const float*,
                                  const float*, const float*, const float*, const float*,
-                                 const float*, const float*, const float*, const float*, float*,
-                                 float*, float*, float*, float*, float*, MixerIn, MixerGrad);
+                                 const float*, const float*, const float*, const float*, Out*,
+                                 Out*, Out*, float*, float*, float*, MixerIn, MixerGrad);
 __global__ void floor_reduce_kernel(Dims, const float*, float*, const float*);
 __global__ void mixer_finish_kernel(Dims, const float*, float*, const float*, const float*,
                                     const float*, float*, float*, float*, float*, float*);
@@ -184,10 +184,13 @@ int configure() {
       {(const void*)m4::bwd_dy_kernel<m4::bf16_t, false, false, NV>, kChunkLdsBytes},         \
       {(const void*)m4::bwd_dy_kernel<float, true, false, NV>, kChunkLdsBytes},               \
       {(const void*)m4::bwd_dy_kernel<float, true, true, NV>, kChunkLdsBytes},                \
-      {(const void*)m4::bwd_grads_kernel<float, false, false, NV>, kGradsLdsBytes},           \
-      {(const void*)m4::bwd_grads_kernel<m4::bf16_t, false, false, NV>, kGradsLdsBytes},      \
-      {(const void*)m4::bwd_grads_kernel<float, true, false, NV>, kGradsLdsBytes},            \
-      {(const void*)m4::bwd_grads_kernel<float, true, true, NV>, kGradsGateLdsBytes}
+      {(const void*)m4::bwd_grads_kernel<float, false, false, NV, float>, kGradsLdsBytes},    \
+      {(const void*)m4::bwd_grads_kernel<m4::bf16_t, false, false, NV, float>,                \
+       kGradsLdsBytes},                                                                       \
+      {(const void*)m4::bwd_grads_kernel<m4::bf16_t, false, false, NV, m4::bf16_t>,           \
+       kGradsLdsBytes},                                                                       \
+      {(const void*)m4::bwd_grads_kernel<float, true, false, NV, float>, kGradsLdsBytes},     \
+      {(const void*)m4::bwd_grads_kernel<float, true, true, NV, float>, kGradsGateLdsBytes}
              M4_CHUNK_ATTRS(1),
              M4_CHUNK_ATTRS(2),
 #undef M4_CHUNK_ATTRS
@@ -493,13 +496,13 @@ int forward_impl(const char* entry, const In* keys, const In* values, const In* 
 // d_keys, d_queries, d_beta, d_log_decay and d_variance are unused, d_floor
 // is the floor_raw gradient); the per-head parameter partials are left in
 // mg.dy_part and mg.grads_part for the caller's head sums.
-template <typename In, bool MIX, bool GATE = false>
+template <typename In, bool MIX, bool GATE = false, typename Out = float>
 int backward_impl(const char* entry, const In* keys, const In* values, const In* queries,
                   const float* beta, const float* log_decay, const float* floor, int B, int T,
                   int H, int value_dim, int chunk, const float* solved, const float* factors,
                   const float* start_evidence, const float* start_cross, const float* d_output,
                   const float* d_variance, const float* d_final_evidence,
-                  const float* d_final_cross, float* d_keys, float* d_values, float* d_queries,
+                  const float* d_final_cross, Out* d_keys, Out* d_values, Out* d_queries,
                   float* d_beta, float* d_log_decay, float* d_floor, float* d_init_evidence,
                   float* d_init_cross, void* workspace, size_t workspace_bytes, void* stream,
                   const m4::MixerIn& mix = {}, bool spill_free = false,
@@ -514,7 +517,7 @@ int backward_impl(const char* entry, const In* keys, const In* values, const In*
     if (mix.previous && misaligned(mix.previous))
       return fail(M4MR_EINVAL, std::string(entry) + ": arrays must be 16-byte aligned");
   }
-  if (GATE) {
+  if constexpr (GATE) {
     // The gated backward's own outputs and inputs stand in for the plain ones.
     d_output = mg.d_out;
     d_variance = mg.d_var;
@@ -600,8 +603,8 @@ int backward_impl(const char* entry, const In* keys, const In* values, const In*
   }
   if (rc) return rc;
   rc = launch("bwd_grads", st, [&] {
-    const auto grads = d.NV == 1 ? m4::bwd_grads_kernel<In, MIX, GATE, 1>
-                                 : m4::bwd_grads_kernel<In, MIX, GATE, 2>;
+    const auto grads = d.NV == 1 ? m4::bwd_grads_kernel<In, MIX, GATE, 1, Out>
+                                 : m4::bwd_grads_kernel<In, MIX, GATE, 2, Out>;
     hipLaunchKernelGGL(grads, dim3(persistent_grid(seqs, 1)),
                        dim3(512), GATE ? kGradsGateLdsBytes : kGradsLdsBytes, st, d, keys,
                        values, beta, log_decay, solved,
@@ -858,7 +861,7 @@ int m4mr_mixer_read_backward(const float* key, const float* value, const float* 
   mg.d_beta_bias = d_beta_bias;
   mg.d_dt_bias = d_dt_bias;
   mg.d_a_log = d_a_log;
-  return backward_impl<float, true, true>(
+  return backward_impl<float, true, true, float>(
       entry, nullptr, value, nullptr, beta, log_decay, floor, B, T, H, value_dim, chunk, solved,
       factors, start_evidence, start_cross, nullptr, nullptr, d_final_evidence, d_final_cross,
       nullptr, d_value, nullptr, nullptr, nullptr, d_floor_raw, d_init_evidence, d_init_cross,
@@ -914,6 +917,25 @@ int m4mr_backward_bf16(const uint16_t* keys, const uint16_t* values, const uint1
                        d_output, d_variance, d_final_evidence, d_final_cross, d_keys, d_values,
                        d_queries, d_beta, d_log_decay, d_floor, d_init_evidence, d_init_cross,
                        workspace, workspace_bytes, stream);
+}
+
+int m4mr_backward_bf16_to_bf16(
+    const uint16_t* keys, const uint16_t* values, const uint16_t* queries, const float* beta,
+    const float* log_decay, const float* floor, int B, int T, int H, int value_dim, int chunk,
+    const float* solved, const float* factors, const float* start_evidence,
+    const float* start_cross, const float* d_output, const float* d_variance,
+    const float* d_final_evidence, const float* d_final_cross, uint16_t* d_keys,
+    uint16_t* d_values, uint16_t* d_queries, float* d_beta, float* d_log_decay, float* d_floor,
+    float* d_init_evidence, float* d_init_cross, void* workspace, size_t workspace_bytes,
+    void* stream) {
+  return backward_impl<m4::bf16_t, false, false, m4::bf16_t>(
+      "m4mr_backward_bf16_to_bf16", reinterpret_cast<const m4::bf16_t*>(keys),
+      reinterpret_cast<const m4::bf16_t*>(values), reinterpret_cast<const m4::bf16_t*>(queries),
+      beta, log_decay, floor, B, T, H, value_dim, chunk, solved, factors, start_evidence,
+      start_cross, d_output, d_variance, d_final_evidence, d_final_cross,
+      reinterpret_cast<m4::bf16_t*>(d_keys), reinterpret_cast<m4::bf16_t*>(d_values),
+      reinterpret_cast<m4::bf16_t*>(d_queries), d_beta, d_log_decay, d_floor, d_init_evidence,
+      d_init_cross, workspace, workspace_bytes, stream);
 }
 
 int m4mr_backward_noalloc(const float* keys, const float* values, const float* queries,

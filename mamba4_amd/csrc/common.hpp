@@ -27,6 +27,21 @@ __device__ __forceinline__ f4 load4(const bf16_t* p) {
             __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u)};
 }
 __device__ __forceinline__ float load1(const float* p) { return *p; }
+// Two and four float32 values to consecutive elements, rounded to the nearest
+// bfloat16 (ties to even) for bf16_t.
+__device__ __forceinline__ void store2(float* p, float2 v) { *reinterpret_cast<float2*>(p) = v; }
+__device__ __forceinline__ void store4(float* p, f4 v) { *reinterpret_cast<f4*>(p) = v; }
+__device__ __forceinline__ unsigned bf16_pair(float x, float y) {
+  typedef __bf16 pair __attribute__((ext_vector_type(2)));
+  typedef float two __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(two{x, y}, pair));
+}
+__device__ __forceinline__ void store2(bf16_t* p, float2 v) {
+  *reinterpret_cast<unsigned*>(p) = bf16_pair(v.x, v.y);
+}
+__device__ __forceinline__ void store4(bf16_t* p, f4 v) {
+  *reinterpret_cast<uint2*>(p) = uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
+}
 
 // Raw buffer loads: an offset at or past the resource's byte size reads zero
 // without a memory access, so rows past a chunk's end need no branch (and a

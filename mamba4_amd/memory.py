@@ -186,7 +186,7 @@ class _MemoryRead(torch.autograd.Function):
     def backward(ctx, d_output, d_variance, d_final_s, d_final_c):
         dim, value_dim = ctx.dims
         grads = memread_backward(*ctx.saved_tensors, ctx.chunk, d_output, d_variance,
-                                 d_final_s, d_final_c)
+                                 d_final_s, d_final_c, narrow=True)
         d_keys, d_values, d_queries, d_floor, d_init_s, d_init_c = _resized(
             (grads[0], None, dim, 0), (grads[1], None, value_dim, 0), (grads[2], None, dim, 0),
             (grads[5], None, dim, 0),
@@ -197,10 +197,12 @@ class _MemoryRead(torch.autograd.Function):
 
 
 def memread_backward(keys, values, queries, beta, log_decay, floor, solved, factors, start_s,
-                     start_c, chunk, d_output, d_variance, d_final_s, d_final_c, mixer=None):
+                     start_c, chunk, d_output, d_variance, d_final_s, d_final_c, mixer=None,
+                     narrow=False):
     """m4mr_backward on the forward's inputs and residual set: returns
     (d_keys, d_values, d_queries, d_beta, d_log_decay, d_floor, d_init_evidence,
-    d_init_cross), all float32.  None cotangents are zero.  With
+    d_init_cross), all float32, or with ``narrow`` the first three in the
+    keys' dtype.  None cotangents are zero.  With
     ``mixer = (previous, key_shift)``, keys and queries are the mixer's raw
     projections and m4mr_mixer_backward normalises them on load (the
     gradients are still those of the normalised keys and queries)."""
@@ -218,8 +220,10 @@ def memread_backward(keys, values, queries, beta, log_decay, floor, solved, fact
     d_final_s = None if d_final_s is None else d_final_s.to(torch.float32).contiguous()
     d_final_c = None if d_final_c is None else d_final_c.to(torch.float32).contiguous()
     f32 = dict(dtype=torch.float32, device=keys.device)
-    grads = [torch.empty(t.shape, **f32) for t in (keys, values, queries, beta, log_decay,
-                                                    floor)]
+    narrow = narrow and keys.dtype == torch.bfloat16
+    rows = dict(dtype=torch.bfloat16, device=keys.device) if narrow else f32
+    grads = [torch.empty(t.shape, **(rows if i < 3 else f32))
+             for i, t in enumerate((keys, values, queries, beta, log_decay, floor))]
     d_init_s = torch.empty((batch, heads, _lib.KEY_DIM, _lib.KEY_DIM), **f32)
     d_init_c = torch.empty((batch, heads, width, _lib.KEY_DIM), **f32)
     nbytes = lib.m4mr_backward_workspace_bytes(batch, time, heads, width, chunk)
@@ -233,7 +237,9 @@ def memread_backward(keys, values, queries, beta, log_decay, floor, solved, fact
         previous, key_shift = mixer
         _lib.check(lib.m4mr_mixer_backward(*head, _ptr(previous), int(key_shift), *tail))
     else:
-        entry = lib.m4mr_backward_bf16 if keys.dtype == torch.bfloat16 else lib.m4mr_backward
+        entry = (lib.m4mr_backward_bf16_to_bf16 if narrow
+                 else lib.m4mr_backward_bf16 if keys.dtype == torch.bfloat16
+                 else lib.m4mr_backward)
         _lib.check(entry(*head, *tail))
     return (*grads, d_init_s, d_init_c)
 
