@@ -113,6 +113,8 @@ const char* const kKernelNames[] = {"fwd_stats",      "fwd_scan",  "fwd_states",
                                     "order_carry",    "order_apply", "order_bwd_local",
                                     "order_bwd_carry", "order_bwd_apply", "order_walk", "order_bwd_walk",
                                     "m3_walk",        "m3_out",    "m3_walk_bwd", "m3_grad",
+                                    "m3_phases",      "m3_local",  "m3_carry",    "m3_local_bwd",
+                                    "m3_carry_bwd",
                                     "m3_finish",      "m3_bias",   "m3_suffix",
                                     "mixer_finish",   "diag_eigen", "diag_summary",
                                     "spd_wide",       "spd_wide_backward", "resize"};
@@ -201,20 +203,28 @@ int configure() {
              {(const void*)m4::states_kernel<false, float, true, 2>, kStatesLdsBytes},
              {(const void*)m4::states_kernel<true, float, true, 2>,
               kStatesLdsBytes + kStatesBwdExtra},
-             {(const void*)m3::walk_kernel<false, float, true>, m3::kWalkLds},
-             {(const void*)m3::walk_kernel<true, float, true>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<false, float, true, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<false, float, true, true>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<true, float, true, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<true, float, true, true>, m3::kWalkLds},
              {(const void*)m3::out_kernel<float, true>, m3::kOutLds},
              {(const void*)m3::grad_kernel<float, true>, m3::kGradLds},
-             {(const void*)m3::walk_kernel<false, m3::bf16_t, true>, m3::kWalkLds},
-             {(const void*)m3::walk_kernel<true, m3::bf16_t, true>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<false, m3::bf16_t, true, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<false, m3::bf16_t, true, true>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<true, m3::bf16_t, true, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<true, m3::bf16_t, true, true>, m3::kWalkLds},
              {(const void*)m3::out_kernel<m3::bf16_t, true>, m3::kOutLdsBf16},
              {(const void*)m3::grad_kernel<m3::bf16_t, true>, m3::kGradLds},
-             {(const void*)m3::walk_kernel<false, float, false>, m3::kWalkLds},
-             {(const void*)m3::walk_kernel<true, float, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<false, float, false, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<false, float, false, true>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<true, float, false, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<true, float, false, true>, m3::kWalkLds},
              {(const void*)m3::out_kernel<float, false>, m3::kOutLds},
              {(const void*)m3::grad_kernel<float, false>, m3::kGradLds},
-             {(const void*)m3::walk_kernel<false, m3::bf16_t, false>, m3::kWalkLds},
-             {(const void*)m3::walk_kernel<true, m3::bf16_t, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<false, m3::bf16_t, false, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<false, m3::bf16_t, false, true>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<true, m3::bf16_t, false, false>, m3::kWalkLds},
+             {(const void*)m3::walk_kernel<true, m3::bf16_t, false, true>, m3::kWalkLds},
              {(const void*)m3::out_kernel<m3::bf16_t, false>, m3::kOutLdsBf16},
              {(const void*)m3::grad_kernel<m3::bf16_t, false>, m3::kGradLds},
              {(const void*)m3::finish_kernel, m3::kFinishLdsMax},
@@ -1502,6 +1512,24 @@ int m3_groups(int B, int T, int H) {
   return (int)((H + hpg - 1) / hpg);
 }
 
+// Whether the Mamba-3 states are formed chunk by chunk in parallel and then
+// carried (walk_kernel's SPLIT and carry_kernel) rather than walked.  A walk
+// takes, per chunk, 4.7 us with at most one half-sequence block per compute
+// unit, 6.1 with two, 8.1 with three (resident at once; more take turns); the
+// split form about 10 us, 8 more per further sixteen chunks of phases, and
+// 0.033 per sequence and chunk.  Forward + backward, walk against split: B1
+// T1000 H24 77 + 77 / 31 + 21 us, B4 T1024 H24 80 + 79 / 67 + 56, B8 T1024 H24
+// 102 + 100 / 118 + 107, B1 T128 H2 13 + 12 / 16 + 13.  The split is taken
+// where it is estimated 10% faster.
+bool m3_split_walk(int B, int H, int NC) {
+  if (NC > 65535) return false;  // a grid dimension
+  const double blocks = 2.0 * B * H, cus = g_cus;
+  const double step = blocks <= cus ? 4.7 : blocks <= 2 * cus ? 6.1 : 8.1;
+  const double walk = NC * step * std::ceil(blocks / (3 * cus));
+  const double split = 10.0 + 8.0 * ((NC - 1) / 16) + 0.033 * B * H * NC;
+  return split < 0.9 * walk;
+}
+
 struct M3Workspace {
   float *dh1, *dgam, *dscale, *ddt_loc, *D, *qb_part, *kb_part, *dc_part, *db_part, *dang_part;
 };
@@ -1572,12 +1600,34 @@ int m3_forward_impl(const char* entry, const In* c, const In* b, const In* x, co
   const m3::Shape s{B, T, H, N, P, A, (T + m3::C - 1) / m3::C};
   // Value rows load as 4-element vectors when P allows (a kernel per case).
   const bool v4 = P % 4 == 0;
-  const auto walk = v4 ? m3::walk_kernel<false, In, true> : m3::walk_kernel<false, In, false>;
   const auto out = v4 ? m3::out_kernel<In, true> : m3::out_kernel<In, false>;
-  int rc = launch("m3_walk", st, [&] {
-    hipLaunchKernelGGL(walk, dim3(2 * B * H), dim3(256), m3::kWalkLds, st, s, b, k_bias, x, adt, dt,
-                       trap_logits, angles, phases, starts, nullptr, final_state);
-  });
+  int rc;
+  if (m3_split_walk(B, H, s.NC)) {
+    if (A > 0) {
+      rc = launch("m3_phases", st, [&] {
+        hipLaunchKernelGGL(m3::phase_kernel, dim3(B * H), dim3(1024), 0, st, s, dt, angles, phases);
+      });
+      if (rc) return rc;
+    }
+    const auto local = v4 ? m3::walk_kernel<false, In, true, true>
+                          : m3::walk_kernel<false, In, false, true>;
+    rc = launch("m3_local", st, [&] {
+      hipLaunchKernelGGL(local, dim3(2 * B * H, s.NC), dim3(256), m3::kWalkLds, st, s, b, k_bias, x,
+                         adt, dt, trap_logits, angles, phases, starts, nullptr, nullptr);
+    });
+    if (rc) return rc;
+    rc = launch("m3_carry", st, [&] {
+      hipLaunchKernelGGL(m3::carry_kernel<false>, dim3(B * H, 8), dim3(256), 0, st, s, adt, starts,
+                         final_state);
+    });
+  } else {
+    const auto walk = v4 ? m3::walk_kernel<false, In, true, false>
+                         : m3::walk_kernel<false, In, false, false>;
+    rc = launch("m3_walk", st, [&] {
+      hipLaunchKernelGGL(walk, dim3(2 * B * H), dim3(256), m3::kWalkLds, st, s, b, k_bias, x, adt,
+                         dt, trap_logits, angles, phases, starts, nullptr, final_state);
+    });
+  }
   if (rc) return rc;
   // bfloat16 tiles: two blocks per compute unit.
   const bool bf = std::is_same<In, m3::bf16_t>::value;
@@ -1621,13 +1671,30 @@ int m3_backward_impl(const char* entry, const In* c, const In* b, const In* x, c
                       ws.ddt_loc,  ws.D,         ws.qb_part,    ws.kb_part,
                       ws.dc_part,  ws.db_part,   ws.dang_part};
   const bool v4 = P % 4 == 0;
-  const auto walk = v4 ? m3::walk_kernel<true, In, true> : m3::walk_kernel<true, In, false>;
   const auto grad = v4 ? m3::grad_kernel<In, true> : m3::grad_kernel<In, false>;
-  int rc = launch("m3_walk_bwd", st, [&] {
-    hipLaunchKernelGGL(walk, dim3(2 * B * H), dim3(256), m3::kWalkLds, st, s, c, q_bias, d_y, adt, dt,
-                       trap_logits, angles, const_cast<float*>(phases), ws.dh1, d_final,
-                       nullptr);
-  });
+  int rc;
+  if (m3_split_walk(B, H, s.NC)) {
+    const auto local = v4 ? m3::walk_kernel<true, In, true, true>
+                          : m3::walk_kernel<true, In, false, true>;
+    rc = launch("m3_local_bwd", st, [&] {
+      hipLaunchKernelGGL(local, dim3(2 * B * H, s.NC), dim3(256), m3::kWalkLds, st, s, c, q_bias,
+                         d_y, adt, dt, trap_logits, angles, const_cast<float*>(phases), ws.dh1,
+                         nullptr, nullptr);
+    });
+    if (rc) return rc;
+    rc = launch("m3_carry_bwd", st, [&] {
+      hipLaunchKernelGGL(m3::carry_kernel<true>, dim3(B * H, 8), dim3(256), 0, st, s, adt, ws.dh1,
+                         const_cast<float*>(d_final));
+    });
+  } else {
+    const auto walk = v4 ? m3::walk_kernel<true, In, true, false>
+                         : m3::walk_kernel<true, In, false, false>;
+    rc = launch("m3_walk_bwd", st, [&] {
+      hipLaunchKernelGGL(walk, dim3(2 * B * H), dim3(256), m3::kWalkLds, st, s, c, q_bias, d_y, adt,
+                         dt, trap_logits, angles, const_cast<float*>(phases), ws.dh1, d_final,
+                         nullptr);
+    });
+  }
   if (rc) return rc;
   rc = launch("m3_grad", st, [&] {
     hipLaunchKernelGGL(grad, dim3(B * s.NC * groups), dim3(512), m3::kGradLds, st, s, groups, c,

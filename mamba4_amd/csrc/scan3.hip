@@ -918,7 +918,12 @@ __device__ __forceinline__ void store_state_t(const f4 (&v)[2048 / NTH], TT* dst
 // [C][LA] (columns = the half's angles), th0 [AM], scalars.
 constexpr int LQH = 64 + 4;
 
-template <bool BWD, typename In, bool V4>
+// SPLIT: one block per (b, h, half, chunk) instead, for few sequences: each
+// chunk's own contribution from zero goes where the walk puts the state it
+// starts from, the start phases come from phase_kernel and carry_kernel turns
+// the contributions into states.  B2 T1000 H24 (96 blocks of sixteen steps
+// otherwise): forward 78 -> 43 us, backward 77 -> 33.
+template <bool BWD, typename In, bool V4, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void walk_kernel(
     Shape s, const In* rows, const float* bias, const In* vals, const float* adt, const float* dt,
     const float* trap, const float* ang, float* theta0, float* saved, const float* init,
@@ -957,11 +962,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
     for (int i = 0; i < 4; ++i) {
       const int n = n0 + 16 * w + 4 * q + i, p = 16 * j + r;
       float v = 0.f;
-      if (BWD && init && n < s.N && p < s.P) v = init[(((long)b * s.H + h) * s.N + n) * s.P + p];
+      if (BWD && !SPLIT && init && n < s.N && p < s.P) v = init[(((long)b * s.H + h) * s.N + n) * s.P + p];
       acc[j][i] = v;
     }
   }
-  if (!BWD && tid < AM) th0[tid] = 0.f;
+  if (!BWD && !SPLIT && tid < AM) th0[tid] = 0.f;
   // This lane's coordinate pair (32 per half, two tokens per wave step).
   const int pr = l & 31, n = n0 + 2 * pr;
   const bool col = n < s.N;
@@ -984,7 +989,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
         rates[k] = ldb(ra, jj < na ? (t * s.A + j0 + jj) * 4 : kNoLoad);
       }
     }
-    if (BWD)
+    if (BWD || SPLIT)
       th_in = ldb(rsrc(theta0 + phase_offset(s, b, h, c) + j0, 4L * na), tid < 64 ? tid * 4 : kNoLoad);
     const Rsrc rr = chunk_rsrc(s, rows, b, c, s.N);
 #pragma unroll
@@ -994,15 +999,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
     }
     fetch_values<256, V4>(s, vals, b, c, h, v);
   };
-  fetch(BWD ? s.NC - 1 : 0);
+  fetch(SPLIT ? blockIdx.y : BWD ? s.NC - 1 : 0);
 
-  for (int step = 0; step < s.NC; ++step) {
-    const int c = BWD ? s.NC - 1 - step : step;
+  const int steps = SPLIT ? 1 : s.NC;
+  for (int step = 0; step < steps; ++step) {
+    const int c = SPLIT ? (int)blockIdx.y : BWD ? s.NC - 1 - step : step;
     __syncthreads();  // the previous chunk's reads of the LDS tiles are done
     // This chunk's state (a lane's four rows of one column), stored by waves
     // 1-3 while wave 0 turns the token inputs into the chunk's scalars.
     float* out = saved + state_offset(s, b, h, c);
-    if (w != 0) {
+    if (!SPLIT && w != 0) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -1014,7 +1020,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
       const int e = tid + 256 * k;
       tab[(e >> 5) * LA + (e & 31)] = rates[k];
     }
-    if (BWD) {
+    if (BWD || SPLIT) {
       if (tid < na) th0[tid] = th_in;
     } else {
       // Lanes at or past the half's angles store out of range (dropped).
@@ -1042,7 +1048,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
         const int jj = w + 4 * m;
         if (jj < na) {
           tab[l * LA + jj] = x[m];
-          if (!BWD && l == 63) th0[jj] = reduce_turns(x[m]);
+          if (!BWD && !SPLIT && l == 63) th0[jj] = reduce_turns(x[m]);
         }
       }
     }
@@ -1065,21 +1071,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
     store_values<256>(v, BWD ? S.ep : S.u, vt);
     // The next chunk's inputs (this chunk's again after the last: every
     // iteration issues the same loads), then wave 0's rows of the state.
-    fetch(step + 1 < s.NC ? (BWD ? c - 1 : c + 1) : c);
-    if (w == 0) {
+    if (!SPLIT) fetch(step + 1 < s.NC ? (BWD ? c - 1 : c + 1) : c);
+    if (!SPLIT && w == 0) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) out[(n0 + 16 * w + 4 * q + i) * PT + 16 * j + r] = acc[j][i];
     }
     __syncthreads();
-    const float decay = expf(S.p[63]);
+    if (!SPLIT) {
+      const float decay = expf(S.p[63]);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] *= decay;
+      for (int j = 0; j < 4; ++j) acc[j] *= decay;
+    }
     // rows^T vals: A(n, t) = rt[t * LQH + n], B(t, p) = vt[t * LV + p].
     mma<4, 1, LQH, LV, 1, BF>(acc, rt, 16 * w, vt, 0, 0, C);
+    if (SPLIT) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[(n0 + 16 * w + 4 * q + i) * PT + 16 * j + r] = acc[j][i];
+    }
   }
-  if (!BWD && final_state) {
+  if (!BWD && !SPLIT && final_state) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -1090,6 +1104,107 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
       }
   }
 }
+
+// The split walk's start phases: one sixteen-wave block per (b, h), a chunk
+// per wave and sixteen chunks a step.  theta0[c] = the phase that walk_kernel
+// carries to chunk c, with its arithmetic (each chunk's scan of angle times
+// dt, a token per lane, reduced modulo 2 pi at its end): the same to the bit.
+// Bound by its loads, which touch a line per lane: four angles a load where
+// their count allows (T = 1000, A = 32: 10 us, one by one 18).
+__global__ __launch_bounds__(1024) void phase_kernel(Shape s, const float* dt, const float* ang,
+                                                     float* theta0) {
+  __shared__ float total[16][AM];
+  const int bh = blockIdx.x, b = bh / s.H, h = bh % s.H;
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+  const bool quads = s.A % 4 == 0;
+  float phase = 0.f;  // thread j < A: angle j
+  for (int first = 0; first < s.NC; first += 16) {
+    const int c = first + w;
+    if (c < s.NC) {  // uniform over the wave
+      const float d = ldb(chunk_rsrc(s, dt, b, c, s.H), (l * s.H + h) * 4);
+      const Rsrc ra = chunk_rsrc(s, ang, b, c, s.A);
+      for (int j0 = 0; j0 < s.A; j0 += 32) {
+        f4 x[8];
+        if (quads) {
+#pragma unroll
+          for (int m = 0; m < 8; ++m)
+            x[m] = raw4(ra, j0 + 4 * m < s.A ? (l * s.A + j0 + 4 * m) * 4 : kNoLoad, ang);
+        } else {
+#pragma unroll
+          for (int m = 0; m < 8; ++m)
+            x[m] = raw4_n(ra, (l * s.A + j0 + 4 * m) * 4, s.A - (j0 + 4 * m), ang);
+        }
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float sum = wave_scan(x[m][k] * d);
+            if (l == 63 && j0 + 4 * m + k < s.A) total[w][j0 + 4 * m + k] = sum;
+          }
+      }
+    }
+    __syncthreads();
+    if (tid < s.A)
+      for (int k = 0; k < 16 && first + k < s.NC; ++k) {
+        theta0[phase_offset(s, b, h, first + k) + tid] = phase;
+        phase = reduce_turns(phase + total[k][tid]);
+      }
+    __syncthreads();
+  }
+}
+
+// The split walk's carry: saved[c] holds each chunk's own contribution and
+// becomes the state the chunk starts from (BWD: the cotangent at its end),
+// chunk by chunk, a quad of the state per thread.  Forward writes the state
+// after the last chunk to `boundary` [N,P] (may be NULL), backward starts
+// from it.
+template <bool BWD>
+__global__ __launch_bounds__(256) void carry_kernel(Shape s, const float* adt, float* saved,
+                                                    float* boundary) {
+  __shared__ float decay[64];
+  const int bh = blockIdx.x, b = bh / s.H, h = bh % s.H;
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+  const int e = (blockIdx.y * 256 + tid) * 4, n = e / PT, p = e % PT;  // NT * PT / 4 threads
+  float* edge = boundary ? boundary + (((long)b * s.H + h) * s.N + n) * s.P + p : nullptr;
+  f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+  if (BWD && edge && n < s.N)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (p + k < s.P) acc[k] = edge[k];
+  for (int first = 0; first < s.NC; first += 64) {
+    const int count = min(64, s.NC - first);
+    __syncthreads();  // the previous step's decays are read
+    for (int k = w; k < count; k += 4) {
+      const int c = BWD ? s.NC - 1 - (first + k) : first + k, t = c * C + l;
+      const float a = t < s.T ? adt[((long)b * s.T + t) * s.H + h] : 0.f;
+      const float total = wave_scan(a);
+      if (l == 63) decay[k] = expf(total);
+    }
+    __syncthreads();
+    for (int k0 = 0; k0 < count; k0 += 8) {
+      f4 own[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = first + min(k0 + j, count - 1);
+        own[j] = *reinterpret_cast<const f4*>(
+            saved + state_offset(s, b, h, BWD ? s.NC - 1 - k : k) + e);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (k0 + j < count) {
+          const int k = first + k0 + j;
+          *reinterpret_cast<f4*>(saved + state_offset(s, b, h, BWD ? s.NC - 1 - k : k) + e) = acc;
+          acc = decay[k0 + j] * acc + own[j];
+        }
+    }
+  }
+  if (!BWD && edge && n < s.N)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (p + k < s.P) edge[k] = acc[k];
+}
+template __global__ void carry_kernel<false>(Shape, const float*, float*, float*);
+template __global__ void carry_kernel<true>(Shape, const float*, float*, float*);
 
 // Block index -> (b, chunk, h), heads fastest.  Consecutive blocks land on
 // different XCDs (round robin over 8); the remap gives each XCD a contiguous
@@ -1969,15 +2084,15 @@ __global__ __launch_bounds__(1024) void bias_kernel(Shape s, GradOut o, float* d
   }
 }
 
+#define M3_WALK_KERNEL(BWD, In, V4, SPLIT)                                                     \
+  template __global__ void walk_kernel<BWD, In, V4, SPLIT>(                                      \
+      Shape, const In*, const float*, const In*, const float*, const float*, const float*,       \
+      const float*, float*, float*, const float*, float*);
 #define M3_SCAN_KERNELS(In, V4)                                                                \
-  template __global__ void walk_kernel<false, In, V4>(Shape, const In*, const float*, const In*, \
-                                                      const float*, const float*, const float*,  \
-                                                      const float*, float*, float*,              \
-                                                      const float*, float*);                     \
-  template __global__ void walk_kernel<true, In, V4>(Shape, const In*, const float*, const In*,  \
-                                                     const float*, const float*, const float*,   \
-                                                     const float*, float*, float*, const float*, \
-                                                     float*);                                    \
+  M3_WALK_KERNEL(false, In, V4, false)                                                           \
+  M3_WALK_KERNEL(true, In, V4, false)                                                            \
+  M3_WALK_KERNEL(false, In, V4, true)                                                            \
+  M3_WALK_KERNEL(true, In, V4, true)                                                             \
   template __global__ void out_kernel<In, V4>(Shape, const In*, const In*, const In*,            \
                                               const float*, const float*, const float*,          \
                                               const float*, const float*, const float*,          \

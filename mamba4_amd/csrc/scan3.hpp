@@ -59,7 +59,8 @@ inline size_t finish_lds(int H, int A) {
 // In: the model dtype of the rows, values and their cotangents (float, or
 // bf16_t with the reference's bfloat16 matrix operands).  V4: the value width
 // P is a multiple of 4 (vector loads of value rows; otherwise per element).
-template <bool BWD, typename In, bool V4>
+// SPLIT: one chunk per block, the states then carried by carry_kernel.
+template <bool BWD, typename In, bool V4, bool SPLIT>
 __global__ void walk_kernel(Shape, const In*, const float*, const In*, const float*,
                             const float*, const float*, const float*, float*, float*,
                             const float*, float*);
@@ -71,6 +72,9 @@ template <typename In, bool V4>
 __global__ void grad_kernel(Shape, int, const In*, const In*, const In*, const float*,
                             const float*, const float*, const float*, const float*, const float*,
                             const float*, const float*, const float*, const In*, GradOut);
+__global__ void phase_kernel(Shape, const float*, const float*, float*);
+template <bool BWD>
+__global__ void carry_kernel(Shape, const float*, float*, float*);
 __global__ void finish_kernel(Shape, int, const float*, const float*, const float*, GradOut,
                               float*, float*, float*, float*, float*);
 __global__ void suffix_kernel(Shape, GradOut);
