@@ -146,14 +146,14 @@ __device__ __forceinline__ float row_value(float x, int mu) {
 }
 
 // Wave W's half of the evidence that its pair's spans start from, to LDS: the
-// sub-chunks' start states times -c, then the rank-one updates of the
-// `catchup` tokens before each span (per 16-lane row; the first is sequence
-// token `first`).  A token's update is the turn's, a product by the decay and
-// one multiply-add, here on the rank-one four-block fp32 MFMA over blocks in
-// the exchanged layout (rows16.hpp), so a token's evidence is the same to the
-// bit however its sub-chunk is split.  Per wave and token 80 multiplies and
-// five MFMAs; on DPP-fed multiply-adds in the row layout (224 instructions)
-// a token took 0.75 us; it takes 0.42.
+// sub-chunk's start states times -c, decayed over the `catchup` tokens before
+// each span (per 16-lane row; the first is sequence token `first`), and their
+// weighted outer products.  Those are summed from the last token back, each
+// weighted by the decays after it, on the rank-one four-block fp32 MFMA (one
+// rounding per token and element, as the turns' updates have) over blocks in
+// the exchanged layout (rows16.hpp).  Per wave and token five MFMAs; applying
+// the turns' updates one by one took 0.42 us a token with the same MFMAs, and
+// 0.75 on DPP-fed multiply-adds in the row layout, instead of 0.28.
 template <typename In, bool MIX, int W>
 __device__ __forceinline__ void stage_evidence(f4* evidence, const float* start_s, int slot,
                                                float c, int sexp, int catchup, int first,
@@ -163,68 +163,61 @@ __device__ __forceinline__ void stage_evidence(f4* evidence, const float* start_
   const int lane = threadIdx.x & 63, a = lane & 15, g = lane >> 4;
   f16 E[5];
 #pragma unroll
-  for (int mu = 0; mu < 4; ++mu) {
-    const float* s0 = start_s + (long)__builtin_amdgcn_readlane(slot, 16 * mu) * 4096;
-    const float nc = -row_value(c, mu);
-    for_staged_blocks<W>([&](int i, int I, int K) {
-      const f4 v = *reinterpret_cast<const f4*>(s0 + (16 * I + a) * 64 + 16 * K + 4 * g);
+  for (int i = 0; i < 5; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) E[i][4 * mu + e] = nc * v[e];
-    });
-  }
+    for (int r = 0; r < 16; ++r) E[i][r] = 0.f;
   const int most = wave_max4(catchup);
   // A group's inputs are in flight while the previous group is applied.  Rows
   // without a token to catch up read one in bounds and take a zero update.
   TokenInputs cur[CATCHUP_GROUP], next[CATCHUP_GROUP];
   bool kzero[CATCHUP_GROUP] = {};
-  auto load = [&](TokenInputs (&in)[CATCHUP_GROUP], int from) {
+  auto load = [&](TokenInputs (&in)[CATCHUP_GROUP], int done) {
 #pragma unroll
     for (int j = 0; j < CATCHUP_GROUP; ++j) {
-      const int t = from + j < catchup ? first + from + j : 0;
+      const int back = catchup - 1 - (done + j), t = back >= 0 ? first + back : 0;
       if constexpr (MIX)
         load_token_mix(in[j], kzero[j], d, mix, beta, log_decay, b, h, t, a);
       else
         load_token(in[j], d, keys, keys, beta, log_decay, b, h, t, a);
     }
   };
+  float after = 0.f;  // summed log decays after the token
   if (most > 0) load(cur, 0);
-  for (int from = 0; from < most; from += CATCHUP_GROUP) {
+  for (int done = 0; done < most; done += CATCHUP_GROUP) {
     if constexpr (MIX)
 #pragma unroll
       for (int j = 0; j < CATCHUP_GROUP; ++j) mix_token(cur[j], kzero[j]);
-    load(next, from + CATCHUP_GROUP);
+    load(next, done + CATCHUP_GROUP);
 #pragma unroll
     for (int j = 0; j < CATCHUP_GROUP; ++j) {
-      const bool in = from + j < catchup;
-      const float lam = in ? expf(cur[j].log_lam) : 1.f;
-      const float cbeta = __builtin_ldexpf(cur[j].beta, 2 * sexp);
+      const bool in = done + j < catchup;
+      const float weight = __builtin_ldexpf(cur[j].beta, 2 * sexp) * expf(after);
       float k[4], nbk[4];
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         k[m] = in ? cur[j].k[m] : 0.f;
-        nbk[m] = in ? -cbeta * cur[j].k[m] : 0.f;
-      }
-#pragma unroll
-      for (int mu = 0; mu < 4; ++mu) {
-        const float l = row_value(lam, mu);
-        for_staged_blocks<W>([&](int i, int, int) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) E[i][4 * mu + e] *= l;
-        });
+        nbk[m] = in ? -weight * cur[j].k[m] : 0.f;
       }
       for_staged_blocks<W>([&](int i, int I, int K) {
         E[i] = __builtin_amdgcn_mfma_f32_16x16x1f32(k[K], nbk[I], E[i], 0, 0, 0);
       });
+      after += in ? cur[j].log_lam : 0.f;
     }
 #pragma unroll
     for (int j = 0; j < CATCHUP_GROUP; ++j) cur[j] = next[j];
   }
-  for_staged_blocks<W>([&](int i, int I, int K) {
+  const float scale = -c * expf(after);  // -c without a token before the span
 #pragma unroll
-    for (int mu = 0; mu < 4; ++mu)
+  for (int mu = 0; mu < 4; ++mu) {
+    const float* s0 = start_s + (long)__builtin_amdgcn_readlane(slot, 16 * mu) * 4096;
+    const float w = row_value(scale, mu);
+    for_staged_blocks<W>([&](int i, int I, int K) {
+      const f4 v = *reinterpret_cast<const f4*>(s0 + (16 * I + a) * 64 + 16 * K + 4 * g);
       evidence[slot_quad(I, 4 * K + g) * 64 + 16 * mu + a] =
-          f4{E[i][4 * mu], E[i][4 * mu + 1], E[i][4 * mu + 2], E[i][4 * mu + 3]};
-  });
+          f4{w * v[0] + E[i][4 * mu], w * v[1] + E[i][4 * mu + 1], w * v[2] + E[i][4 * mu + 2],
+             w * v[3] + E[i][4 * mu + 3]};
+    });
+  }
 }
 
 // A sequence is a span of a sub-chunk's tokens, 1/nspan of it (the launch
@@ -358,11 +351,8 @@ __global__ __launch_bounds__(128 * PAIRS) void fwd_factor_kernel(
         f4 sv = evidence[slot_quad(m, q) * 64 + lane];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          // The product by the decay rounded, then one multiply-add:
-          // stage_evidence's MFMA updates round the same way.
-#pragma clang fp contract(off)
           const int k = 4 * q + e;
-          sv[e] = __builtin_fmaf(nbk, bcast16(cur.k[k >> 4], k & 15), lam * sv[e]);
+          sv[e] = lam * sv[e] + nbk * bcast16(cur.k[k >> 4], k & 15);
           A[m][k] = sv[e];
         }
         if (m != 0 || q != 3 || lane != 0) evidence[slot_quad(m, q) * 64 + lane] = sv;
