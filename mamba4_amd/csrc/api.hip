@@ -87,11 +87,14 @@ __global__ void order_bwd_walk_kernel(OrderDims, const float*, const float*, con
 __global__ void spd_solve_kernel(const float*, const float*, long, int, float*, float*);
 __global__ void spd_backward_kernel(const float*, const float*, const float*, long, int, float*,
                                     float*);
-template <bool LDS>
 __global__ void spd_wide_kernel(const float*, const float*, int, float*, float*);
-template <bool LDS>
 __global__ void spd_wide_backward_kernel(const float*, const float*, const float*, int, float*,
                                          float*);
+template <int NW>
+__global__ void spd_block_kernel(const float*, const float*, int, float*, float*);
+template <int NW>
+__global__ void spd_block_backward_kernel(const float*, const float*, const float*, int, float*,
+                                          float*);
 __global__ void resize_kernel(ResizeJobs);
 __global__ void diag_eigen_kernel(const float*, const float*, const float*, int, int, int, float*);
 __global__ void diag_summary_kernel(const float*, int, const float*, int, float*);
@@ -151,12 +154,9 @@ constexpr size_t kGradsGateLdsBytes = 8 * m4::TILE * sizeof(float);  // + the S0
 constexpr size_t kStatesLdsBytes = 4 * m4::TILE * sizeof(float);
 // The backward walks add one tile (the evidence state's transpose).
 constexpr size_t kStatesBwdExtra = m4::TILE * sizeof(float);
-// The widest LDS request of the wide SPD solves (an LDS-resident 128-wide
-// system, or the vectors of a 4096-wide one).
-constexpr size_t kWideLdsMax =
-    sizeof(float) * (m4::wide_lds_floats(m4::kWideLdsDim) > m4::wide_lds_floats(m4::kWideMaxDim)
-                         ? m4::wide_lds_floats(m4::kWideLdsDim)
-                         : m4::wide_lds_floats(m4::kWideMaxDim));
+// The widest LDS requests of the blocked SPD solves and of the wider ones.
+constexpr size_t kBlockLdsMax = sizeof(float) * m4::block_lds_floats(m4::kBlockMaxDim);
+constexpr size_t kWideLdsMax = sizeof(float) * 3 * m4::kWideMaxDim;
 
 bool configured = false;
 int g_cus = 256;  // compute units of the device (set by configure())
@@ -228,10 +228,14 @@ int configure() {
              {(const void*)m3::out_kernel<m3::bf16_t, false>, m3::kOutLdsBf16},
              {(const void*)m3::grad_kernel<m3::bf16_t, false>, m3::kGradLds},
              {(const void*)m3::finish_kernel, m3::kFinishLdsMax},
-             {(const void*)m4::spd_wide_kernel<true>, kWideLdsMax},
-             {(const void*)m4::spd_wide_kernel<false>, kWideLdsMax},
-             {(const void*)m4::spd_wide_backward_kernel<true>, kWideLdsMax},
-             {(const void*)m4::spd_wide_backward_kernel<false>, kWideLdsMax}};
+             {(const void*)m4::spd_wide_kernel, kWideLdsMax},
+             {(const void*)m4::spd_wide_backward_kernel, kWideLdsMax},
+             {(const void*)m4::spd_block_kernel<2>, kBlockLdsMax},
+             {(const void*)m4::spd_block_kernel<3>, kBlockLdsMax},
+             {(const void*)m4::spd_block_kernel<4>, kBlockLdsMax},
+             {(const void*)m4::spd_block_backward_kernel<2>, kBlockLdsMax},
+             {(const void*)m4::spd_block_backward_kernel<3>, kBlockLdsMax},
+             {(const void*)m4::spd_block_backward_kernel<4>, kBlockLdsMax}};
   for (auto& k : big) {
     hipError_t e = hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)k.bytes);
@@ -1062,17 +1066,25 @@ int m4mr_spd_solve(const float* precision, const float* rhs, long N, int dim, fl
     return fail(M4MR_EINVAL, "m4mr_spd_solve: a required pointer is NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dim > M4MR_KEY_DIM) {
-    const bool lds = dim <= m4::kWideLdsDim;
-    if (!lds && !factors)
+    if (dim > 128 && !factors)
       return fail(M4MR_EINVAL,
                   "m4mr_spd_solve: above width 128 the factors buffer is required (the "
                   "factorization runs in it)");
     if (int rc = configure()) return rc;
-    const size_t bytes = sizeof(float) * m4::wide_lds_floats(dim);
+    if (dim <= m4::kBlockMaxDim) {
+      const int waves = m4::block_waves(dim);
+      const auto kernel = waves == 2   ? m4::spd_block_kernel<2>
+                          : waves == 3 ? m4::spd_block_kernel<3>
+                                       : m4::spd_block_kernel<4>;
+      return launch("spd_wide", st, [&] {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)N), dim3(64 * waves),
+                           sizeof(float) * m4::block_lds_floats(dim), st, precision, rhs, dim,
+                           solution, factors);
+      });
+    }
     return launch("spd_wide", st, [&] {
-      hipLaunchKernelGGL(lds ? m4::spd_wide_kernel<true> : m4::spd_wide_kernel<false>,
-                         dim3((unsigned)N), dim3(m4::kWideThreads), bytes, st, precision, rhs,
-                         dim, solution, factors);
+      hipLaunchKernelGGL(m4::spd_wide_kernel, dim3((unsigned)N), dim3(m4::kWideThreads),
+                         sizeof(float) * 3 * dim, st, precision, rhs, dim, solution, factors);
     });
   }
   if ((factors && misaligned(factors)) || (dim == M4MR_KEY_DIM && misaligned(precision)))
@@ -1096,14 +1108,22 @@ int m4mr_spd_solve_backward(const float* factors, const float* solution,
     return fail(M4MR_EINVAL, "m4mr_spd_solve_backward: a required pointer is NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dim > M4MR_KEY_DIM) {
-    const bool lds = dim <= m4::kWideLdsDim;
     if (int rc = configure()) return rc;
-    const size_t bytes = sizeof(float) * m4::wide_lds_floats(dim);
+    if (dim <= m4::kBlockMaxDim) {
+      const int waves = m4::block_waves(dim);
+      const auto kernel = waves == 2   ? m4::spd_block_backward_kernel<2>
+                          : waves == 3 ? m4::spd_block_backward_kernel<3>
+                                       : m4::spd_block_backward_kernel<4>;
+      return launch("spd_wide_backward", st, [&] {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)N), dim3(64 * waves),
+                           sizeof(float) * m4::block_lds_floats(dim), st, factors, solution,
+                           d_solution, dim, d_precision, d_rhs);
+      });
+    }
     return launch("spd_wide_backward", st, [&] {
-      hipLaunchKernelGGL(lds ? m4::spd_wide_backward_kernel<true>
-                             : m4::spd_wide_backward_kernel<false>,
-                         dim3((unsigned)N), dim3(m4::kWideThreads), bytes, st, factors, solution,
-                         d_solution, dim, d_precision, d_rhs);
+      hipLaunchKernelGGL(m4::spd_wide_backward_kernel, dim3((unsigned)N), dim3(m4::kWideThreads),
+                         sizeof(float) * 3 * dim, st, factors, solution, d_solution, dim,
+                         d_precision, d_rhs);
     });
   }
   if (misaligned(factors) || (dim == M4MR_KEY_DIM && misaligned(d_precision)))

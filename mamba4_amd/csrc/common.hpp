@@ -560,15 +560,22 @@ __device__ __forceinline__ void zero2(f4 acc[2]) {
 // Kernels built on these tiles run 256 threads (4 waves).
 constexpr int BLOCK = 256;
 
-// SPD solves wider than 64 (spd_wide.hip): one 256-thread block per
-// system, factored in LDS up to kWideLdsDim, in the factor buffer above.
+// SPD solves wider than 64 (spd_wide.hip): one block per system, blocked in
+// LDS up to kBlockMaxDim, a column at a time in the factor buffer above (256
+// threads; three vectors of LDS).
 constexpr int kWideThreads = 256;
-constexpr int kWideLdsDim = 128;
 constexpr int kWideMaxDim = 4096;
-// LDS floats a block takes: the column, two vectors and, for LDS systems,
-// the matrix (row stride dim + 1).
-__host__ __device__ constexpr long wide_lds_floats(int dim) {
-  return 3L * dim + (dim <= kWideLdsDim ? (long)dim * (dim + 1) : 0L);
+constexpr int kBlockMaxDim = 208;
+constexpr int kBlockTile = 16 * 17;  // floats of a 16x16 tile in LDS
+// Waves of a block: 48 rows each below a 16-column panel.
+__host__ __device__ constexpr int block_waves(int dim) {
+  return dim <= 112 ? 2 : dim <= 160 ? 3 : 4;
+}
+// LDS floats: the lower triangle's tiles, a vector and the panel's rows (20
+// floats each; a second vector in the backward).
+__host__ __device__ constexpr long block_lds_floats(int dim) {
+  const int nb = (dim + 15) / 16;
+  return (long)nb * (nb + 1) / 2 * kBlockTile + 16L * nb * 21;
 }
 
 // One 64x64 tile staged through registers: thread i fetches the float4 at

@@ -90,7 +90,7 @@ def test_batch_dims_and_every_backend_agree(gpu_lib):
 
 @pytest.mark.parametrize("count,dim", [(3, 65), (5, 100), (4, 128), (3, 129), (2, 200), (1, 384)])
 def test_wide_systems_match_oracle(gpu_lib, count, dim):
-    """Widths above 64 (one block per system; LDS-resident up to 128, in the
+    """Widths above 64 (one block per system; LDS-resident up to 208, in the
     factor buffer above), the reference's any-width solve
     (lm/kernels/mamba4.py:164-217)."""
     announce(f"spd_solve wide N={count} d={dim} (upper triangle holds garbage)")
@@ -103,6 +103,35 @@ def test_wide_systems_match_oracle(gpu_lib, count, dim):
     assert normwise(d_rhs, want_rhs) <= 1e-3
     assert normwise(d_a, want_a) <= 1e-3
     np.testing.assert_array_equal(d_a, np.swapaxes(d_a, -1, -2))
+
+
+@pytest.mark.parametrize("dim", [79, 80, 81, 96, 112, 113, 144, 160, 161, 192, 208, 209])
+def test_wide_solves_at_the_edges_of_tiles_and_waves(gpu_lib, dim):
+    """Widths around a 16-column tile, around 112 and 160 (one more wave per
+    block) and around 208 (the last width factored in LDS), with a right-hand
+    side whose solution is known and an upper triangle of NaN."""
+    from mamba4_amd import spd_solve
+
+    announce(f"spd_solve edges d={dim}")
+    rng = np.random.default_rng(dim)
+    half = rng.normal(size=(3, dim, 2 * dim))
+    a = half @ np.swapaxes(half, -1, -2) / (2 * dim) + 0.25 * np.eye(dim)
+    a = a.astype(np.float32).astype(np.float64)
+    lower = np.tril(a)
+    a = lower + np.swapaxes(np.tril(lower, -1), -1, -2)
+    stored = np.where(np.tril(np.ones((dim, dim), bool)), lower, np.nan)
+    rhs, g = rng.normal(size=(2, 3, dim)).astype(np.float32)
+    at, bt = (torch.tensor(x, dtype=torch.float32, device="cuda:0").requires_grad_(True)
+              for x in (stored, rhs))
+    y = spd_solve(at, bt)
+    d_a, d_rhs = torch.autograd.grad(y, (at, bt), torch.tensor(g, device="cuda:0"))
+    torch.cuda.synchronize()
+    # Condition about 20: float32 sums of up to 208 terms.
+    want = np.linalg.solve(a, rhs[..., None].astype(np.float64))[..., 0]
+    z = np.linalg.solve(a, g[..., None].astype(np.float64))[..., 0]
+    outer = z[..., :, None] * want[..., None, :]
+    assert normwise(host(y), want) <= 1e-5 and normwise(host(d_rhs), z) <= 1e-5
+    assert normwise(host(d_a), -0.5 * (outer + np.swapaxes(outer, -1, -2))) <= 1e-5
 
 
 @pytest.mark.parametrize("dim", [65, 160])
