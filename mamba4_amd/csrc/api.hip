@@ -319,13 +319,15 @@ int turn_polls() {
 // as measured for spans of 2 to 32 tokens from 2 to 12,288 sub-chunks: a round
 // takes 6, and with one wave per SIMD (up to two pairs per compute unit) 11.4 a
 // pass and 0.28 a caught-up token, with two waves 18 and 0.8.
-int factor_spans(long subseqs, int sub) {
+// Empty and short sub-chunks at a sequence's end count as their tokens.
+int factor_spans(long tokens, int sub) {
   int best = 1;
   double best_us = 0.0;
   for (int nspan = 1; nspan <= 16 && nspan <= sub; nspan *= 2) {
     const int span = (sub + nspan - 1) / nspan, passes = (span + 1) / 2;
     const double catchup = (double)(nspan - 1) * span;  // of the last span; half on average
-    const long pairs = (subseqs * nspan + 3) / 4, full = 4L * g_cus, rest = pairs % full;
+    const long work = (tokens * nspan + sub - 1) / sub;  // sub-chunks' spans
+    const long pairs = (work + 3) / 4, full = 4L * g_cus, rest = pairs % full;
     double us = (double)(pairs / full) * (6.0 + 18.0 * passes + 0.4 * catchup);
     if (rest > full / 2)
       us += (0.9 + 0.1 * (2.0 * rest / full - 1.0)) * (6.0 + 18.0 * passes + 0.8 * catchup);
@@ -479,7 +481,7 @@ int forward_impl(const char* entry, const In* keys, const In* values, const In* 
   rc = launch("fwd_factor", st, [&] {
     // Four spans per wave pair; four pairs per block when those blocks fill
     // the chip in whole rounds (one resident per CU), else two.
-    const int nspan = factor_spans(subseqs, d.sub);
+    const int nspan = factor_spans((long)B * H * T, d.sub);
     const unsigned spans = subseqs * nspan;
     const unsigned blocks4 = (spans + 15) / 16;
     const int pairs = blocks4 % (unsigned)g_cus == 0 ? 4 : 2;
@@ -1487,7 +1489,7 @@ int m4mr_resize(const m4mr_resize_array* arrays, int count, void* stream) {
   if (!arrays || count < 1 || count > m4::kResizeJobs)
     return fail(M4MR_EINVAL, "m4mr_resize: need 1.." + std::to_string(m4::kResizeJobs) + " arrays");
   m4::ResizeJobs jobs{};
-  long elements = 0;
+  long total = 0;
   for (int i = 0; i < count; ++i) {
     const m4mr_resize_array& a = arrays[i];
     if (a.outer < 0 || a.src_rows < 0 || a.src_cols < 0 || a.dst_rows < 0 || a.dst_cols < 0 ||
@@ -1500,16 +1502,20 @@ int m4mr_resize(const m4mr_resize_array* arrays, int count, void* stream) {
     if (n == 0) continue;
     if (!a.dst || (!a.src && a.src_rows > 0 && a.src_cols > 0))
       return fail(M4MR_EINVAL, "m4mr_resize: a required pointer is NULL");
-    jobs.job[jobs.count++] = m4::ResizeJob{a.src,      a.dst,      n,       a.src_rows, a.src_cols,
-                                           a.dst_rows, a.dst_cols, a.bytes, a.fill};
-    elements += n;
+    const long quads = a.outer * a.dst_rows * ((a.dst_cols + 3L) / 4);
+    const int aligned =
+        a.dst_cols % 4 == 0 && (reinterpret_cast<uintptr_t>(a.dst) & (4 * a.bytes - 1)) == 0;
+    jobs.job[jobs.count++] =
+        m4::ResizeJob{a.src,      a.dst,      quads,   a.src_rows, a.src_cols,
+                      a.dst_rows, a.dst_cols, a.bytes, aligned,    a.fill};
+    total += quads;
   }
-  if (elements == 0) return M4MR_OK;
-  if ((elements + 255) / 256 > INT_MAX) return fail(M4MR_EINVAL, "m4mr_resize: arrays too large");
+  if (total == 0) return M4MR_OK;
+  if ((total + 255) / 256 > INT_MAX) return fail(M4MR_EINVAL, "m4mr_resize: arrays too large");
   hipStream_t st = static_cast<hipStream_t>(stream);
   return launch("resize", st, [&] {
-    hipLaunchKernelGGL(m4::resize_kernel, dim3((unsigned)((elements + 255) / 256)), dim3(256), 0,
-                       st, jobs);
+    hipLaunchKernelGGL(m4::resize_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
+                       jobs);
   });
 }
 

@@ -832,12 +832,13 @@ struct StateArgs {
 // tokens, NC of them.
 // One array of resize_kernel: `outer` matrices src_rows x src_cols to
 // dst_rows x dst_cols of `bytes`-byte elements (4 or 2), cut off or padded with
-// `fill`; `elements` of the destination.
+// `fill`; `quads` of four columns in the destination, `aligned` where each
+// can be stored at once.
 struct ResizeJob {
   const void* src;
   void* dst;
-  long elements;
-  int src_rows, src_cols, dst_rows, dst_cols, bytes;
+  long quads;
+  int src_rows, src_cols, dst_rows, dst_cols, bytes, aligned;
   unsigned fill;
 };
 constexpr int kResizeJobs = 8;

@@ -207,12 +207,19 @@ __device__ __forceinline__ void stage_evidence(f4* evidence, const float* start_
     for (int j = 0; j < CATCHUP_GROUP; ++j) cur[j] = next[j];
   }
   const float scale = -c * expf(after);  // -c without a token before the span
+  f4 start[4][5];
 #pragma unroll
   for (int mu = 0; mu < 4; ++mu) {
     const float* s0 = start_s + (long)__builtin_amdgcn_readlane(slot, 16 * mu) * 4096;
+    for_staged_blocks<W>([&](int i, int I, int K) {
+      start[mu][i] = *reinterpret_cast<const f4*>(s0 + (16 * I + a) * 64 + 16 * K + 4 * g);
+    });
+  }
+#pragma unroll
+  for (int mu = 0; mu < 4; ++mu) {
     const float w = row_value(scale, mu);
     for_staged_blocks<W>([&](int i, int I, int K) {
-      const f4 v = *reinterpret_cast<const f4*>(s0 + (16 * I + a) * 64 + 16 * K + 4 * g);
+      const f4 v = start[mu][i];
       evidence[slot_quad(I, 4 * K + g) * 64 + 16 * mu + a] =
           f4{w * v[0] + E[i][4 * mu], w * v[1] + E[i][4 * mu + 1], w * v[2] + E[i][4 * mu + 2],
              w * v[3] + E[i][4 * mu + 3]};
