@@ -277,16 +277,23 @@ int launch(const char* name, hipStream_t stream, F&& body) {
 }
 
 // The chunk-boundary states run as one fused walk per (b, h) state sequence
-// when there are enough sequences to give every compute unit one; fewer
-// sequences take the chunk-parallel statistics plus a separate carry.  The
-// environment variable M4MR_STATE_WALK = "fused" or "split" overrides the
-// choice (both give the same states up to summation order).
+// when there are enough sequences to give every compute unit one, or few
+// enough chunks to walk; else as chunk-parallel statistics plus a separate
+// carry.  A walk takes about 2 us and 2.2 a chunk while every block has a
+// compute unit, the pair 8 us (two launches) and 0.0156 a walk and chunk (its
+// states written, read and written).  Forward + backward, walk against pair:
+// B4 T1024 H8 P64 (64 walks) 37 + 36 / 25 + 23 us, B8 T1024 H8 P128 (192) 42 + 41
+// / 52 + 50, B6 T4096 H8 P64 (96) 139 + 130 / 100 + 93, B16 T1024 H8 P64 (256)
+// 46 + 44 / 71 + 69.  The environment variable M4MR_STATE_WALK = "fused" or
+// "split" overrides the choice (both give the same states up to summation
+// order).
 bool fused_states(int B, int H, const Dims& d) {
   if (const char* mode = std::getenv("M4MR_STATE_WALK")) {
     if (std::strcmp(mode, "fused") == 0) return true;
     if (std::strcmp(mode, "split") == 0) return false;
   }
-  return (long)B * H * (1 + d.NV) >= g_cus;
+  const double walks = (double)B * H * (1 + d.NV);
+  return walks >= g_cus || 2.0 + 2.2 * d.NC <= 8.0 + 0.0156 * walks * d.NC;
 }
 
 // The fused walks with one LDS step buffer (three blocks per CU) when their
@@ -466,7 +473,8 @@ int forward_impl(const char* entry, const In* keys, const In* values, const In* 
     });
   } else {
     rc = launch("fwd_stats", st, [&] {
-      hipLaunchKernelGGL(m4::fwd_stats_kernel<In>, dim3(seqs), dim3(256), kStatsLdsBytes, st, d,
+      hipLaunchKernelGGL(m4::fwd_stats_kernel<In>, dim3(seqs), dim3(256),
+                         (1 + d.NV) * m4::TILE * sizeof(float), st, d,
                          keys, values, beta, log_decay, start_evidence, start_cross);
     });
     if (rc) return rc;

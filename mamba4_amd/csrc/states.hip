@@ -28,6 +28,28 @@ namespace m4 {
 
 __device__ __forceinline__ float* mat(float* base, long index) { return base + index * 4096; }
 
+// acc += (A diag(wt))^T B over k in [k0, k0 + 16) for rows 16 w.. of the result
+// and its columns 4r + jb: A(i, k) = A[k][16w + i] wt[k], B(k, c) = B[k][c]
+// (tile_mma's QUAD convention, the weights applied as the operand leaves LDS).
+__device__ __forceinline__ void weighted_strip(f4 acc[4], const float* A, const float* B,
+                                               const float* wt, int k0, int w) {
+  const int l = lane_id(), r = l & 15, kk = k0 + 4 * (l >> 4);
+  const f4 t = *reinterpret_cast<const f4*>(wt + kk);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float a = A[(kk + e) * LDT + 16 * w + r] * t[e];
+    const f4 bv = *reinterpret_cast<const f4*>(B + (kk + e) * LDT + 4 * r);
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb)
+      acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bv[jb], acc[jb], 0, 0, 0);
+  }
+}
+
+// One block per chunk of a sequence.  Every tile is loaded at once and staged
+// behind one barrier, and each product weighs its tokens as it reads them: a
+// weighted copy of the keys and values in LDS (an exponential per element,
+// two barriers per product) had a B1 T2000 H12 P128 launch at 23.8 us, now 13.9 (and bwd_local
+// at B8 T1737 H8 P64 44.9, now 35.1).
 template <typename In>
 __global__ __launch_bounds__(256) void fwd_stats_kernel(
     Dims d, const In* __restrict__ keys, const In* __restrict__ values,
@@ -35,58 +57,47 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(
     float* __restrict__ start_s, float* __restrict__ start_c) {
   extern __shared__ float smem[];
   float* K = smem;
-  float* V = K + TILE;
-  float* W = V + TILE;
+  float* V = K + TILE;  // NV tiles
   __shared__ ChunkScalars cs;
+  __shared__ alignas(16) float wt[3][MAXC];  // the sub-chunks' weights, then the chunk's
   const long seq = blockIdx.x;
   const int n = (int)(seq % d.NC), bh = (int)(seq / d.NC), b = bh / d.H, h = bh % d.H;
   const int len = chunk_len(d, n), w = threadIdx.x >> 6, c4 = 4 * (lane_id() & 15);
-  const int kt = k_terms(len);
-  auto rows = [&](const In* base, int width, int offset) {
-    return [=](int s) { return base + token_head(d, b, n * d.chunk + s, h) * width + offset; };
-  };
-  TileRegs rk, rv;
-  rk.fetch_rows(len, rows(keys, 64, 0));
-  rv.fetch_rows(len, rows(values, d.P, 0));
-  rk.store(K);
-  rv.store(V);
+  const long row = token_head(d, b, n * d.chunk, h);
+  RowTile<In> rk, rv0, rv1;
+  rk.fetch_tokens(len, keys + row * 64, (unsigned)(d.H * 64));
+  rv0.fetch_tokens(len, values + row * d.P, (unsigned)(d.H * d.P));
+  rv1.fetch_tokens(d.NV > 1 ? len : 0, values + row * d.P + (d.NV > 1 ? 64 : 0),
+                   (unsigned)(d.H * d.P));
   load_chunk_scalars(cs, d, beta, log_decay, b, h, n);
-  __syncthreads();
-
-  for (int u = 0; u < d.rsub; ++u) {
-    const int first = sub_first(d, u), cnt = sub_len(d, n, u);
-    const float p_end = cnt > 0 ? cs.prefix[first + cnt - 1] : 0.f;
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-      const int s = e >> 6, c = e & 63;
-      const bool in = s >= first && s < first + cnt;
-      W[s * LDT + c] = in ? cs.beta[s] * expf(p_end - cs.prefix[s]) * K[s * LDT + c] : 0.f;
+  if (threadIdx.x < 64) {
+    const int s = threadIdx.x;
+    const float p = cs.prefix[s], bt = cs.beta[s];  // this wave's own writes
+    for (int u = 0; u < d.rsub; ++u) {
+      const int first = sub_first(d, u), cnt = sub_len(d, n, u);
+      const float p_end = cnt > 0 ? cs.prefix[first + cnt - 1] : 0.f;
+      wt[u][s] = s >= first && s < first + cnt ? bt * expf(p_end - p) : 0.f;
     }
-    __syncthreads();
+    wt[2][s] = s < len ? cs.tail[s] : 0.f;
+  }
+  rk.store(K);
+  rv0.store(V);
+  if (d.NV > 1) rv1.store(V + TILE);
+  __syncthreads();
+  for (int u = 0; u < d.rsub; ++u) {
+    const int first = sub_first(d, u), end = first + sub_len(d, n, u);
     f4 acc[4];
     zero4(acc);
-    tile_mma<true, false>(acc, W, K, kt, w);  // sum_s tail_s k_s k_s^T
+    for (int k0 = first & ~15; k0 < end; k0 += 16) weighted_strip(acc, K, K, wt[u], k0, w);
     float* out = mat(start_s, (long)bh * d.NS + (long)n * d.rsub + u);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       *reinterpret_cast<f4*>(out + acc_row(w, q) * 64 + c4) = quad_row(acc, q);
-    __syncthreads();
   }
   for (int v = 0; v < d.NV; ++v) {
-    if (v > 0) {
-      // Value tile v replaces tile v - 1 once every wave has read it.
-      rv.fetch_rows(len, rows(values, d.P, 64 * v));
-      __syncthreads();
-      rv.store(V);
-      __syncthreads();
-    }
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-      const int s = e >> 6, c = e & 63;
-      W[s * LDT + c] = s < len ? cs.tail[s] * V[s * LDT + c] : 0.f;
-    }
-    __syncthreads();
     f4 acc[4];
     zero4(acc);
-    tile_mma<true, false>(acc, W, K, kt, w);  // sum_s tail_s v_s k_s^T
+    for (int k0 = 0; k0 < len; k0 += 16) weighted_strip(acc, V + v * TILE, K, wt[2], k0, w);
     float* out = mat(start_c, ((long)bh * d.NC + n) * d.NV + v);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -94,23 +105,33 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(
   }
 }
 
-// exp(sum of log decays) over the tokens of step `i` of the scan: a
-// sub-chunk (evidence) or a chunk (cross statistics).
-__device__ __forceinline__ float step_decay(const Dims& d, const float* log_decay, int b, int h,
-                                            int i, bool sub) {
-  int first, cnt;
+// exp(sum of log decays) over the tokens of the scan's steps first .. first +
+// count - 1 (count <= 64): sub-chunks (evidence) or chunks (cross statistics).
+// A 256-thread block, four threads a step, sixteen tokens each, every load at
+// once (a thread per step walked up to 64 of them, eight at a time).
+__device__ __forceinline__ void step_decays(float* decay, const Dims& d, const float* log_decay,
+                                            int b, int h, int first, int count, bool sub) {
+  const int k = threadIdx.x >> 2, part = threadIdx.x & 3, i = first + min(k, count - 1);
+  int t0, cnt;
   if (sub) {
     const int n = i / d.rsub, u = i % d.rsub;
-    first = n * d.chunk + sub_first(d, u);
+    t0 = n * d.chunk + sub_first(d, u);
     cnt = sub_len(d, n, u);
   } else {
-    first = i * d.chunk;
+    t0 = i * d.chunk;
     cnt = chunk_len(d, i);
   }
-  float g = 0.f;
-#pragma unroll 8
-  for (int t = 0; t < cnt; ++t) g += log_decay[token_head(d, b, first + t, h)];
-  return expf(g);
+  float x[16], g = 0.f;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int t = 16 * part + j;
+    x[j] = log_decay[token_head(d, b, min(t0 + (t < cnt ? t : 0), d.T - 1), h)];
+  }
+#pragma unroll
+  for (int j = 0; j < 16; ++j) g += 16 * part + j < cnt ? x[j] : 0.f;
+  g += dpp_read<0xB1>(g);  // quad_perm [1,0,3,2]
+  g += dpp_read<0x4E>(g);  // quad_perm [2,3,0,1]
+  if (part == 0 && k < count) decay[k] = expf(g);
 }
 
 // Steps of a scan whose loads are issued together.
@@ -130,26 +151,33 @@ __global__ __launch_bounds__(256) void fwd_scan_kernel(
   const long size = cross ? 4096L * d.NV : 4096L;  // floats per state
   float* buf = (cross ? start_c : start_s) + (long)bh * steps * size;
   const float* init = cross ? init_c : init_s;
-  __shared__ float decay[256];
+  __shared__ float decay[64];
   f4 running = f4{0.f, 0.f, 0.f, 0.f};
   if (init) running = *reinterpret_cast<const f4*>(init + (long)bh * size + elem);
-  for (int base = 0; base < steps; base += 256) {
-    const int count = min(256, steps - base);
-    __syncthreads();
-    if (threadIdx.x < count)
-      decay[threadIdx.x] = step_decay(d, log_decay, b, h, base + threadIdx.x, !cross);
+  for (int base = 0; base < steps; base += 64) {
+    const int count = min(64, steps - base);
+    f4 stat[SCAN_BATCH];
+    // Steps past the last read it again: no branch around a load.
+    auto load = [&](int i0) {
+#pragma unroll
+      for (int j = 0; j < SCAN_BATCH; ++j)
+        stat[j] = *reinterpret_cast<const f4*>(buf + (long)min(base + i0 + j, steps - 1) * size +
+                                               elem);
+    };
+    load(0);
+    __syncthreads();  // the previous steps' decays are read
+    step_decays(decay, d, log_decay, b, h, base, count, !cross);
     __syncthreads();
     for (int i0 = 0; i0 < count; i0 += SCAN_BATCH) {
-      const int m = min(SCAN_BATCH, count - i0);
-      f4 stat[SCAN_BATCH];
+      f4 cur[SCAN_BATCH];
+#pragma unroll
+      for (int j = 0; j < SCAN_BATCH; ++j) cur[j] = stat[j];
+      if (i0 + SCAN_BATCH < count) load(i0 + SCAN_BATCH);
 #pragma unroll
       for (int j = 0; j < SCAN_BATCH; ++j)
-        if (j < m) stat[j] = *reinterpret_cast<const f4*>(buf + (long)(base + i0 + j) * size + elem);
-#pragma unroll
-      for (int j = 0; j < SCAN_BATCH; ++j)
-        if (j < m) {
+        if (i0 + j < count) {
           *reinterpret_cast<f4*>(buf + (long)(base + i0 + j) * size + elem) = running;
-          running = decay[i0 + j] * running + stat[j];
+          running = decay[i0 + j] * running + cur[j];
         }
     }
   }
@@ -157,46 +185,52 @@ __global__ __launch_bounds__(256) void fwd_scan_kernel(
   *reinterpret_cast<f4*>(fin + (long)bh * size + elem) = running;
 }
 
+// One block per chunk, loads and weights as in fwd_stats_kernel.
 __global__ __launch_bounds__(256) void bwd_local_kernel(
     Dims d, const float* __restrict__ beta, const float* __restrict__ log_decay,
     const float* __restrict__ solved, const float* __restrict__ z,
     const float* __restrict__ d_output, float* __restrict__ end_s, float* __restrict__ end_c) {
   extern __shared__ float smem[];
   float* Y = smem;
-  float* Zw = Y + TILE;
-  float* Dw = Zw + TILE;
-  float* M = Dw + TILE;
+  float* Z = Y + TILE;
+  float* D = Z + TILE;
+  float* M = D + TILE;
   __shared__ ChunkScalars cs;
+  __shared__ alignas(16) float wt[MAXC];
   const long seq = blockIdx.x;
   const int n = (int)(seq % d.NC), bh = (int)(seq / d.NC), b = bh / d.H, h = bh % d.H;
   const int len = chunk_len(d, n), w = threadIdx.x >> 6, c4 = 4 * (lane_id() & 15);
-  const int kt = k_terms(len);
-  auto rows = [&](const float* base, int width, int offset) {
-    return [=](int s) { return base + token_head(d, b, n * d.chunk + s, h) * width + offset; };
-  };
-  TileRegs ry, rz, rd;
-  ry.fetch_rows(len, rows(solved, 64, 0));
-  rz.fetch_rows(len, rows(z, 64, 0));
-  rd.fetch_rows(len, rows(d_output, d.P, 0));
-  ry.store(Y);
-  rz.store(Zw);
-  rd.store(Dw);
+  const long row = token_head(d, b, n * d.chunk, h);
+  RowTile<float> ry, rz, rd0, rd1;
+  ry.fetch_tokens(len, solved + row * 64, (unsigned)(d.H * 64));
+  rz.fetch_tokens(len, z + row * 64, (unsigned)(d.H * 64));
+  rd0.fetch_tokens(len, d_output + row * d.P, (unsigned)(d.H * d.P));
+  rd1.fetch_tokens(d.NV > 1 ? len : 0, d_output + row * d.P + (d.NV > 1 ? 64 : 0),
+                   (unsigned)(d.H * d.P));
   load_chunk_scalars(cs, d, beta, log_decay, b, h, n);
+  if (threadIdx.x < 64)
+    wt[threadIdx.x] = (int)threadIdx.x < len ? expf(cs.prefix[threadIdx.x]) : 0.f;
+  ry.store(Y);
+  rz.store(Z);
+  rd0.store(D);
   __syncthreads();
-  for (int e = threadIdx.x; e < len * 64; e += 256) {
-    const int t = e >> 6, c = e & 63;
-    const float carried = expf(cs.prefix[t]);
-    Zw[t * LDT + c] *= carried;
-    Dw[t * LDT + c] *= carried;
-  }
-  __syncthreads();
-  f4 acc[4];
+  auto store_cross = [&](const f4 (&acc)[4], int v) {
+    float* uc = mat(end_c, ((long)bh * d.NC + n) * d.NV + v);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<f4*>(uc + acc_row(w, q) * 64 + c4) = quad_row(acc, q);
+  };
+  f4 acc[4], cross[4];
   zero4(acc);
-  tile_mma<true, false>(acc, Zw, Y, kt, w);  // M = sum_t e^P z_t y_t^T
+  for (int k0 = 0; k0 < len; k0 += 16) weighted_strip(acc, Z, Y, wt, k0, w);  // sum_t e^P z_t y_t^T
 #pragma unroll
   for (int q = 0; q < 4; ++q)
     *reinterpret_cast<f4*>(M + acc_row(w, q) * LDT + c4) = quad_row(acc, q);
-  __syncthreads();
+  zero4(cross);
+  for (int k0 = 0; k0 < len; k0 += 16) weighted_strip(cross, D, Y, wt, k0, w);  // e^P dout y^T
+  store_cross(cross, 0);
+  __syncthreads();  // M is whole, and Z and D are read
+  if (d.NV > 1) rd1.store(Z);
   float* us = mat(end_s, (long)bh * d.NC + n);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -206,25 +240,11 @@ __global__ __launch_bounds__(256) void bwd_local_kernel(
     for (int jb = 0; jb < 4; ++jb) v[jb] = -(acc[jb][q] + M[(c4 + jb) * LDT + i]);
     *reinterpret_cast<f4*>(us + i * 64 + c4) = v;
   }
-  for (int v = 0; v < d.NV; ++v) {
-    if (v > 0) {
-      // Value tile v of the read cotangent replaces tile v - 1.
-      rd.fetch_rows(len, rows(d_output, d.P, 64 * v));
-      __syncthreads();
-      rd.store(Dw);
-      __syncthreads();
-      for (int e = threadIdx.x; e < len * 64; e += 256) {
-        const int t = e >> 6, c = e & 63;
-        Dw[t * LDT + c] *= expf(cs.prefix[t]);
-      }
-      __syncthreads();
-    }
-    zero4(acc);
-    tile_mma<true, false>(acc, Dw, Y, kt, w);  // V = sum_t e^P dout_t y_t^T
-    float* uc = mat(end_c, ((long)bh * d.NC + n) * d.NV + v);
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      *reinterpret_cast<f4*>(uc + acc_row(w, q) * 64 + c4) = quad_row(acc, q);
+  if (d.NV > 1) {
+    __syncthreads();
+    zero4(cross);
+    for (int k0 = 0; k0 < len; k0 += 16) weighted_strip(cross, Z, Y, wt, k0, w);
+    store_cross(cross, 1);
   }
 }
 
@@ -239,7 +259,7 @@ __global__ __launch_bounds__(256) void bwd_scan_kernel(
   const long size = cross ? 4096L * d.NV : 4096L;  // floats per state
   float* buf = (cross ? end_c : end_s) + (long)bh * d.NC * size;
   const float* fin = cross ? d_final_c : d_final_s;
-  __shared__ float decay[256];
+  __shared__ float decay[64];
   // Evidence: the scan carries G + G^T (it starts from D + D^T and adds the
   // local terms 2U = -(M + M^T), as bwd_local_kernel stores them), so every
   // stored end-state cotangent is symmetric; the initial-state gradient is
@@ -258,23 +278,28 @@ __global__ __launch_bounds__(256) void bwd_scan_kernel(
       running += tr;
     }
   }
-  for (int top = d.NC; top > 0; top -= 256) {
-    const int count = min(256, top);
-    __syncthreads();
-    if (threadIdx.x < count)
-      decay[threadIdx.x] = step_decay(d, log_decay, b, h, top - count + threadIdx.x, false);
+  for (int top = d.NC; top > 0; top -= 64) {
+    const int count = min(64, top), low = top - count;  // chunks low .. top - 1
+    f4 local[SCAN_BATCH];
+    auto load = [&](int i0) {
+#pragma unroll
+      for (int j = 0; j < SCAN_BATCH; ++j)
+        local[j] = *reinterpret_cast<const f4*>(buf + (long)(low + max(i0 - j, 0)) * size + elem);
+    };
+    load(count - 1);
+    __syncthreads();  // the previous steps' decays are read
+    step_decays(decay, d, log_decay, b, h, low, count, false);
     __syncthreads();
     for (int i0 = count - 1; i0 >= 0; i0 -= SCAN_BATCH) {
-      const int m = min(SCAN_BATCH, i0 + 1);
-      f4 local[SCAN_BATCH];
+      f4 cur[SCAN_BATCH];
+#pragma unroll
+      for (int j = 0; j < SCAN_BATCH; ++j) cur[j] = local[j];
+      if (i0 - SCAN_BATCH >= 0) load(i0 - SCAN_BATCH);
 #pragma unroll
       for (int j = 0; j < SCAN_BATCH; ++j)
-        if (j < m) local[j] = *reinterpret_cast<const f4*>(buf + (long)(top - count + i0 - j) * size + elem);
-#pragma unroll
-      for (int j = 0; j < SCAN_BATCH; ++j)
-        if (j < m) {
-          *reinterpret_cast<f4*>(buf + (long)(top - count + i0 - j) * size + elem) = running;
-          running = local[j] + decay[i0 - j] * running;
+        if (i0 - j >= 0) {
+          *reinterpret_cast<f4*>(buf + (long)(low + i0 - j) * size + elem) = running;
+          running = cur[j] + decay[i0 - j] * running;
           total *= decay[i0 - j];
         }
     }
