@@ -436,7 +436,7 @@ def selective_decode(state, key, value, query, beta, log_decay, floor, solver=No
     device = evidence.device
     f32 = dict(dtype=torch.float32, device=device)
     key, value, query = (torch.as_tensor(a).to(**f32).contiguous() for a in (key, value, query))
-    floor = torch.as_tensor(floor, **f32).expand(evidence.shape[1], dim).contiguous()
+    floor = _expanded(floor, (evidence.shape[1], dim), device).contiguous()
     wide = _lib.KEY_DIM
     with torch.cuda.device(device):
         old_s, old_c, key, value, query, floor = _resized(
@@ -447,7 +447,7 @@ def selective_decode(state, key, value, query, beta, log_decay, floor, solver=No
     # The kernel reads the states 16 bytes at a time.
     old_s, old_c = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (old_s, old_c))
     new = SelectiveState(torch.empty(old_s.shape, **f32), torch.empty(old_c.shape, **f32))
-    out = _decode_step(SelectiveState(old_s, old_c), new, key, value, query, beta, log_decay, floor)
+    out = _decode_step(old_s, old_c, new, key, value, query, beta, log_decay, floor)
     if (dim, value_dim) == (wide, width):
         return out
     return SelectiveResult(
@@ -470,30 +470,30 @@ def selective_decode_(state, key, value, query, beta, log_decay, floor, solver=N
         raise ValueError("the in-place decode needs D = 64 and P = 64 or 128 states")
     if evidence.dtype != torch.float32 or not evidence.is_contiguous() or not cross.is_contiguous():
         raise ValueError("the in-place decode needs contiguous float32 states")
-    f32 = dict(dtype=torch.float32, device=evidence.device)
-    key, value, query = (torch.as_tensor(a).to(**f32).contiguous() for a in (key, value, query))
-    floor = torch.as_tensor(floor, **f32).expand(evidence.shape[1], dim).contiguous()
-    return _decode_step(state, state, key, value, query, beta, log_decay, floor)
-
-
-def _decode_step(old, new, key, value, query, beta, log_decay, floor):
-    """m4mr_decode_step_to from the state `old` to `new` (which may be the
-    same) at the library's widths."""
-    lib = _lib.load()
-    batch, heads = old.evidence.shape[:2]
-    width = old.cross.shape[-2]
-    device = old.evidence.device
+    device = evidence.device
     f32 = dict(dtype=torch.float32, device=device)
-    beta = torch.as_tensor(beta, **f32).expand(batch, heads).contiguous()
-    log_decay = torch.as_tensor(log_decay, **f32).expand(batch, heads).contiguous()
-    output = torch.empty((batch, heads, width), **f32)
-    variance = torch.empty((batch, heads), **f32)
+    key, value, query = (torch.as_tensor(a).to(**f32).contiguous() for a in (key, value, query))
+    floor = _expanded(floor, (evidence.shape[1], dim), device).contiguous()
+    return _decode_step(evidence, cross, state, key, value, query, beta, log_decay, floor)
+
+
+def _decode_step(evidence, cross, new, key, value, query, beta, log_decay, floor):
+    """m4mr_decode_step_to from the state (evidence, cross) to the state `new`
+    (which may hold the same tensors) at the library's widths."""
+    batch, heads = evidence.shape[:2]
+    width = cross.shape[-2]
+    device = evidence.device
+    beta = _expanded(beta, (batch, heads), device).contiguous()
+    log_decay = _expanded(log_decay, (batch, heads), device).contiguous()
+    output = torch.empty((batch, heads, width), dtype=torch.float32, device=device)
+    variance = torch.empty((batch, heads), dtype=torch.float32, device=device)
     with torch.cuda.device(device):
         _lib.check(
-            lib.m4mr_decode_step_to(
-                _ptr(old.evidence), _ptr(old.cross), _ptr(key), _ptr(value), _ptr(query),
-                _ptr(beta), _ptr(log_decay), _ptr(floor), batch * heads, heads, width,
-                _ptr(new.evidence), _ptr(new.cross), _ptr(output), _ptr(variance), _stream(),
+            _lib.load().m4mr_decode_step_to(
+                evidence.data_ptr(), cross.data_ptr(), key.data_ptr(), value.data_ptr(),
+                query.data_ptr(), beta.data_ptr(), log_decay.data_ptr(), floor.data_ptr(),
+                batch * heads, heads, width, new.evidence.data_ptr(), new.cross.data_ptr(),
+                output.data_ptr(), variance.data_ptr(), _stream(),
             )
         )
     return SelectiveResult(output, variance, new)
