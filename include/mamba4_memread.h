@@ -172,7 +172,7 @@ typedef struct {
  * beta_raw, dt_raw [B,T,H]; outputs as m4mr_forward (output gated), plus
  * read [B,T,H,P].  With params->key_shift and a non-NULL `shifted`
  * [B,H,D], the raw key of position T-1 (the next call's `previous`) is
- * written there.  Always takes the fused state walk.
+ * written there.
  */
 int m4mr_mixer_forward(const float* key, const float* value, const float* query,
                        const float* beta_raw, const float* dt_raw,
@@ -240,7 +240,6 @@ size_t m4mr_mixer_read_backward_workspace_bytes(int B, int T, int H, int value_d
  * d_skip [H]; d_floor_raw [H,D]; d_previous [B,H,D] (may be NULL; zero
  * without the key shift); d_init_evidence, d_init_cross as m4mr_backward.
  * workspace: m4mr_mixer_read_backward_workspace_bytes, 256-byte aligned.
- * Always takes the fused state walk.
  */
 int m4mr_mixer_read_backward(const float* key, const float* value, const float* query,
                              const float* dt_raw, const m4mr_mixer_params* params,

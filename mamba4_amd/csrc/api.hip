@@ -20,13 +20,14 @@
 #include "scan3.hpp"
 
 namespace m4 {
-template <typename In>
+template <typename In, bool MIX>
 __global__ void fwd_stats_kernel(Dims, const In*, const In*, const float*, const float*, float*,
-                                 float*);
+                                 float*, MixerIn, MixerGates);
 __global__ void fwd_scan_kernel(Dims, const float*, const float*, const float*, float*, float*,
                                 float*, float*);
+template <bool GATE>
 __global__ void bwd_local_kernel(Dims, const float*, const float*, const float*, const float*,
-                                 const float*, float*, float*);
+                                 const float*, float*, float*, const float*, const float*);
 __global__ void bwd_scan_kernel(Dims, const float*, const float*, const float*, float*, float*,
                                 float*, float*);
 template <bool BWD, typename In, bool MIX, int NBUF>
@@ -175,9 +176,11 @@ int configure() {
   struct {
     const void* fn;
     size_t bytes;
-  } big[] = {{(const void*)m4::fwd_stats_kernel<float>, kStatsLdsBytes},
-             {(const void*)m4::fwd_stats_kernel<m4::bf16_t>, kStatsLdsBytes},
-             {(const void*)m4::bwd_local_kernel, kChunkLdsBytes},
+  } big[] = {{(const void*)m4::fwd_stats_kernel<float, false>, kStatsLdsBytes},
+             {(const void*)m4::fwd_stats_kernel<m4::bf16_t, false>, kStatsLdsBytes},
+             {(const void*)m4::fwd_stats_kernel<float, true>, kStatsLdsBytes},
+             {(const void*)m4::bwd_local_kernel<false>, kChunkLdsBytes},
+             {(const void*)m4::bwd_local_kernel<true>, kChunkLdsBytes},
 #define M4_CHUNK_ATTRS(NV)                                                                    \
   {(const void*)m4::fwd_read_kernel<float, false, NV>, kChunkLdsBytes},                       \
       {(const void*)m4::fwd_read_kernel<m4::bf16_t, false, NV>, kChunkLdsBytes},              \
@@ -422,7 +425,7 @@ bool misaligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) !=
 // values and queries (the C entry points below).
 // The forward launch sequence.  MIX: keys and queries come from the mixer's
 // raw projections (`mix`; the plain key and query pointers are unused), the
-// state walk is always the fused one, and the output is gated (`gate`).
+// output is gated (`gate`).
 template <typename In, bool MIX>
 int forward_impl(const char* entry, const In* keys, const In* values, const In* queries,
                  const float* beta, const float* log_decay, const float* floor,
@@ -460,7 +463,7 @@ int forward_impl(const char* entry, const In* keys, const In* values, const In* 
   const unsigned seqs = (unsigned)B * H * d.NC;
   const unsigned subseqs = (unsigned)B * H * d.NS;
   int rc;
-  if (MIX || fused_states(B, H, d)) {
+  if (fused_states(B, H, d)) {
     m4::StateArgs args{keys,            values,      keys,           beta,   log_decay,
                        init_evidence,   init_cross,  start_evidence, start_cross,
                        final_evidence,  final_cross, mix};
@@ -473,9 +476,9 @@ int forward_impl(const char* entry, const In* keys, const In* values, const In* 
     });
   } else {
     rc = launch("fwd_stats", st, [&] {
-      hipLaunchKernelGGL(m4::fwd_stats_kernel<In>, dim3(seqs), dim3(256),
+      hipLaunchKernelGGL((m4::fwd_stats_kernel<In, MIX>), dim3(seqs), dim3(256),
                          (1 + d.NV) * m4::TILE * sizeof(float), st, d,
-                         keys, values, beta, log_decay, start_evidence, start_cross);
+                         keys, values, beta, log_decay, start_evidence, start_cross, mix, gates);
     });
     if (rc) return rc;
     rc = launch("fwd_scan", st, [&] {
@@ -593,9 +596,7 @@ int backward_impl(const char* entry, const In* keys, const In* values, const In*
                        st, factors, ws.z, ws.z, tokens);
   });
   if (rc) return rc;
-  // The gated backward always takes the fused walk, whose cross weights
-  // take the read gate.
-  if (GATE || fused_states(B, H, d)) {
+  if (fused_states(B, H, d)) {
     m4::StateArgs args{ws.z,             d_output,       solved,   beta,   log_decay,
                        d_final_evidence, d_final_cross,  ws.end_s, ws.end_c,
                        d_init_evidence,  d_init_cross};
@@ -614,8 +615,9 @@ int backward_impl(const char* entry, const In* keys, const In* values, const In*
     });
   } else {
     rc = launch("bwd_local", st, [&] {
-      hipLaunchKernelGGL(m4::bwd_local_kernel, dim3(seqs), dim3(256), kChunkLdsBytes, st, d,
-                         beta, log_decay, solved, ws.z, d_output, ws.end_s, ws.end_c);
+      hipLaunchKernelGGL(m4::bwd_local_kernel<GATE>, dim3(seqs), dim3(256), kChunkLdsBytes, st, d,
+                         beta, log_decay, solved, ws.z, d_output, ws.end_s, ws.end_c,
+                         mg.variance, mg.scale);
     });
     if (rc) return rc;
     rc = launch("bwd_scan", st, [&] {

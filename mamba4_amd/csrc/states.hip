@@ -50,11 +50,15 @@ __device__ __forceinline__ void weighted_strip(f4 acc[4], const float* A, const 
 // weighted copy of the keys and values in LDS (an exponential per element,
 // two barriers per product) had a B1 T2000 H12 P128 launch at 23.8 us, now 13.9 (and bwd_local
 // at B8 T1737 H8 P64 44.9, now 35.1).
-template <typename In>
+//
+// MIX: the keys come from the mixer's raw projections, shifted and normalised
+// as they are staged, and the gates from theirs (`gates`), written out for the
+// later kernels (as states_kernel's evidence walks do).
+template <typename In, bool MIX>
 __global__ __launch_bounds__(256) void fwd_stats_kernel(
     Dims d, const In* __restrict__ keys, const In* __restrict__ values,
     const float* __restrict__ beta, const float* __restrict__ log_decay,
-    float* __restrict__ start_s, float* __restrict__ start_c) {
+    float* __restrict__ start_s, float* __restrict__ start_c, MixerIn mix, MixerGates gates) {
   extern __shared__ float smem[];
   float* K = smem;
   float* V = K + TILE;  // NV tiles
@@ -65,11 +69,35 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(
   const int len = chunk_len(d, n), w = threadIdx.x >> 6, c4 = 4 * (lane_id() & 15);
   const long row = token_head(d, b, n * d.chunk, h);
   RowTile<In> rk, rv0, rv1;
-  rk.fetch_tokens(len, keys + row * 64, (unsigned)(d.H * 64));
+  if constexpr (MIX)
+    rk.fetch_mix_keys(len, mix, d, b, h, n * d.chunk);
+  else
+    rk.fetch_tokens(len, keys + row * 64, (unsigned)(d.H * 64));
   rv0.fetch_tokens(len, values + row * d.P, (unsigned)(d.H * d.P));
   rv1.fetch_tokens(d.NV > 1 ? len : 0, values + row * d.P + (d.NV > 1 ? 64 : 0),
                    (unsigned)(d.H * d.P));
-  load_chunk_scalars(cs, d, beta, log_decay, b, h, n);
+  if constexpr (MIX) {
+    if (threadIdx.x < 64) {
+      const int s = threadIdx.x;
+      const long th = row + (long)(s < len ? s : 0) * d.H;
+      const float dt = gates.dt_raw[th], bt = gates.beta_raw[th];
+      const float g = s < len ? mix_log_decay(gates, dt, h) : 0.f;
+      const float be = s < len ? mix_beta(gates, bt, h) : 0.f;
+      if (s < len) {
+        gates.log_decay[th] = g;
+        gates.beta[th] = be;
+      }
+      finish_chunk_scalars(cs, g, be);
+      if (n == 0 && b == 0)
+        gates.floor[h * 64 + s] = gates.floor_min + mix_softplus(gates.floor_raw[h * 64 + s]);
+    }
+    if (n == 0 && gates.shifted && threadIdx.x < 16)
+      *reinterpret_cast<f4*>(gates.shifted + (long)bh * 64 + 4 * threadIdx.x) =
+          *reinterpret_cast<const f4*>(mix.key + token_head(d, b, d.T - 1, h) * 64 +
+                                       4 * threadIdx.x);
+  } else {
+    load_chunk_scalars(cs, d, beta, log_decay, b, h, n);
+  }
   if (threadIdx.x < 64) {
     const int s = threadIdx.x;
     const float p = cs.prefix[s], bt = cs.beta[s];  // this wave's own writes
@@ -80,7 +108,10 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(
     }
     wt[2][s] = s < len ? cs.tail[s] : 0.f;
   }
-  rk.store(K);
+  if constexpr (MIX)
+    rk.store_unit(K, mix.key_shift && !mix.previous && n == 0);
+  else
+    rk.store(K);
   rv0.store(V);
   if (d.NV > 1) rv1.store(V + TILE);
   __syncthreads();
@@ -185,18 +216,21 @@ __global__ __launch_bounds__(256) void fwd_scan_kernel(
   *reinterpret_cast<f4*>(fin + (long)bh * size + elem) = running;
 }
 
-// One block per chunk, loads and weights as in fwd_stats_kernel.
+// One block per chunk, loads and weights as in fwd_stats_kernel.  GATE: d_output
+// is the gated output's cotangent, each token's weighed by its read gate.
+template <bool GATE>
 __global__ __launch_bounds__(256) void bwd_local_kernel(
     Dims d, const float* __restrict__ beta, const float* __restrict__ log_decay,
     const float* __restrict__ solved, const float* __restrict__ z,
-    const float* __restrict__ d_output, float* __restrict__ end_s, float* __restrict__ end_c) {
+    const float* __restrict__ d_output, float* __restrict__ end_s, float* __restrict__ end_c,
+    const float* __restrict__ variance, const float* __restrict__ confidence_scale) {
   extern __shared__ float smem[];
   float* Y = smem;
   float* Z = Y + TILE;
   float* D = Z + TILE;
   float* M = D + TILE;
   __shared__ ChunkScalars cs;
-  __shared__ alignas(16) float wt[MAXC];
+  __shared__ alignas(16) float wt[MAXC], wt_cross[MAXC];
   const long seq = blockIdx.x;
   const int n = (int)(seq % d.NC), bh = (int)(seq / d.NC), b = bh / d.H, h = bh % d.H;
   const int len = chunk_len(d, n), w = threadIdx.x >> 6, c4 = 4 * (lane_id() & 15);
@@ -208,8 +242,14 @@ __global__ __launch_bounds__(256) void bwd_local_kernel(
   rd1.fetch_tokens(d.NV > 1 ? len : 0, d_output + row * d.P + (d.NV > 1 ? 64 : 0),
                    (unsigned)(d.H * d.P));
   load_chunk_scalars(cs, d, beta, log_decay, b, h, n);
-  if (threadIdx.x < 64)
-    wt[threadIdx.x] = (int)threadIdx.x < len ? expf(cs.prefix[threadIdx.x]) : 0.f;
+  if (threadIdx.x < 64) {
+    const int s = threadIdx.x;
+    const float e = s < len ? expf(cs.prefix[s]) : 0.f;
+    wt[s] = e;
+    wt_cross[s] = e;
+    if (GATE && s < len)
+      wt_cross[s] = read_gate(confidence_scale[h], variance[row + (long)s * d.H]) * e;
+  }
   ry.store(Y);
   rz.store(Z);
   rd0.store(D);
@@ -227,7 +267,7 @@ __global__ __launch_bounds__(256) void bwd_local_kernel(
   for (int q = 0; q < 4; ++q)
     *reinterpret_cast<f4*>(M + acc_row(w, q) * LDT + c4) = quad_row(acc, q);
   zero4(cross);
-  for (int k0 = 0; k0 < len; k0 += 16) weighted_strip(cross, D, Y, wt, k0, w);  // e^P dout y^T
+  for (int k0 = 0; k0 < len; k0 += 16) weighted_strip(cross, D, Y, wt_cross, k0, w);  // e^P dout y^T
   store_cross(cross, 0);
   __syncthreads();  // M is whole, and Z and D are read
   if (d.NV > 1) rd1.store(Z);
@@ -243,7 +283,7 @@ __global__ __launch_bounds__(256) void bwd_local_kernel(
   if (d.NV > 1) {
     __syncthreads();
     zero4(cross);
-    for (int k0 = 0; k0 < len; k0 += 16) weighted_strip(cross, Z, Y, wt, k0, w);
+    for (int k0 = 0; k0 < len; k0 += 16) weighted_strip(cross, Z, Y, wt_cross, k0, w);
     store_cross(cross, 1);
   }
 }
@@ -692,9 +732,18 @@ M4_STATES(true, float, false)
 M4_STATES(false, float, true)
 M4_STATES(true, float, true)
 #undef M4_STATES
-template __global__ void fwd_stats_kernel<float>(Dims, const float*, const float*, const float*,
-                                                 const float*, float*, float*);
-template __global__ void fwd_stats_kernel<bf16_t>(Dims, const bf16_t*, const bf16_t*,
-                                                  const float*, const float*, float*, float*);
+#define M4_STATS_KERNEL(In, MIX)                                                              \
+  template __global__ void fwd_stats_kernel<In, MIX>(Dims, const In*, const In*, const float*, \
+                                                     const float*, float*, float*, MixerIn,    \
+                                                     MixerGates);
+M4_STATS_KERNEL(float, false)
+M4_STATS_KERNEL(bf16_t, false)
+M4_STATS_KERNEL(float, true)
+template __global__ void bwd_local_kernel<false>(Dims, const float*, const float*, const float*,
+                                                 const float*, const float*, float*, float*,
+                                                 const float*, const float*);
+template __global__ void bwd_local_kernel<true>(Dims, const float*, const float*, const float*,
+                                                const float*, const float*, float*, float*,
+                                                const float*, const float*);
 
 }  // namespace m4
