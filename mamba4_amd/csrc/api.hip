@@ -322,13 +322,14 @@ int turn_polls() {
 // kernel (the spans after the first bring the start evidence up to their own
 // first token, stage_evidence).  A pair walks its span two tokens a pass, a
 // chain that few sequences leave most of the chip waiting for (B1 T512 H8:
-// 186 us in one span, 29 in sixteen), while a full chip only pays the extra
-// updates (B16 T1024 H8: 304 us in one, 311 in two).  A finer split is taken
+// 188 us in one span, 32 in sixteen), while a full chip only pays the extra
+// updates (B16 T1024 H8: 308 us in one, 324 in two).  A finer split is taken
 // where it is estimated at least 5% faster (the estimate's own error: B16
-// T1024 H12 is a tie).  The estimate adds up rounds of pairs, in microseconds
-// as measured for spans of 2 to 32 tokens from 2 to 12,288 sub-chunks: a round
-// takes 6, and with one wave per SIMD (up to two pairs per compute unit) 11.4 a
-// pass and 0.28 a caught-up token, with two waves 18 and 0.8.
+// T1024 H12 is a tie).  The estimate adds up
+// rounds of pairs, in microseconds as measured for spans of 2 to 32 tokens
+// from 2 to 12,288 sub-chunks: a round takes 6, and with one wave per SIMD (up
+// to two pairs per compute unit) 11.4 a pass and 0.42 a caught-up token, with
+// two waves 18 and 1.
 // Empty and short sub-chunks at a sequence's end count as their tokens.
 int factor_spans(long tokens, int sub) {
   int best = 1;
@@ -338,11 +339,11 @@ int factor_spans(long tokens, int sub) {
     const double catchup = (double)(nspan - 1) * span;  // of the last span; half on average
     const long work = (tokens * nspan + sub - 1) / sub;  // sub-chunks' spans
     const long pairs = (work + 3) / 4, full = 4L * g_cus, rest = pairs % full;
-    double us = (double)(pairs / full) * (6.0 + 18.0 * passes + 0.4 * catchup);
+    double us = (double)(pairs / full) * (6.0 + 18.0 * passes + 0.5 * catchup);
     if (rest > full / 2)
-      us += (0.9 + 0.1 * (2.0 * rest / full - 1.0)) * (6.0 + 18.0 * passes + 0.8 * catchup);
+      us += (0.9 + 0.1 * (2.0 * rest / full - 1.0)) * (6.0 + 18.0 * passes + catchup);
     else if (rest > 0)
-      us += 6.0 + 11.4 * passes + 0.28 * catchup;
+      us += 6.0 + 11.4 * passes + 0.42 * catchup;
     if (nspan == 1 || us < 0.95 * best_us) {
       best = nspan;
       best_us = us;

@@ -78,11 +78,14 @@ __device__ __forceinline__ void load_token_mix(TokenInputs& in, bool& kzero, con
 }
 
 // MIX: unit-normalise the key and query rows (the 16 lanes of the row hold
-// its 64 elements, 4 each).
+// its 64 elements, 4 each).  The multiply-adds are spelled out: left to the
+// compiler, which product it folds into which differs between a span's
+// catch-up and its turns, and a token's key has to be the same bits in both.
+__device__ __forceinline__ float squares4(const float (&x)[4]) {
+  return __builtin_fmaf(x[3], x[3], __builtin_fmaf(x[2], x[2], __builtin_fmaf(x[1], x[1], x[0] * x[0])));
+}
 __device__ __forceinline__ void mix_token(TokenInputs& in, bool kzero) {
-  float sk = 0.f, sq = 0.f;
-  sk += in.k[0] * in.k[0] + in.k[1] * in.k[1] + in.k[2] * in.k[2] + in.k[3] * in.k[3];
-  sq += in.q[0] * in.q[0] + in.q[1] * in.q[1] + in.q[2] * in.q[2] + in.q[3] * in.q[3];
+  const float sk = squares4(in.k), sq = squares4(in.q);
   const float rk = kzero ? 0.f : __builtin_amdgcn_rsqf(sum16(sk) + 1e-6f);
   const float rq = __builtin_amdgcn_rsqf(sum16(sq) + 1e-6f);
 #pragma unroll
@@ -145,15 +148,24 @@ __device__ __forceinline__ float row_value(float x, int mu) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 16 * mu));
 }
 
+// E = l E + kk, one rounding, l per 16-lane row (four elements each).
+__device__ __forceinline__ void decay_add(f16& E, const float (&l)[4], const f16& kk) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) E[r] = __builtin_fmaf(l[r >> 2], E[r], kk[r]);
+}
+
 // Wave W's half of the evidence that its pair's spans start from, to LDS: the
-// sub-chunk's start states times -c, decayed over the `catchup` tokens before
-// each span (per 16-lane row; the first is sequence token `first`), and their
-// weighted outer products.  Those are summed from the last token back, each
-// weighted by the decays after it, on the rank-one four-block fp32 MFMA (one
-// rounding per token and element, as the turns' updates have) over blocks in
-// the exchanged layout (rows16.hpp).  Per wave and token five MFMAs; applying
-// the turns' updates one by one took 0.42 us a token with the same MFMAs, and
-// 0.75 on DPP-fed multiply-adds in the row layout, instead of 0.28.
+// sub-chunks' start states times -c, then the rank-one updates of the
+// `catchup` tokens before each span (per 16-lane row; the first is sequence
+// token `first`).  A token's update is the turn's, the product rounded and
+// one multiply-add by the decay, here on the rank-one four-block fp32 MFMA over blocks in
+// the exchanged layout (rows16.hpp), so a token's evidence is the same to the
+// bit however its sub-chunk is split.  Per wave and token five MFMAs and 80
+// multiply-adds, a block's MFMA beside the multiply-adds of the block before
+// it; on DPP-fed multiply-adds in the row layout (224 instructions) a token
+// took 0.75 us, with each MFMA waited for about 1 us; it takes 0.42.  (Summing
+// the tokens' products first and decaying the start state once took 0.28, but
+// a batch row's bits then changed with the batch size.)
 template <typename In, bool MIX, int W>
 __device__ __forceinline__ void stage_evidence(f4* evidence, const float* start_s, int slot,
                                                float c, int sexp, int catchup, int first,
@@ -161,52 +173,7 @@ __device__ __forceinline__ void stage_evidence(f4* evidence, const float* start_
                                                const float* log_decay, const MixerIn& mix, int b,
                                                int h) {
   const int lane = threadIdx.x & 63, a = lane & 15, g = lane >> 4;
-  f16 E[5];
-#pragma unroll
-  for (int i = 0; i < 5; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) E[i][r] = 0.f;
-  const int most = wave_max4(catchup);
-  // A group's inputs are in flight while the previous group is applied.  Rows
-  // without a token to catch up read one in bounds and take a zero update.
-  TokenInputs cur[CATCHUP_GROUP], next[CATCHUP_GROUP];
-  bool kzero[CATCHUP_GROUP] = {};
-  auto load = [&](TokenInputs (&in)[CATCHUP_GROUP], int done) {
-#pragma unroll
-    for (int j = 0; j < CATCHUP_GROUP; ++j) {
-      const int back = catchup - 1 - (done + j), t = back >= 0 ? first + back : 0;
-      if constexpr (MIX)
-        load_token_mix(in[j], kzero[j], d, mix, beta, log_decay, b, h, t, a);
-      else
-        load_token(in[j], d, keys, keys, beta, log_decay, b, h, t, a);
-    }
-  };
-  float after = 0.f;  // summed log decays after the token
-  if (most > 0) load(cur, 0);
-  for (int done = 0; done < most; done += CATCHUP_GROUP) {
-    if constexpr (MIX)
-#pragma unroll
-      for (int j = 0; j < CATCHUP_GROUP; ++j) mix_token(cur[j], kzero[j]);
-    load(next, done + CATCHUP_GROUP);
-#pragma unroll
-    for (int j = 0; j < CATCHUP_GROUP; ++j) {
-      const bool in = done + j < catchup;
-      const float weight = __builtin_ldexpf(cur[j].beta, 2 * sexp) * expf(after);
-      float k[4], nbk[4];
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        k[m] = in ? cur[j].k[m] : 0.f;
-        nbk[m] = in ? -weight * cur[j].k[m] : 0.f;
-      }
-      for_staged_blocks<W>([&](int i, int I, int K) {
-        E[i] = __builtin_amdgcn_mfma_f32_16x16x1f32(k[K], nbk[I], E[i], 0, 0, 0);
-      });
-      after += in ? cur[j].log_lam : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < CATCHUP_GROUP; ++j) cur[j] = next[j];
-  }
-  const float scale = -c * expf(after);  // -c without a token before the span
+  // Every start state's loads go out together.
   f4 start[4][5];
 #pragma unroll
   for (int mu = 0; mu < 4; ++mu) {
@@ -215,16 +182,68 @@ __device__ __forceinline__ void stage_evidence(f4* evidence, const float* start_
       start[mu][i] = *reinterpret_cast<const f4*>(s0 + (16 * I + a) * 64 + 16 * K + 4 * g);
     });
   }
+  f16 E[5];
 #pragma unroll
   for (int mu = 0; mu < 4; ++mu) {
-    const float w = row_value(scale, mu);
-    for_staged_blocks<W>([&](int i, int I, int K) {
-      const f4 v = start[mu][i];
-      evidence[slot_quad(I, 4 * K + g) * 64 + 16 * mu + a] =
-          f4{w * v[0] + E[i][4 * mu], w * v[1] + E[i][4 * mu + 1], w * v[2] + E[i][4 * mu + 2],
-             w * v[3] + E[i][4 * mu + 3]};
-    });
+    const float nc = -row_value(c, mu);
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) E[i][4 * mu + e] = nc * start[mu][i][e];
   }
+  const int most = wave_max4(catchup);
+  // A group's inputs are in flight while the previous group is applied.  Rows
+  // without a token to catch up read one in bounds and take a zero update.
+  TokenInputs cur[CATCHUP_GROUP], next[CATCHUP_GROUP];
+  bool kzero[CATCHUP_GROUP] = {};
+  auto load = [&](TokenInputs (&in)[CATCHUP_GROUP], int from) {
+#pragma unroll
+    for (int j = 0; j < CATCHUP_GROUP; ++j) {
+      const int t = from + j < catchup ? first + from + j : 0;
+      if constexpr (MIX)
+        load_token_mix(in[j], kzero[j], d, mix, beta, log_decay, b, h, t, a);
+      else
+        load_token(in[j], d, keys, keys, beta, log_decay, b, h, t, a);
+    }
+  };
+  if (most > 0) load(cur, 0);
+  for (int from = 0; from < most; from += CATCHUP_GROUP) {
+    if constexpr (MIX)
+#pragma unroll
+      for (int j = 0; j < CATCHUP_GROUP; ++j) mix_token(cur[j], kzero[j]);
+    load(next, from + CATCHUP_GROUP);
+#pragma unroll
+    for (int j = 0; j < CATCHUP_GROUP; ++j) {
+      const bool in = from + j < catchup;
+      const float lam = in ? expf(cur[j].log_lam) : 1.f;
+      const float cbeta = __builtin_ldexpf(cur[j].beta, 2 * sexp);
+      float k[4], nbk[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        k[m] = in ? cur[j].k[m] : 0.f;
+        nbk[m] = in ? -cbeta * cur[j].k[m] : 0.f;
+      }
+      float l[4];
+#pragma unroll
+      for (int mu = 0; mu < 4; ++mu) l[mu] = row_value(lam, mu);
+      // A block's product is under way while the block before it is updated.
+      f16 kk[5];
+      for_staged_blocks<W>([&](int i, int I, int K) {
+        kk[i] = __builtin_amdgcn_mfma_f32_16x16x1f32(k[K], nbk[I], f16{}, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (i > 0) decay_add(E[i - 1], l, kk[i - 1]);
+      });
+      decay_add(E[4], l, kk[4]);
+    }
+#pragma unroll
+    for (int j = 0; j < CATCHUP_GROUP; ++j) cur[j] = next[j];
+  }
+  for_staged_blocks<W>([&](int i, int I, int K) {
+#pragma unroll
+    for (int mu = 0; mu < 4; ++mu)
+      evidence[slot_quad(I, 4 * K + g) * 64 + 16 * mu + a] =
+          f4{E[i][4 * mu], E[i][4 * mu + 1], E[i][4 * mu + 2], E[i][4 * mu + 3]};
+  });
 }
 
 // A sequence is a span of a sub-chunk's tokens, 1/nspan of it (the launch
@@ -348,7 +367,10 @@ __global__ __launch_bounds__(128 * PAIRS) void fwd_factor_kernel(
     const int seen = wait_turn(turn_count, tt, polls);
     const bool gave_up = seen < tt || (polls < 0 && off + tt > 0);
     if (gave_up && lane == 0) raise_count(turn_count, kPoisoned);
-    const float lam = gave_up || seen >= kPoisoned ? __builtin_nanf("") : expf(cur.log_lam);
+    float lam = gave_up || seen >= kPoisoned ? __builtin_nanf("") : expf(cur.log_lam);
+    // Keeps the choice of decay here (the compiler moves it onto every
+    // updated element: 160 selects a turn).
+    asm volatile("" : "+v"(lam));
     const float cbeta = __builtin_ldexpf(cur.beta, 2 * sexp);
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
@@ -358,8 +380,12 @@ __global__ __launch_bounds__(128 * PAIRS) void fwd_factor_kernel(
         f4 sv = evidence[slot_quad(m, q) * 64 + lane];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+          // The update's product rounded, then one multiply-add by the
+          // decay (rounding the larger product instead was 4% less exact):
+          // stage_evidence rounds the same way.
+#pragma clang fp contract(off)
           const int k = 4 * q + e;
-          sv[e] = lam * sv[e] + nbk * bcast16(cur.k[k >> 4], k & 15);
+          sv[e] = __builtin_fmaf(lam, sv[e], nbk * bcast16(cur.k[k >> 4], k & 15));
           A[m][k] = sv[e];
         }
         if (m != 0 || q != 3 || lane != 0) evidence[slot_quad(m, q) * 64 + lane] = sv;
