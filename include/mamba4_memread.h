@@ -456,8 +456,8 @@ int m4mr_spd_solve_backward(const float* factors, const float* solution,
  *          precision_max_condition (max over states of max / max(min,
  *          1e-30)), state_all_finite (1 / 0), cross_max_abs, floor_min,
  *          floor_max, in the reference's order.
- * The eigenvalues come from a cyclic Jacobi iteration in fp32, one wave per
- * state (absolute error about 1e-7 of the largest eigenvalue); the
+ * The eigenvalues come from a tridiagonalisation and Sturm counts in float64,
+ * one 256-thread block per state, rounded to float32; the
  * reference's eigvalsh (LAPACK on the host, or its TPU lowering) has no
  * counterpart to call on the device.
  */

@@ -20,7 +20,6 @@ mode, lm/kernels/mamba4_fused.py:183-232).
 from typing import NamedTuple
 
 import torch
-import torch.nn.functional as F
 
 from mamba4_amd import _lib
 
@@ -319,9 +318,16 @@ def _expanded(x, shape, device):
     return x if x.shape == shape else x.expand(shape)
 
 
-def _pad_last(x, width, value=0.0):
-    extra = width - x.shape[-1]
-    return x if extra == 0 else F.pad(x, (0, extra), value=value)
+def _aligned(t):
+    """t, or a copy where its storage offset leaves it off the 16 bytes that
+    the kernels read a state by."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _check_state(evidence):
+    """The decode step counts its states by the first two axes."""
+    if evidence.dim() != 4:
+        raise ValueError(f"a state's evidence is [B,H,D,D]; got {tuple(evidence.shape)}")
 
 
 def selective_gaussian_memory(
@@ -373,7 +379,7 @@ def selective_gaussian_memory(
         init_s = torch.as_tensor(initial.evidence).to(torch.float32)
         init_c = torch.as_tensor(initial.cross).to(torch.float32)
         _require_device(init_s, init_c)
-        init_s, init_c = init_s.contiguous(), init_c.contiguous()
+        init_s, init_c = _aligned(init_s.contiguous()), _aligned(init_c.contiguous())
     chunk = min(int(chunk_size), _lib.MAX_CHUNK)
     k, v, q, f = (t.contiguous() for t in (keys, values, queries, floor))
     beta, log_decay = beta.contiguous(), log_decay.contiguous()
@@ -411,6 +417,7 @@ def selective_decode(state, key, value, query, beta, log_decay, floor, solver=No
     evidence = torch.as_tensor(state.evidence)
     cross = torch.as_tensor(state.cross)
     _require_device(evidence, cross)
+    _check_state(evidence)
     inputs = (evidence, cross, key, value, query, beta, log_decay, floor)
     if torch.is_grad_enabled() and any(
         isinstance(t, torch.Tensor) and t.requires_grad for t in inputs
@@ -444,8 +451,7 @@ def selective_decode(state, key, value, query, beta, log_decay, floor, solver=No
             (cross.to(torch.float32).contiguous(), width, wide, 0),
             (key, None, wide, 0), (value, None, width, 0), (query, None, wide, 0),
             (floor, None, wide, 1))
-    # The kernel reads the states 16 bytes at a time.
-    old_s, old_c = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (old_s, old_c))
+    old_s, old_c = _aligned(old_s), _aligned(old_c)
     new = SelectiveState(torch.empty(old_s.shape, **f32), torch.empty(old_c.shape, **f32))
     out = _decode_step(old_s, old_c, new, key, value, query, beta, log_decay, floor)
     if (dim, value_dim) == (wide, width):
@@ -465,6 +471,7 @@ def selective_decode_(state, key, value, query, beta, log_decay, floor, solver=N
     _check_solver(solver)
     evidence, cross = state.evidence, state.cross
     _require_device(evidence, cross)
+    _check_state(evidence)
     dim, value_dim = evidence.shape[-1], cross.shape[-2]
     if dim != _lib.KEY_DIM or value_dim not in (_lib.VALUE_DIM, _lib.MAX_VALUE_DIM):
         raise ValueError("the in-place decode needs D = 64 and P = 64 or 128 states")
@@ -520,7 +527,7 @@ def selective_diagnostics(state, floor):
 
     ``state.evidence`` [..., D, D] (D <= 64) and ``state.cross`` [..., P, D]
     on the GPU; ``floor`` broadcasts to [..., D].  The eigenvalues come from
-    a Jacobi iteration on the device (m4mr_diagnostics).
+    a tridiagonalisation and Sturm counts on the device (m4mr_diagnostics).
     """
     lib = _lib.load()
     evidence, cross = state.evidence, state.cross

@@ -78,3 +78,40 @@ def test_narrow_decode_leaves_the_state_and_matches_padding(gpu_lib):
         assert torch.equal(got.output, want.output[..., :width])
         assert torch.equal(got.state.evidence, want.state.evidence[..., :dim, :dim])
         assert torch.equal(got.state.cross, want.state.cross[..., :width, :dim])
+
+
+def test_a_state_off_16_bytes_starts_a_prefill(gpu_lib):
+    """An initial state that is a view at any address, as decode takes it."""
+    import mamba4_amd as m4
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(4)
+    k, q = (torch.randn(1, 5, 2, 64, device="cuda", generator=gen) / 8 for _ in range(2))
+    v = torch.randn(1, 5, 2, 64, device="cuda", generator=gen)
+    beta, decay = torch.full((1, 5, 2), 0.5, device="cuda"), torch.full((1, 5, 2), -0.1, device="cuda")
+    floor = torch.ones(2, 64, device="cuda")
+    state = torch.eye(64, device="cuda").repeat(1, 2, 1, 1), torch.randn(1, 2, 64, 64, device="cuda")
+    skewed = []
+    for t in state:
+        flat = torch.zeros(t.numel() + 1, device="cuda")
+        flat[1:] = t.reshape(-1)
+        skewed.append(flat[1:].view(t.shape))
+    for grad in (False, True):
+        k = k.detach().requires_grad_(grad)
+        announce(f"skewed initial state grad={grad}")
+        want, got = (m4.selective_gaussian_memory(k, v, q, beta, decay, floor,
+                                                  initial=m4.SelectiveState(*s))
+                     for s in (state, skewed))
+        assert torch.equal(want.output, got.output)
+        assert torch.equal(want.state.cross, got.state.cross)
+
+
+def test_decode_refuses_a_state_without_batch_and_head_axes(gpu_lib):
+    import mamba4_amd as m4
+
+    flat = m4.SelectiveState(torch.zeros(6, 64, 64, device="cuda"),
+                             torch.zeros(6, 64, 64, device="cuda"))
+    k, v, q = (torch.zeros(6, 1, 64, device="cuda") for _ in range(3))
+    for step in (m4.selective_decode, m4.selective_decode_):
+        with pytest.raises(ValueError):
+            step(flat, k, v, q, 0.5, -0.1, torch.ones(1, 64, device="cuda"))
