@@ -1,7 +1,7 @@
 """selective_diagnostics on the GPU (m4mr_diagnostics) against the oracle.
 
-The eigenvalue extremes come from a float64 Jacobi iteration on the float32
-state, rounded to float32: they are checked to 2e-7 of themselves (fp32
+The eigenvalue extremes come from a float64 tridiagonalisation of the float32
+state and its Sturm counts, rounded to float32: they are checked to 2e-7 of themselves (fp32
 rounding is 6e-8) plus 1e-10 of the state's largest eigenvalue, and the
 condition number to 5e-7 relative; the finiteness flag, the cross maximum
 and the floor range are exact.
