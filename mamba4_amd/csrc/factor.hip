@@ -81,8 +81,10 @@ __device__ __forceinline__ void load_token_mix(TokenInputs& in, bool& kzero, con
 // its 64 elements, 4 each).  The multiply-adds are spelled out: left to the
 // compiler, which product it folds into which differs between a span's
 // catch-up and its turns, and a token's key has to be the same bits in both.
+// The second square is the rounded one, as the compiler has it where it is
+// free to choose.
 __device__ __forceinline__ float squares4(const float (&x)[4]) {
-  return __builtin_fmaf(x[3], x[3], __builtin_fmaf(x[2], x[2], __builtin_fmaf(x[1], x[1], x[0] * x[0])));
+  return __builtin_fmaf(x[3], x[3], __builtin_fmaf(x[2], x[2], __builtin_fmaf(x[0], x[0], x[1] * x[1])));
 }
 __device__ __forceinline__ void mix_token(TokenInputs& in, bool kzero) {
   const float sk = squares4(in.k), sq = squares4(in.q);

@@ -251,3 +251,39 @@ def test_mixer_read_full_size(gpu_lib, monkeypatch):
                                            chunk=64)
     expected = oracle.epilogue(read, var, row["value"], row["confidence_scale"], row["skip"])
     assert normwise(_host(res.output[3:4]), expected) <= 1e-4
+
+
+@pytest.mark.gpu
+def test_factor_kernel_rounds_the_second_square(gpu_lib):
+    """The factor kernel's lane sums four squares of a row, elements a, a + 16,
+    a + 32 and a + 48, the second one rounded before the multiply-adds: rows
+    (u, v, 0, 0) and (v, 0, u, 0) then have the same norm to the bit.  With
+    beta = 0 and a floor of 1 the solution is the normalised query itself."""
+    import torch
+
+    from gpu_helpers import announce
+    from mamba4_amd import mixer_read
+
+    time = 4096
+    announce("mixer_read: rounding of the factor kernel's row norms")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(31)
+    u, v = torch.randn(2, time, device="cuda", generator=gen)
+
+    def solved(elements):
+        query = torch.zeros(1, time, 1, 64, device="cuda")
+        for i, x in elements:
+            query[0, :, 0, i] = x
+        query.requires_grad_(True)
+        rows = torch.ones(1, time, 1, 64, device="cuda")
+        off = torch.full((1, time, 1), -200.0, device="cuda")
+        head = torch.zeros(1, device="cuda")
+        r = mixer_read(rows, rows, query, off, off, head, head, head,
+                       torch.full((1, 64), -200.0, device="cuda"), head, head, floor_min=1.0)
+        saved = r.output.grad_fn.saved_tensors
+        assert torch.equal(saved[16], torch.ones(1, 64, device="cuda"))  # the floor
+        return saved[17][0, :, 0]
+
+    a, b = solved([(0, u), (16, v)]), solved([(0, v), (32, u)])
+    torch.cuda.synchronize()
+    assert torch.equal(a[:, 0], b[:, 32]) and torch.equal(a[:, 16], b[:, 0])
