@@ -1079,18 +1079,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
         for (int i = 0; i < 4; ++i) out[(n0 + 16 * w + 4 * q + i) * PT + 16 * j + r] = acc[j][i];
     }
     __syncthreads();
-    if (!SPLIT) {
-      const float decay = expf(S.p[63]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] *= decay;
-    }
-    // rows^T vals: A(n, t) = rt[t * LQH + n], B(t, p) = vt[t * LV + p].
-    mma<4, 1, LQH, LV, 1, BF>(acc, rt, 16 * w, vt, 0, 0, C);
+    // rows^T vals: A(n, t) = rt[t * LQH + n], B(t, p) = vt[t * LV + p], summed
+    // from zero and then added to the decayed state by one multiply-add, as
+    // carry_kernel adds it: the states are the same bits in both forms.
+    f4 own[4];
+    zero(own);
+    mma<4, 1, LQH, LV, 1, BF>(own, rt, 16 * w, vt, 0, 0, C);
     if (SPLIT) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out[(n0 + 16 * w + 4 * q + i) * PT + 16 * j + r] = acc[j][i];
+        for (int i = 0; i < 4; ++i) out[(n0 + 16 * w + 4 * q + i) * PT + 16 * j + r] = own[j][i];
+    } else {
+      const float decay = expf(S.p[63]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[j][i] = __builtin_fmaf(decay, acc[j][i], own[j][i]);
     }
   }
   if (!BWD && !SPLIT && final_state) {
@@ -1194,7 +1199,8 @@ __global__ __launch_bounds__(256) void carry_kernel(Shape s, const float* adt, f
         if (k0 + j < count) {
           const int k = first + k0 + j;
           *reinterpret_cast<f4*>(saved + state_offset(s, b, h, BWD ? s.NC - 1 - k : k) + e) = acc;
-          acc = decay[k0 + j] * acc + own[j];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(decay[k0 + j], acc[i], own[j][i]);
         }
     }
   }

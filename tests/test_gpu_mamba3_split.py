@@ -1,6 +1,6 @@
 """The Mamba-3 scan's chunk-boundary states formed in parallel and carried (few
 sequences) against the walk (many): a batch row alone takes the first, in its
-batch the second."""
+batch the second, with the same bits."""
 
 import pytest
 import torch
@@ -55,9 +55,13 @@ def test_split_states_match_the_walk(gpu_lib, time, state, width, angles, dtype,
     walks, many = run(slice(0, batch))
     splits, one = run(slice(row, row + 1))
     assert walks == [1, 1, 0, 0, 0, 0] and splits == [0, 0, 1, 1, 1, 1]
-    # The states differ by float32 rounding (a chunk's sum added to the carried
-    # state rather than accumulated on it); with bfloat16 operands that turns a
-    # rounding of one in some thousands.  Phases and everything else are equal.
-    for i, (a, b) in enumerate(zip(many, one)):
-        a, b = a[row].double(), b[0].double()
-        assert (a - b).norm() <= tolerance * a.norm(), i
+    # The shared rows' gradients (c, b, angles) are summed over groups of heads
+    # that the batch size chooses: they agree to rounding, one of some thousands
+    # of bfloat16 ones turned by it.  Everything else is equal to the bit.
+    names = ["y", "final", "c", "b", "x", "adt", "dt", "trap", "angles"]
+    for name, a, b in zip(names, many, one):
+        if name in ("c", "b", "angles"):
+            a, b = a[row].double(), b[0].double()
+            assert (a - b).norm() <= tolerance * a.norm(), name
+        else:
+            assert torch.equal(a[row], b[0]), name
