@@ -541,9 +541,11 @@ int m4mr_epilogue_backward(const float* read, const float* variance, const float
  * (lm/models/mamba4.py:59-95; order_memory :46-56 is the same scan from the
  * decays) and, over one token from the cached state, the order head's cached
  * step (:283-287).  values, output [B,T,H,W] with 1 <= W <= 256; log_decay
- * [B,T,H]; chunk 1..64 (the result does not depend on it beyond rounding).
+ * [B,T,H]; chunk 1..64 (the kernels' own chunks are of 64 tokens whatever it
+ * is).  A batch row's results are the same bits at any batch size, as are its
+ * gradients (m4mr_order_backward).
  * workspace: m4mr_order_workspace_bytes(B, T, H, W, chunk) bytes, 256-byte
- * aligned (per-chunk carries).
+ * aligned (the carries of runs of 32 tokens).
  */
 size_t m4mr_order_workspace_bytes(int B, int T, int H, int W, int chunk);
 int m4mr_order_forward(const float* values, const float* log_decay, const float* initial,

@@ -1369,13 +1369,14 @@ bool bad_order_dims(int B, int T, int H, int W, int chunk, std::string* why) {
   return false;
 }
 
-m4::OrderDims order_dims(int B, int T, int H, int W, int chunk) {
-  return m4::OrderDims{B, T, H, W, chunk, (T + chunk - 1) / chunk};
+// The kernels' chunks and runs don't depend on the caller's chunk.
+m4::OrderDims order_dims(int B, int T, int H, int W) {
+  return m4::OrderDims{B, T, H, W, (T + 63) / 64, (T + 31) / 32};
 }
 
-// Chunk states [B,H,NC,W] then chunk totals [B,H,NC].
+// Run states [B,H,NR,W] then run decays [B,H,NR].
 size_t order_workspace(const m4::OrderDims& d, float** states, float** totals, void* base) {
-  const size_t slots = (size_t)d.B * d.H * d.NC;
+  const size_t slots = (size_t)d.B * d.H * d.NR;
   const size_t first = align256(slots * d.W * sizeof(float));
   if (base) {
     *states = static_cast<float*>(base);
@@ -1398,10 +1399,10 @@ unsigned order_walk_threads(int T, int W) {
 // 256 at 128), one block per compute unit at a time, and at best the time of
 // its traffic; the chunk kernels three launches of about 4 us and 3/2 of the
 // traffic at 4.5 TB/s.  Forward + backward, one pass against three: B16
-// T1000 H12 W128 103 / 152 us, B16 T1024 H8 W64 40 / 56, B1 T512 H1 W64
-// 15 / 35; the other way round B2 T4096 H16 W128 197 / 121, B4 T2048 H8 W64
-// 52 / 41.  Near the line (B4 T4096 H16 W64 114 / 109) three passes are taken
-// unless one is estimated 20% faster.
+// T1000 H12 W128 111 / 156 us, B16 T1024 H8 W64 48 / 68, B1 T512 H1 W64
+// 21 / 46; the other way round B2 T4096 H16 W128 201 / 129, B4 T2048 H8 W64
+// 62 / 57.  Near the line (B16 T4096 H3 W64 109 / 104) three passes are taken
+// unless one is estimated 20% faster.  Both give the same bits.
 bool order_walks(int B, int T, int H, int W) {
   const double runs = (T + 31) / 32, waves = order_walk_threads(T, W) / 64;
   const double steps = std::ceil(runs * ((W + 63) / 64) / waves);
@@ -1415,7 +1416,7 @@ bool order_walks(int B, int T, int H, int W) {
 size_t m4mr_order_workspace_bytes(int B, int T, int H, int W, int chunk) {
   std::string why;
   if (bad_order_dims(B, T, H, W, chunk, &why)) return 0;
-  return order_workspace(order_dims(B, T, H, W, chunk), nullptr, nullptr, nullptr);
+  return order_workspace(order_dims(B, T, H, W), nullptr, nullptr, nullptr);
 }
 
 int m4mr_order_forward(const float* values, const float* log_decay, const float* initial, int B,
@@ -1428,7 +1429,7 @@ int m4mr_order_forward(const float* values, const float* log_decay, const float*
     return fail(M4MR_EINVAL, "m4mr_order_forward: a required pointer is NULL");
   if (reinterpret_cast<uintptr_t>(workspace) & 255)
     return fail(M4MR_EINVAL, "m4mr_order_forward: workspace must be 256-byte aligned");
-  const m4::OrderDims d = order_dims(B, T, H, W, chunk);
+  const m4::OrderDims d = order_dims(B, T, H, W);
   float *states = nullptr, *totals = nullptr;
   if (workspace_bytes < order_workspace(d, &states, &totals, workspace))
     return fail(M4MR_EINVAL, "m4mr_order_forward: workspace too small");
@@ -1467,7 +1468,7 @@ int m4mr_order_backward(const float* values, const float* log_decay, const float
     return fail(M4MR_EINVAL, "m4mr_order_backward: a required pointer is NULL");
   if (reinterpret_cast<uintptr_t>(workspace) & 255)
     return fail(M4MR_EINVAL, "m4mr_order_backward: workspace must be 256-byte aligned");
-  const m4::OrderDims d = order_dims(B, T, H, W, chunk);
+  const m4::OrderDims d = order_dims(B, T, H, W);
   float *heads = nullptr, *totals = nullptr;
   if (workspace_bytes < order_workspace(d, &heads, &totals, workspace))
     return fail(M4MR_EINVAL, "m4mr_order_backward: workspace too small");

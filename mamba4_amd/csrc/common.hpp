@@ -828,8 +828,6 @@ struct StateArgs {
   const float* confidence_scale;
 };
 
-// Shape of the order head's scan: values [B,T,H,W] in chunks of `chunk`
-// tokens, NC of them.
 // One array of resize_kernel: `outer` matrices src_rows x src_cols to
 // dst_rows x dst_cols of `bytes`-byte elements (4 or 2), cut off or padded with
 // `fill`; `quads` of four columns in the destination, `aligned` where each
@@ -847,8 +845,10 @@ struct ResizeJobs {
   int count;
 };
 
+// Shape of the order head's scan: values [B,T,H,W] in NC chunks of 64 tokens,
+// NR runs of 32.
 struct OrderDims {
-  int B, T, H, W, chunk, NC;
+  int B, T, H, W, NC, NR;
 };
 
 }  // namespace m4

@@ -6,19 +6,23 @@
 //
 // Layout: values and output [B,T,H,W], log_decay [B,T,H], initial and the
 // initial-state gradient [B,H,W].  One thread per channel; a block covers
-// every channel of one (b, h) and one chunk of tokens, so a wave's access to
-// a token is one contiguous row of up to 64 floats.  Three passes each way:
-//   forward:  order_local  - each chunk's scan from zero: its end state and
-//                            total log decay;
-//             order_carry  - the state every chunk starts from, chunk by
-//                            chunk per (b, h, channel), in place;
-//             order_apply  - each chunk's scan from its start state.
+// every channel of one (b, h) and one chunk of 64 tokens, two runs of 32, so
+// a wave's access to a token is one contiguous row of up to 64 floats.  Three
+// passes each way:
+//   forward:  order_local  - each run's scan from zero: its end state and
+//                            its decay;
+//             order_carry  - the state every run starts from, run by run per
+//                            (b, h, channel), in place;
+//             order_apply  - each run's scan from its start state.
 //   backward: the same three over the reverse recurrence of the cotangent
 //             g_t = dout_t + lam_(t+1) g_(t+1): d v_t = (1 - lam_t) g_t,
 //             d log_decay_t = lam_t sum_c g_t,c (h_(t-1),c - v_t,c) (summed
 //             over channels in a fixed order), d initial = lam_0 g_0.
 // Where enough (b, h) fill the chip, or the sequence is short, one kernel each
-// way does the whole scan instead (order_walk, order_bwd_walk below).
+// way does the whole scan instead (order_walk, order_bwd_walk below).  Both
+// forms take the same runs, multiply-adds and sums in the same order (which
+// product of a step is rounded is spelled out), so a batch row has the same
+// bits whichever form its batch size selects.
 #include "common.hpp"
 
 namespace m4 {
@@ -38,8 +42,8 @@ __device__ __forceinline__ OrderBlock order_block(const OrderDims& d) {
   o.bh = blockIdx.x / d.NC;
   o.b = o.bh / d.H;
   o.h = o.bh % d.H;
-  o.t0 = o.n * d.chunk;
-  o.len = min(d.chunk, d.T - o.t0);
+  o.t0 = o.n * MAXC;
+  o.len = min(MAXC, d.T - o.t0);
   return o;
 }
 
@@ -55,6 +59,8 @@ __device__ __forceinline__ OrderBlock order_block(const OrderDims& d) {
 // ahead of their use instead of minimising registers.
 constexpr int ORDER_GROUP = 16;
 constexpr int ORDER_GROUPS = MAXC / ORDER_GROUP;
+constexpr int ORDER_RUN = MAXC / 2;
+constexpr int ORDER_RUN_GROUPS = ORDER_RUN / ORDER_GROUP;
 
 struct RowGroup {
   float x[ORDER_GROUP];
@@ -85,9 +91,9 @@ struct TokenGates {
     lam = expf(lg);
     inflow = -expm1f(lg);
   }
-  // Summed log decay of the chunk (every lane receives it).
-  __device__ __forceinline__ float total() const {
-    return group4_sum(row16_sum(lg));
+  // The decay over the chunk's run k (every lane receives it).
+  __device__ __forceinline__ float total(int k) const {
+    return expf(group4_sum(row16_sum(lane_id() / ORDER_RUN == k ? lg : 0.f)));
   }
 };
 
@@ -95,15 +101,20 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
 }
 
-// Forward pass 1: ends[bh][n][c] = the chunk's scan from zero at its last
-// token; totals[bh][n] = its summed log decay.
+// One step of the scan.
+__device__ __forceinline__ float order_step(float lam, float s, float inflow, float v) {
+  return __builtin_fmaf(lam, s, inflow * v);
+}
+
+// Forward pass 1: ends[bh][run][c] = the run's scan from zero at its last
+// token; totals[bh][run] = its decay.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void order_local_kernel(OrderDims d, const float* values,
                                                           const float* log_decay, float* ends,
                                                           float* totals) {
   const OrderBlock o = order_block(d);
   const int c = threadIdx.x, cc = min(c, d.W - 1);
   const TokenGates gate(d, o, log_decay);
-  const float g = gate.total();
+  const float decay[2] = {gate.total(0), gate.total(1)};
   const long stride = (long)d.H * d.W;
   const float* first = values + order_row(d, o.b, o.t0, o.h) * d.W + cc;
   RowGroup r[2];
@@ -115,42 +126,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 #pragma unroll
     for (int i = 0; i < ORDER_GROUP; ++i) {
       const int t = k * ORDER_GROUP + i;
-      s = lane_value(gate.lam, t) * s + lane_value(gate.inflow, t) * r[k & 1].x[i];
+      s = order_step(lane_value(gate.lam, t), s, lane_value(gate.inflow, t), r[k & 1].x[i]);
+    }
+    if ((k + 1) % ORDER_RUN_GROUPS == 0) {  // a run is done
+      const int half = k / ORDER_RUN_GROUPS, run = 2 * o.n + half;
+      const long slot = (long)o.bh * d.NR + run;
+      if (run < d.NR) {
+        if (c < d.W) ends[slot * d.W + c] = s;
+        if (c == 0) totals[slot] = decay[half];
+      }
+      s = 0.f;
     }
   }
-  const long slot = (long)o.bh * d.NC + o.n;
-  if (c < d.W) ends[slot * d.W + c] = s;
-  if (c == 0) totals[slot] = g;
 }
 
-// Chunks of a carry whose loads are issued together.
-constexpr int ORDER_CARRY_BATCH = 8;
+// Runs of a carry whose loads are issued together.
+constexpr int ORDER_CARRY_BATCH = 16;
 
-// Forward pass 2, grid B*H: turns ends into the state each chunk starts from
+// Forward pass 2, grid B*H: turns ends into the state each run starts from
 // (in place), starting from `initial`.
 __global__ __launch_bounds__(256) void order_carry_kernel(OrderDims d, const float* initial,
                                                           float* ends, const float* totals) {
   const int bh = blockIdx.x, c = threadIdx.x;
   if (c >= d.W) return;
   float s = initial ? initial[(long)bh * d.W + c] : 0.f;
-  for (int n0 = 0; n0 < d.NC; n0 += ORDER_CARRY_BATCH) {
+  for (int n0 = 0; n0 < d.NR; n0 += ORDER_CARRY_BATCH) {
     float local[ORDER_CARRY_BATCH], decay[ORDER_CARRY_BATCH];
 #pragma unroll
     for (int j = 0; j < ORDER_CARRY_BATCH; ++j) {
-      const long slot = (long)bh * d.NC + min(n0 + j, d.NC - 1);
+      const long slot = (long)bh * d.NR + min(n0 + j, d.NR - 1);
       local[j] = ends[slot * d.W + c];
       decay[j] = totals[slot];
     }
 #pragma unroll
     for (int j = 0; j < ORDER_CARRY_BATCH; ++j)
-      if (n0 + j < d.NC) {
-        ends[((long)bh * d.NC + n0 + j) * d.W + c] = s;
-        s = expf(decay[j]) * s + local[j];
+      if (n0 + j < d.NR) {
+        ends[((long)bh * d.NR + n0 + j) * d.W + c] = s;
+        s = __builtin_fmaf(decay[j], s, local[j]);
       }
   }
 }
 
-// Forward pass 3: each chunk's scan from its start state.
+// Forward pass 3: each run's scan from its start state.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void order_apply_kernel(OrderDims d, const float* values,
                                                           const float* log_decay,
                                                           const float* starts, float* output) {
@@ -161,78 +178,88 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   const float* first = values + order_row(d, o.b, o.t0, o.h) * d.W + cc;
   RowGroup r[2];
   load_group(r[0], o, 0, first, stride);
-  float s = starts[((long)o.bh * d.NC + o.n) * d.W + cc];
+  const float* start = starts + (long)o.bh * d.NR * d.W + cc;
+  const float next = start[(long)min(2 * o.n + 1, d.NR - 1) * d.W];
+  float s = start[2L * o.n * d.W];
   float* out = output + order_row(d, o.b, o.t0, o.h) * d.W + c;
 #pragma unroll
   for (int k = 0; k < ORDER_GROUPS; ++k) {
     if (k + 1 < ORDER_GROUPS) load_group(r[(k + 1) & 1], o, k + 1, first, stride);
+    if (k == ORDER_RUN_GROUPS) s = next;
 #pragma unroll
     for (int i = 0; i < ORDER_GROUP; ++i) {
       const int t = k * ORDER_GROUP + i;
-      s = lane_value(gate.lam, t) * s + lane_value(gate.inflow, t) * r[k & 1].x[i];
+      s = order_step(lane_value(gate.lam, t), s, lane_value(gate.inflow, t), r[k & 1].x[i]);
       if (t < o.len && c < d.W) out[t * stride] = s;
     }
   }
 }
 
-// Backward pass 1: the chunk's reverse scan of the cotangent from zero;
-// heads[bh][n][c] = lam_first g_first (what reaches the previous chunk),
-// totals[bh][n] = the chunk's summed log decay.
+// Backward pass 1: each run's reverse scan of the cotangent from zero;
+// heads[bh][run][c] = lam_first g_first (what reaches the previous run),
+// totals[bh][run] = the run's decay.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void order_bwd_local_kernel(OrderDims d, const float* d_output,
                                                               const float* log_decay,
                                                               float* heads, float* totals) {
   const OrderBlock o = order_block(d);
   const int c = threadIdx.x, cc = min(c, d.W - 1);
   const TokenGates gate(d, o, log_decay);
-  const float g = gate.total();
+  const float decay[2] = {gate.total(0), gate.total(1)};
   const long stride = (long)d.H * d.W;
   const float* first = d_output + order_row(d, o.b, o.t0, o.h) * d.W + cc;
   RowGroup r[2];
   load_group(r[1], o, ORDER_GROUPS - 1, first, stride);
-  float acc = 0.f;
+  float g = 0.f, up = 1.f;  // g_(t+1) and its decay lam_(t+1)
 #pragma unroll
   for (int k = ORDER_GROUPS - 1; k >= 0; --k) {
     if (k > 0) load_group(r[(k - 1) & 1], o, k - 1, first, stride);
 #pragma unroll
     for (int i = ORDER_GROUP - 1; i >= 0; --i) {
       const int t = k * ORDER_GROUP + i;
-      acc = lane_value(gate.lam, t) * ((t < o.len ? r[k & 1].x[i] : 0.f) + acc);
+      g = __builtin_fmaf(up, g, t < o.len ? r[k & 1].x[i] : 0.f);
+      up = lane_value(gate.lam, t);
+    }
+    if (k % ORDER_RUN_GROUPS == 0) {  // a run is done
+      const int half = k / ORDER_RUN_GROUPS, run = 2 * o.n + half;
+      const long slot = (long)o.bh * d.NR + run;
+      if (run < d.NR) {
+        if (c < d.W) heads[slot * d.W + c] = up * g;
+        if (c == 0) totals[slot] = decay[half];
+      }
+      g = 0.f;
+      up = 1.f;
     }
   }
-  const long slot = (long)o.bh * d.NC + o.n;
-  if (c < d.W) heads[slot * d.W + c] = acc;
-  if (c == 0) totals[slot] = g;
 }
 
-// Backward pass 2, grid B*H: heads become the cotangent reaching each
-// chunk's last token from later chunks (in place); what reaches the initial
-// state is its gradient.
+// Backward pass 2, grid B*H: heads become the cotangent reaching each run's
+// last token from later runs (in place); what reaches the initial state is
+// its gradient.
 __global__ __launch_bounds__(256) void order_bwd_carry_kernel(OrderDims d, float* heads,
                                                               const float* totals,
                                                               float* d_initial) {
   const int bh = blockIdx.x, c = threadIdx.x;
   if (c >= d.W) return;
   float s = 0.f;
-  for (int top = d.NC; top > 0; top -= ORDER_CARRY_BATCH) {
+  for (int top = d.NR; top > 0; top -= ORDER_CARRY_BATCH) {
     float local[ORDER_CARRY_BATCH], decay[ORDER_CARRY_BATCH];
 #pragma unroll
     for (int j = 0; j < ORDER_CARRY_BATCH; ++j) {
-      const long slot = (long)bh * d.NC + max(top - 1 - j, 0);
+      const long slot = (long)bh * d.NR + max(top - 1 - j, 0);
       local[j] = heads[slot * d.W + c];
       decay[j] = totals[slot];
     }
 #pragma unroll
     for (int j = 0; j < ORDER_CARRY_BATCH; ++j)
       if (top - 1 - j >= 0) {
-        heads[((long)bh * d.NC + top - 1 - j) * d.W + c] = s;
-        s = local[j] + expf(decay[j]) * s;
+        heads[((long)bh * d.NR + top - 1 - j) * d.W + c] = s;
+        s = __builtin_fmaf(decay[j], s, local[j]);
       }
   }
   if (d_initial) d_initial[(long)bh * d.W + c] = s;
 }
 
 constexpr int ORDER_MAX_WAVES = 4;  // W <= 256
-constexpr int ORDER_HALF = MAXC / 2;
 
 template <int CTRL>
 __device__ __forceinline__ float order_dpp(float x) {
@@ -243,7 +270,7 @@ __device__ __forceinline__ float order_dpp(float x) {
 // DPP pattern pairing exactly those lanes within a row: the lane with the
 // bit set keeps (and sums) the upper element.
 template <int CTRL, int BIT, int HALF>
-__device__ __forceinline__ void dpp_stage(float (&x)[ORDER_HALF], int l) {
+__device__ __forceinline__ void dpp_stage(float (&x)[ORDER_RUN], int l) {
   const bool hi = (l >> BIT) & 1;
 #pragma unroll
   for (int i = 0; i < HALF; ++i) {
@@ -260,7 +287,7 @@ __device__ __forceinline__ void dpp_stage(float (&x)[ORDER_HALF], int l) {
 // partner's element of the kept half), bits 3..0 by DPP row_mirror (lane
 // 15 - i), row_half_mirror (7 - i) and quad permutations, each pairing lanes
 // that differ in that bit and agree in the bits above it.
-__device__ __forceinline__ float wave_sums32(float (&x)[ORDER_HALF]) {
+__device__ __forceinline__ float wave_sums32(float (&x)[ORDER_RUN]) {
   const int l = lane_id();
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -280,10 +307,12 @@ __device__ __forceinline__ float wave_sums32(float (&x)[ORDER_HALF]) {
   return x[0] + order_dpp<0xB1>(x[0]);  // quad_perm [1,0,3,2]
 }
 
-// Backward pass 3: the chunk's reverse scan from the carried cotangent,
+// Backward pass 3: each run's reverse scan from the carried cotangent,
 // d values, and d log_decay summed over channels (within each wave by the
-// butterfly above, then over the waves in order).  Groups of the chunk from
-// the last down, each loaded while the one after it is used.
+// butterfly above, then over the waves in order).  h_(t-1) is rebuilt from the
+// values and the one stored output before the run, as the one-pass kernel
+// rebuilds it, and needs no pass over the outputs (B2 T4096 H16 W128: 43 us,
+// 53 with one).  Both runs' rows load at once, the second run's first.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void order_bwd_apply_kernel(
     OrderDims d, const float* values, const float* log_decay, const float* initial,
     const float* output, const float* d_output, const float* carried, float* d_values,
@@ -294,46 +323,49 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   const bool on = c < d.W;
   const int cc = min(c, d.W - 1);
   const TokenGates gate(d, o, log_decay);
-  float acc = on ? carried[((long)o.bh * d.NC + o.n) * d.W + c] : 0.f;
-  // The state before the chunk: the previous token's output, or the initial
-  // state (zero when absent) before the first token.
-  const float h_before = o.t0 > 0   ? output[order_row(d, o.b, o.t0 - 1, o.h) * d.W + cc]
-                         : initial ? initial[(long)o.bh * d.W + cc]
-                                   : 0.f;
-  struct Group {
-    float dy[ORDER_GROUP], v[ORDER_GROUP], prev[ORDER_GROUP];
+  struct Run {
+    float dy[ORDER_RUN], v[ORDER_RUN], h, g;
   };
-  auto load = [&](Group& r, int g) {
+  Run r[2];
 #pragma unroll
-    for (int i = 0; i < ORDER_GROUP; ++i) {
-      const int t = min(g * ORDER_GROUP + i, o.len - 1);
-      const long row = order_row(d, o.b, o.t0 + t, o.h);
-      r.dy[i] = d_output[row * d.W + cc];
-      r.v[i] = values[row * d.W + cc];
-      r.prev[i] = t > 0 ? output[(row - d.H) * d.W + cc] : h_before;
+  for (int k = 1; k >= 0; --k) {
+    const int t0 = o.t0 + ORDER_RUN * k;
+    r[k].g = carried[((long)o.bh * d.NR + min(2 * o.n + k, d.NR - 1)) * d.W + cc];
+    // The state before the run: the previous token's output, or the initial
+    // state (zero when absent) before the first token.
+    r[k].h = t0 > 0   ? output[order_row(d, o.b, min(t0, d.T) - 1, o.h) * d.W + cc]
+             : initial ? initial[(long)o.bh * d.W + cc]
+                       : 0.f;
+#pragma unroll
+    for (int i = 0; i < ORDER_RUN; ++i) {
+      const long at = order_row(d, o.b, o.t0 + min(ORDER_RUN * k + i, o.len - 1), o.h) * d.W + cc;
+      r[k].dy[i] = d_output[at];
+      r[k].v[i] = values[at];
     }
     __builtin_amdgcn_sched_barrier(0);
-  };
-  Group r[2];
-  float term[ORDER_HALF];
-  load(r[1], ORDER_GROUPS - 1);
+  }
 #pragma unroll
-  for (int k = ORDER_GROUPS - 1; k >= 0; --k) {
-    if (k > 0) load(r[(k - 1) & 1], k - 1);
-    const Group& cur = r[k & 1];
+  for (int k = 1; k >= 0; --k) {
+    // v becomes h_(t-1) - v_t.
+    float h = r[k].h, g = r[k].g, up = 1.f, term[ORDER_RUN];
 #pragma unroll
-    for (int i = ORDER_GROUP - 1; i >= 0; --i) {
-      const int t = k * ORDER_GROUP + i;
+    for (int i = 0; i < ORDER_RUN; ++i) {
+      const int t = ORDER_RUN * k + i;
+      const float v = r[k].v[i];
+      r[k].v[i] = h - v;
+      h = order_step(lane_value(gate.lam, t), h, lane_value(gate.inflow, t), v);
+    }
+#pragma unroll
+    for (int i = ORDER_RUN - 1; i >= 0; --i) {
+      const int t = ORDER_RUN * k + i;
       const bool in = t < o.len && on;
-      const float gt = (in ? cur.dy[i] : 0.f) + acc;
-      if (in) d_values[order_row(d, o.b, o.t0 + t, o.h) * d.W + c] = lane_value(gate.inflow, t) * gt;
-      term[t % ORDER_HALF] = in ? gt * (cur.prev[i] - cur.v[i]) : 0.f;
-      acc = lane_value(gate.lam, t) * gt;
+      g = __builtin_fmaf(up, g, t < o.len ? r[k].dy[i] : 0.f);
+      if (in) d_values[order_row(d, o.b, o.t0 + t, o.h) * d.W + c] = lane_value(gate.inflow, t) * g;
+      term[i] = in ? g * r[k].v[i] : 0.f;
+      up = lane_value(gate.lam, t);
     }
-    if (k % 2 == 0) {  // a half of the chunk is done
-      const float sum = wave_sums32(term);
-      if ((l & 1) == 0) part[wave][k / 2 * ORDER_HALF + (l >> 1)] = sum;
-    }
+    const float sum = wave_sums32(term);
+    if ((l & 1) == 0) part[wave][ORDER_RUN * k + (l >> 1)] = sum;
   }
   __syncthreads();
   const int waves = (int)(blockDim.x >> 6);
@@ -354,13 +386,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // rebuilds h_(t-1) from the values and the one stored output before its run.
 //
 // Bound by HBM: 2 + 3 passes over the values' size instead of the three-pass
-// kernels' 3 + 5 (B16 T1000 H12 W128: 37 us forward and 66 backward, 5.3 and
-// 4.5 TB/s, against 53 and 99).  It needs a (b, h) per compute unit or so to
+// kernels' 3 + 4 (B16 T1000 H12 W128: 40 us forward and 71 backward, 4.9 and
+// 4.1 TB/s, against 61 and 95).  It needs a (b, h) per compute unit or so to
 // fill the chip, the three-pass kernels a chunk (order_walks in the host code
-// chooses).  A wave's decays stay in scalar registers for both scans (read
-// again from their lanes the forward took 40 us).  Runs of 32 tokens: the
-// backward's two values per token fill the 128 registers that sixteen waves
-// leave each lane.
+// chooses).  The decays and the row offsets are scalars; some 60 of them
+// overflow into lanes of vector registers.  (Stepping from row to row, so that
+// none did, had the forward at 41 us instead of 39 on one card.)  Runs of 32
+// tokens: the backward's two values per token fill the 128 vector registers
+// that sixteen waves leave each lane, without scratch memory as long as its
+// stores step from row to row (by offsets, 12 bytes a lane spilled).
 constexpr int WALK_TOKENS = 32;
 constexpr int WALK_MAX_WAVES = 16;
 
@@ -435,12 +469,12 @@ __global__ __launch_bounds__(64 * WALK_MAX_WAVES) void order_walk_kernel(
     float x[WALK_TOKENS];
     load_run(x, d, w, t0, len, values);
     const WalkGates gate(d, w, t0, len, log_decay);
-    float lam[WALK_TOKENS], s = 0.f;  // the decays in scalar registers
+    float lam[WALK_TOKENS], s = 0.f;
 #pragma unroll
     for (int i = 0; i < WALK_TOKENS; ++i) {
       lam[i] = lane_value(gate.lam, i);
       x[i] *= lane_value(gate.inflow, i);
-      s = lam[i] * s + x[i];
+      s = __builtin_fmaf(lam[i], s, x[i]);
     }
     ends[buf][wave][w.l] = s;
     decays[buf][wave] = gate.total();  // by every lane: its sum crosses lanes
@@ -448,19 +482,19 @@ __global__ __launch_bounds__(64 * WALK_MAX_WAVES) void order_walk_kernel(
     s = carry;
     for (int j = 0; j < w.groups; ++j) {
       if (j == w.tg) s = carry;
-      carry = decays[buf][j * columns] * carry + ends[buf][j * columns + column][w.l];
+      carry = __builtin_fmaf(decays[buf][j * columns], carry, ends[buf][j * columns + column][w.l]);
     }
     float* out = output + order_row(d, w.b, t0, w.h) * d.W + w.c;
     if (len == WALK_TOKENS && w.on) {
 #pragma unroll
       for (int i = 0; i < WALK_TOKENS; ++i) {
-        s = lam[i] * s + x[i];
+        s = __builtin_fmaf(lam[i], s, x[i]);
         out[i * stride] = s;
       }
     } else {
 #pragma unroll
       for (int i = 0; i < WALK_TOKENS; ++i) {
-        s = lam[i] * s + x[i];
+        s = __builtin_fmaf(lam[i], s, x[i]);
         if (i < len && w.on) out[i * stride] = s;
       }
     }
@@ -471,7 +505,7 @@ __global__ __launch_bounds__(64 * WALK_MAX_WAVES) void order_bwd_walk_kernel(
     OrderDims d, const float* values, const float* log_decay, const float* initial,
     const float* output, const float* d_output, float* d_values, float* d_log_decay,
     float* d_initial) {
-  static_assert(WALK_TOKENS == ORDER_HALF, "a run is one butterfly");
+  static_assert(WALK_TOKENS == ORDER_RUN, "a run is one butterfly");
   __shared__ float heads[2][WALK_MAX_WAVES][64];
   __shared__ float decays[2][WALK_MAX_WAVES];
   __shared__ float part[2][WALK_MAX_WAVES][WALK_TOKENS];
@@ -491,44 +525,45 @@ __global__ __launch_bounds__(64 * WALK_MAX_WAVES) void order_bwd_walk_kernel(
               : initial ? initial[(long)w.bh * d.W + w.cc]
                         : 0.f;
     const WalkGates gate(d, w, t0, len, log_decay);
-    float lam[WALK_TOKENS], acc = 0.f;
+    float g = 0.f, up = 1.f;  // g_(t+1) and its decay lam_(t+1)
 #pragma unroll
     for (int i = WALK_TOKENS - 1; i >= 0; --i) {
-      lam[i] = lane_value(gate.lam, i);
-      acc = lam[i] * (dy[i] + acc);
+      g = __builtin_fmaf(up, g, dy[i]);
+      up = lane_value(gate.lam, i);
     }
-    heads[buf][wave][w.l] = acc;
+    heads[buf][wave][w.l] = up * g;
     decays[buf][wave] = gate.total();  // by every lane: its sum crosses lanes
     // v becomes h_(t-1) - v_t.
 #pragma unroll
     for (int i = 0; i < WALK_TOKENS; ++i) {
       const float x = v[i];
       v[i] = h - x;
-      h = lam[i] * h + lane_value(gate.inflow, i) * x;
+      h = order_step(lane_value(gate.lam, i), h, lane_value(gate.inflow, i), x);
     }
     __syncthreads();
-    acc = carry;
+    g = carry;
     for (int j = w.groups - 1; j >= 0; --j) {
-      if (j == w.tg) acc = carry;
-      carry = heads[buf][j * columns + column][w.l] + decays[buf][j * columns] * carry;
+      if (j == w.tg) g = carry;
+      carry = __builtin_fmaf(decays[buf][j * columns], carry, heads[buf][j * columns + column][w.l]);
     }
-    float* dv = d_values + order_row(d, w.b, t0, w.h) * d.W + w.c;
+    up = 1.f;
+    float* dv = d_values + order_row(d, w.b, t0, w.h) * d.W + (WALK_TOKENS - 1) * stride;
     if (len == WALK_TOKENS && w.on) {
 #pragma unroll
-      for (int i = WALK_TOKENS - 1; i >= 0; --i) {
-        const float gt = dy[i] + acc;
-        dv[i * stride] = lane_value(gate.inflow, i) * gt;
-        v[i] *= gt;
-        acc = lam[i] * gt;
+      for (int i = WALK_TOKENS - 1; i >= 0; --i, dv -= stride) {
+        g = __builtin_fmaf(up, g, dy[i]);
+        dv[w.c] = lane_value(gate.inflow, i) * g;
+        v[i] *= g;
+        up = lane_value(gate.lam, i);
       }
     } else {
 #pragma unroll
-      for (int i = WALK_TOKENS - 1; i >= 0; --i) {
-        const float gt = dy[i] + acc;
+      for (int i = WALK_TOKENS - 1; i >= 0; --i, dv -= stride) {
         const bool in = i < len && w.on;
-        if (in) dv[i * stride] = lane_value(gate.inflow, i) * gt;
-        v[i] = in ? gt * v[i] : 0.f;
-        acc = lam[i] * gt;
+        g = __builtin_fmaf(up, g, dy[i]);
+        if (in) dv[w.c] = lane_value(gate.inflow, i) * g;
+        v[i] = in ? g * v[i] : 0.f;
+        up = lane_value(gate.lam, i);
       }
     }
     const float sum = wave_sums32(v);

@@ -72,8 +72,8 @@ def order_memory_chunked(values, log_decay, chunk_size=64, *, initial=None):
     """The gated vector scan of lm/models/mamba4.py:59-95 on the GPU.
 
     values [B,T,H,W] (W <= 256), log_decay [B,T,H]; returns h [B,T,H,W] in
-    float32.  ``chunk_size`` only sets the kernels' chunking (chunks above 64
-    tokens run as 64: the result is the same up to rounding).  ``initial``
+    float32.  ``chunk_size`` has to be positive and does not change the result
+    (the kernels' chunks are of 64 tokens whatever it is).  ``initial``
     [B,H,W] is the state before the first token (zero by default).
     """
     tensors = [values, log_decay] + ([] if initial is None else [initial])

@@ -246,6 +246,56 @@ def test_order_routes_match_oracle(gpu_lib, batch, time, heads, width, walks, in
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("initial", [False, True])
+@pytest.mark.parametrize(
+    "batch,time,heads,width",
+    # In their batch in one pass, alone in three: ragged runs and chunks, one
+    # 64-channel column, two and three.
+    [(300, 2049, 1, 63), (256, 2500, 2, 64), (256, 1500, 2, 130)],
+)
+def test_order_row_has_the_same_bits_in_both_forms(gpu_lib, batch, time, heads, width, initial):
+    from mamba4_amd import _lib, order_memory_chunked
+    from tests.gpu_helpers import announce
+
+    announce(f"order row bits B{batch} T{time} H{heads} W{width} init={initial}")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(time)
+
+    def normal(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen)
+
+    x = [normal(batch, time, heads, width),
+         -torch.nn.functional.softplus(normal(batch, time, heads) - 2.0)]
+    if initial:
+        x.append(normal(batch, heads, width))
+    d, row = normal(batch, time, heads, width), 3
+
+    def run(rows, chunk):
+        leaves = [t[rows].clone().requires_grad_(True) for t in x]
+        _lib.profile_reset()
+        _lib.profile_select(None)
+        _lib.profile_enable(True)
+        try:
+            out = order_memory_chunked(leaves[0], leaves[1], chunk,
+                                       initial=leaves[2] if initial else None)
+            grads = torch.autograd.grad(out, leaves, d[rows])
+            torch.cuda.synchronize()
+        finally:
+            _lib.profile_enable(False)
+        walks = [_lib.profile_read(n)[1] for n in ("order_walk", "order_bwd_walk")]
+        _lib.profile_reset()
+        return walks, [out.detach(), *grads]
+
+    walks, many = run(slice(0, batch), 64)
+    assert walks == [1, 1]
+    for chunk in (64, 24):
+        walks, one = run(slice(row, row + 1), chunk)
+        assert walks == [0, 0]
+        for i, (a, b) in enumerate(zip(many, one)):
+            assert torch.equal(a[row], b[0]), (chunk, i)
+
+
+@pytest.mark.gpu
 def test_order_cached_step_and_decay_form(gpu_lib):
     """The order head's cached decode step (lm/models/mamba4.py:283-287) is
     the scan over one token from the cache; order_memory takes the decays."""
