@@ -644,8 +644,7 @@ def main_mixer_read(args):
         torch.cuda.synchronize()
         return (time.perf_counter() - t0) / steps
 
-    # The separate path's state walk is the fused walk too (the fused entry
-    # point always takes it).  The two are timed in alternation, best of
+    # Both paths on the state walk.  The two are timed in alternation, best of
     # three each, so that neither gets the colder clocks of the first run.
     os.environ["M4MR_STATE_WALK"] = "fused"
     runs = [(timed(fused, args.steps), timed(separate, args.steps)) for _ in range(3)]

@@ -86,10 +86,14 @@ const char* m4mr_last_error(void);
  *          ceil(chunk/2) tokens, so NS = 2*NC, else NS = NC);
  *          start_cross [B,H,NC,P,D], the cross statistics at each chunk start.
  *          m4mr_start_counts() returns NC and NS.
- * The chunk-boundary states (here and in m4mr_backward) come from one fused
- * walk per (b, h) state sequence when B*H*(1 + P/64) reaches the device's
- * compute-unit count, else from chunk-parallel statistics plus a carry; the
- * environment variable M4MR_STATE_WALK=fused|split overrides the choice.
+ * The chunk-boundary states (here, in m4mr_backward and in the mixer's
+ * entries) come from one fused walk per (b, h) state sequence when
+ * B*H*(1 + P/64) reaches the device's compute-unit count or the chunks are
+ * few, else from chunk-parallel statistics plus a carry; the environment
+ * variable M4MR_STATE_WALK=fused|split overrides the choice.  Both forms give
+ * the same bits: a batch row's outputs, states and gradients don't depend on
+ * the batch size (the sums over the batch, d_floor and the per-head
+ * parameters', do).
  * The fused walks run with one LDS step buffer (three per compute unit)
  * when they outnumber two per compute unit, else with two;
  * M4MR_STATE_BUFFERS=1|2 overrides that (the same results either way).

@@ -153,8 +153,9 @@ constexpr size_t kChunkLdsBytes = 4 * m4::TILE * sizeof(float);
 constexpr size_t kGradsLdsBytes = 7 * m4::TILE * sizeof(float);
 constexpr size_t kGradsGateLdsBytes = 8 * m4::TILE * sizeof(float);  // + the S0 tile
 constexpr size_t kStatesLdsBytes = 4 * m4::TILE * sizeof(float);
-// The backward walks add one tile (the evidence state's transpose).
-constexpr size_t kStatesBwdExtra = m4::TILE * sizeof(float);
+// The backward walks add a tile per step buffer (the evidence products'
+// transposes).
+constexpr size_t kStatesBwdLdsBytes = 6 * m4::TILE * sizeof(float);
 // The widest LDS requests of the blocked SPD solves and of the wider ones.
 constexpr size_t kBlockLdsMax = sizeof(float) * m4::block_lds_floats(m4::kBlockMaxDim);
 constexpr size_t kWideLdsMax = sizeof(float) * 3 * m4::kWideMaxDim;
@@ -201,11 +202,9 @@ int configure() {
 #undef M4_CHUNK_ATTRS
              {(const void*)m4::states_kernel<false, float, false, 2>, kStatesLdsBytes},
              {(const void*)m4::states_kernel<false, m4::bf16_t, false, 2>, kStatesLdsBytes},
-             {(const void*)m4::states_kernel<true, float, false, 2>,
-              kStatesLdsBytes + kStatesBwdExtra},
+             {(const void*)m4::states_kernel<true, float, false, 2>, kStatesBwdLdsBytes},
              {(const void*)m4::states_kernel<false, float, true, 2>, kStatesLdsBytes},
-             {(const void*)m4::states_kernel<true, float, true, 2>,
-              kStatesLdsBytes + kStatesBwdExtra},
+             {(const void*)m4::states_kernel<true, float, true, 2>, kStatesBwdLdsBytes},
              {(const void*)m3::walk_kernel<false, float, true, false>, m3::kWalkLds},
              {(const void*)m3::walk_kernel<false, float, true, true>, m3::kWalkLds},
              {(const void*)m3::walk_kernel<true, float, true, false>, m3::kWalkLds},
@@ -288,8 +287,7 @@ int launch(const char* name, hipStream_t stream, F&& body) {
 // B4 T1024 H8 P64 (64 walks) 37 + 36 / 25 + 23 us, B8 T1024 H8 P128 (192) 42 + 41
 // / 52 + 50, B6 T4096 H8 P64 (96) 139 + 130 / 100 + 93, B16 T1024 H8 P64 (256)
 // 46 + 44 / 71 + 69.  The environment variable M4MR_STATE_WALK = "fused" or
-// "split" overrides the choice (both give the same states up to summation
-// order).
+// "split" overrides the choice (both give the same bits).
 bool fused_states(int B, int H, const Dims& d) {
   if (const char* mode = std::getenv("M4MR_STATE_WALK")) {
     if (std::strcmp(mode, "fused") == 0) return true;
@@ -611,8 +609,7 @@ int backward_impl(const char* entry, const In* keys, const In* values, const In*
       const bool one = !spill_free && states_single_buffer(B, H, d);
       const auto walk = one ? m4::states_kernel<true, float, GATE, 1> : m4::states_kernel<true, float, GATE, 2>;
       hipLaunchKernelGGL(walk, dim3(B * H, 1 + d.NV), dim3(512),
-                         (one ? kStatesLdsBytes / 2 : kStatesLdsBytes) + kStatesBwdExtra, st, d,
-                         args);
+                         one ? kStatesBwdLdsBytes / 2 : kStatesBwdLdsBytes, st, d, args);
     });
   } else {
     rc = launch("bwd_local", st, [&] {

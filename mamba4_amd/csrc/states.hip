@@ -13,6 +13,10 @@
 // stacked 64x64 tiles per state; each tile is one more product, and the scans
 // treat the NV * 4096 elements of a cross state alike.
 //
+// Either pair gives the same bits as states_kernel's walk below: the same
+// weights and decays from one scan of a chunk's log decays, a chunk's product
+// summed from zero in the same order, and one multiply-add per state and step.
+//
 // Backward: the transpose of that carry.  bwd_local_kernel computes each
 // chunk's start-state cotangents U = -(M + M^T)/2, M = Z^T diag(e^P) Y, and
 // V = dOut^T diag(e^P) Y; bwd_scan_kernel walks chunks in reverse,
@@ -27,6 +31,14 @@
 namespace m4 {
 
 __device__ __forceinline__ float* mat(float* base, long index) { return base + index * 4096; }
+
+// a x + b, one rounding each.
+__device__ __forceinline__ f4 fma4(float a, const f4& x, const f4& b) {
+  f4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = __builtin_fmaf(a, x[e], b[e]);
+  return r;
+}
 
 // acc += (A diag(wt))^T B over k in [k0, k0 + 16) for rows 16 w.. of the result
 // and its columns 4r + jb: A(i, k) = A[k][16w + i] wt[k], B(k, c) = B[k][c]
@@ -99,14 +111,13 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(
     load_chunk_scalars(cs, d, beta, log_decay, b, h, n);
   }
   if (threadIdx.x < 64) {
-    const int s = threadIdx.x;
+    // The sub-chunks' weights, and the chunk's, as states_kernel stages them.
+    const int s = threadIdx.x, cut = d.rsub == 2 ? min(d.sub, len) : len;
     const float p = cs.prefix[s], bt = cs.beta[s];  // this wave's own writes
-    for (int u = 0; u < d.rsub; ++u) {
-      const int first = sub_first(d, u), cnt = sub_len(d, n, u);
-      const float p_end = cnt > 0 ? cs.prefix[first + cnt - 1] : 0.f;
-      wt[u][s] = s >= first && s < first + cnt ? bt * expf(p_end - p) : 0.f;
-    }
-    wt[2][s] = s < len ? cs.tail[s] : 0.f;
+    const float mid = read_lane(p, cut - 1), last = read_lane(p, 63);
+    wt[0][s] = s < cut ? bt * expf(mid - p) : 0.f;
+    wt[1][s] = s >= cut ? bt * expf(last - p) : 0.f;
+    wt[2][s] = s < len ? bt * expf(read_lane(p, len - 1) - p) : 0.f;
   }
   if constexpr (MIX)
     rk.store_unit(K, mix.key_shift && !mix.previous && n == 0);
@@ -116,7 +127,7 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(
   if (d.NV > 1) rv1.store(V + TILE);
   __syncthreads();
   for (int u = 0; u < d.rsub; ++u) {
-    const int first = sub_first(d, u), end = first + sub_len(d, n, u);
+    const int first = sub_first(d, u), cnt = sub_len(d, n, u), end = cnt > 0 ? first + cnt : 0;
     f4 acc[4];
     zero4(acc);
     for (int k0 = first & ~15; k0 < end; k0 += 16) weighted_strip(acc, K, K, wt[u], k0, w);
@@ -136,33 +147,51 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(
   }
 }
 
-// exp(sum of log decays) over the tokens of the scan's steps first .. first +
-// count - 1 (count <= 64): sub-chunks (evidence) or chunks (cross statistics).
-// A 256-thread block, four threads a step, sixteen tokens each, every load at
-// once (a thread per step walked up to 64 of them, eight at a time).
-__device__ __forceinline__ void step_decays(float* decay, const Dims& d, const float* log_decay,
-                                            int b, int h, int first, int count, bool sub) {
-  const int k = threadIdx.x >> 2, part = threadIdx.x & 3, i = first + min(k, count - 1);
-  int t0, cnt;
-  if (sub) {
-    const int n = i / d.rsub, u = i % d.rsub;
-    t0 = n * d.chunk + sub_first(d, u);
-    cnt = sub_len(d, n, u);
-  } else {
-    t0 = i * d.chunk;
-    cnt = chunk_len(d, i);
-  }
-  float x[16], g = 0.f;
+// The decays of the scan's steps first .. first + count - 1 (count <= 64), the
+// two sub-chunks of each chunk (parts = 2) or chunks (parts = 1), from the
+// chunk's log-decay prefix as states_kernel takes them.  A 256-thread block: a
+// wave per chunk and a token per lane, every load at once, then a thread per
+// exponential (a wave per exponential had fwd_scan at 30 us, now 25, where B1
+// T4096 H8 P64 gives it two times 64 steps).
+struct StepSums {
+  float mid[64], last[64];  // the prefix at the first sub-chunk's end and the chunk's
+};
+__device__ __forceinline__ void step_decays(float* decay, StepSums& sums, const Dims& d,
+                                            const float* log_decay, int b, int h, int first,
+                                            int count, int parts) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
+  const int halves = parts - 1, n0 = first >> halves, chunks = count >> halves;
+  const int tokens = min(chunks * d.chunk, d.T - n0 * d.chunk);
+  // Tokens past the sequence and lanes past the chunk read zero.
+  const BufRsrc rows = buf_rsrc(log_decay + token_head(d, b, n0 * d.chunk, h),
+                                (unsigned)(tokens - 1) * d.H * 4 + 4);
+  const unsigned step = (unsigned)d.chunk * d.H * 4;
+  const unsigned token = l < d.chunk ? (unsigned)l * d.H * 4 : kNoRow;
+  float g[16], mid = 0.f, last = 0.f;  // lane j: of the wave's chunk j
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int t = 16 * part + j;
-    x[j] = log_decay[token_head(d, b, min(t0 + (t < cnt ? t : 0), d.T - 1), h)];
-  }
+  for (int j = 0; j < 16; ++j) g[j] = buf_load1(rows, token + (w + 4 * j) * step);
 #pragma unroll
-  for (int j = 0; j < 16; ++j) g += 16 * part + j < cnt ? x[j] : 0.f;
-  g += dpp_read<0xB1>(g);  // quad_perm [1,0,3,2]
-  g += dpp_read<0x4E>(g);  // quad_perm [2,3,0,1]
-  if (part == 0 && k < count) decay[k] = expf(g);
+  for (int j0 = 0; j0 < 16; j0 += 4) {
+    if (4 * j0 >= chunks) break;
+#pragma unroll
+    for (int j = j0; j < j0 + 4; ++j) {
+      const float p = wave_inclusive_sum(g[j]);
+      const int cut = max(min(d.sub, chunk_len(d, n0 + w + 4 * j)), 1);
+      float at_cut = read_lane(p, cut - 1), at_end = read_lane(p, 63);
+      // Read here, so that the choices below stay selects (no branch per chunk).
+      asm volatile("" : "+s"(at_cut), "+s"(at_end));
+      mid = l == j ? at_cut : mid;
+      last = l == j ? at_end : last;
+    }
+  }
+  if (l < 16) {
+    sums.mid[w + 4 * l] = mid;
+    sums.last[w + 4 * l] = last;
+  }
+  __syncthreads();
+  const int i = threadIdx.x, k = i >> halves;
+  if (i < count)
+    decay[i] = expf(parts == 1 ? sums.last[k] : i & 1 ? sums.last[k] - sums.mid[k] : sums.mid[k]);
 }
 
 // Steps of a scan whose loads are issued together.
@@ -183,6 +212,7 @@ __global__ __launch_bounds__(256) void fwd_scan_kernel(
   float* buf = (cross ? start_c : start_s) + (long)bh * steps * size;
   const float* init = cross ? init_c : init_s;
   __shared__ float decay[64];
+  __shared__ StepSums sums;
   f4 running = f4{0.f, 0.f, 0.f, 0.f};
   if (init) running = *reinterpret_cast<const f4*>(init + (long)bh * size + elem);
   for (int base = 0; base < steps; base += 64) {
@@ -197,7 +227,7 @@ __global__ __launch_bounds__(256) void fwd_scan_kernel(
     };
     load(0);
     __syncthreads();  // the previous steps' decays are read
-    step_decays(decay, d, log_decay, b, h, base, count, !cross);
+    step_decays(decay, sums, d, log_decay, b, h, base, count, cross ? 1 : d.rsub);
     __syncthreads();
     for (int i0 = 0; i0 < count; i0 += SCAN_BATCH) {
       f4 cur[SCAN_BATCH];
@@ -208,7 +238,7 @@ __global__ __launch_bounds__(256) void fwd_scan_kernel(
       for (int j = 0; j < SCAN_BATCH; ++j)
         if (i0 + j < count) {
           *reinterpret_cast<f4*>(buf + (long)(base + i0 + j) * size + elem) = running;
-          running = decay[i0 + j] * running + cur[j];
+          running = fma4(decay[i0 + j], running, cur[j]);
         }
     }
   }
@@ -300,6 +330,7 @@ __global__ __launch_bounds__(256) void bwd_scan_kernel(
   float* buf = (cross ? end_c : end_s) + (long)bh * d.NC * size;
   const float* fin = cross ? d_final_c : d_final_s;
   __shared__ float decay[64];
+  __shared__ StepSums sums;
   // Evidence: the scan carries G + G^T (it starts from D + D^T and adds the
   // local terms 2U = -(M + M^T), as bwd_local_kernel stores them), so every
   // stored end-state cotangent is symmetric; the initial-state gradient is
@@ -328,7 +359,7 @@ __global__ __launch_bounds__(256) void bwd_scan_kernel(
     };
     load(count - 1);
     __syncthreads();  // the previous steps' decays are read
-    step_decays(decay, d, log_decay, b, h, low, count, false);
+    step_decays(decay, sums, d, log_decay, b, h, low, count, 1);
     __syncthreads();
     for (int i0 = count - 1; i0 >= 0; i0 -= SCAN_BATCH) {
       f4 cur[SCAN_BATCH];
@@ -339,13 +370,13 @@ __global__ __launch_bounds__(256) void bwd_scan_kernel(
       for (int j = 0; j < SCAN_BATCH; ++j)
         if (i0 - j >= 0) {
           *reinterpret_cast<f4*>(buf + (long)(low + i0 - j) * size + elem) = running;
-          running = cur[j] + decay[i0 - j] * running;
+          running = fma4(decay[i0 - j], running, cur[j]);
           total *= decay[i0 - j];
         }
     }
   }
   float* dinit = cross ? d_init_c : d_init_s;
-  if (!cross) running = 0.5f * running + total * anti;
+  if (!cross) running = fma4(total, anti, 0.5f * running);
   *reinterpret_cast<f4*>(dinit + (long)bh * size + elem) = running;
 }
 
@@ -359,12 +390,15 @@ __global__ __launch_bounds__(256) void bwd_scan_kernel(
 // statistics never go through HBM.
 //   forward:  a = key (evidence) or value tile, b = key,
 //             wt = beta_t exp(P_last - P_t);  states ascend from init.
-//   backward: evidence a, b = (z, y) and (y, z) with wt = -exp(P_t) / 2,
-//             cross a = d_output tile, b = y with wt = exp(P_t) (MIX: the
-//             read gate g_t exp(P_t), d_output being the cotangent of the
-//             mixer's gated output g_t read_t + skip value_t);  states
-//             descend from the final-state cotangent (the transpose of the
-//             forward carry, as bwd_local_kernel + bwd_scan_kernel).
+//   backward: evidence a, b = (z, y) with wt = -exp(P_t), the product added
+//             with its transpose; cross a = d_output tile, b = y with wt =
+//             exp(P_t) (MIX: the read gate g_t exp(P_t), d_output being the
+//             cotangent of the mixer's gated output g_t read_t + skip
+//             value_t);  states descend from the final-state cotangent (the
+//             transpose of the forward carry, as bwd_local_kernel +
+//             bwd_scan_kernel).
+// A step's product is summed from zero and added to the decayed state by one
+// multiply-add, as the scans of the chunk-parallel pair add it.
 // A step's rows load into registers two steps before it multiplies.  NBUF =
 // 2: LDS holds two step buffers and each step takes one barrier (the next
 // step staged while this one multiplies).  NBUF = 1: one buffer, staged
@@ -387,7 +421,9 @@ struct alignas(16) StepBuffer {  // wt is read as float4
 
 // acc += (A diag(wt))^T-by-B over k in [k0, k0 + 16) for rows 16 s.. of the
 // result and its columns 4r + 2hf + j (j = 0, 1): A(i, k) = A[k][16s + i]
-// wt[k], B(k, c) = B[k][c] (the tile_mma_half QUAD convention).
+// wt[k], B(k, c) = B[k][c] (the tile_mma_half QUAD convention).  FIRST: from
+// zero, whatever acc holds.
+template <bool FIRST>
 __device__ __forceinline__ void weighted_block(f4 acc[2], const float* A, const float* B,
                                                const float* wt, int k0, int s, int hf) {
   const int l = lane_id(), r = l & 15, kk = k0 + 4 * (l >> 4);
@@ -398,8 +434,9 @@ __device__ __forceinline__ void weighted_block(f4 acc[2], const float* A, const 
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float2 b = *reinterpret_cast<const float2*>(B + (kk + e) * LDT + 4 * r + 2 * hf);
-    acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b.x, acc[0], 0, 0, 0);
-    acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b.y, acc[1], 0, 0, 0);
+    const bool zero = FIRST && e == 0;
+    acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b.x, zero ? f4{} : acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b.y, zero ? f4{} : acc[1], 0, 0, 0);
   }
 }
 
@@ -469,77 +506,63 @@ __attribute__((amdgpu_waves_per_eu(NBUF == 1 && BWD ? 6 : 1))) void states_kerne
       acc[1][q] = x.y;
     }
   }
-  // The backward evidence walk adds M + M^T per step (M = Z^T W Y), so its
-  // state is S = D + A + A^T with A the decayed sum of the M alone (one
-  // product per step instead of two) and D the decayed final-state cotangent
-  // (which need not be symmetric): acc holds A, dscale the decay of D, and
-  // A^T comes back through an LDS tile when a state is stored.  The chunk
-  // end states are stored as S + S^T = dscale (D + D^T) + 2 (A + A^T), which
-  // is all the chunk gradients use of them (exactly symmetric: each element
-  // and its mirror add the same two terms), so dfin holds D + D^T; the
-  // initial-state gradient is the full S, with D read again at the end.
-  // Both step buffer counts do this, so a batch's rows give the same bits
-  // whichever variant the batch size selects.  The symmetric store needs
-  // about 100 VGPRs in the two-buffer walk; the one-buffer walk is held to
-  // 80 for three blocks per CU.
+  // The backward evidence walk carries G + G^T: it starts from D + D^T, D the
+  // final-state cotangent (which need not be symmetric), and adds each step's
+  // product with its transpose, which comes back through an LDS tile.  Every
+  // chunk end state is then exactly symmetric, and the chunk gradients use
+  // nothing else of it; the initial-state gradient is half the last one plus
+  // the decayed antisymmetric part of D (dscale the decay), D read again at
+  // the end.  A step's product goes to the tile before the barrier that ends
+  // the reads of its step buffer and is added after it (add_own; one tile per
+  // step buffer).  Both step buffer counts do this, so a batch's rows give the
+  // same bits whichever variant the batch size selects.  The one-buffer walk
+  // is held to 80 VGPRs for three blocks per CU.
   const bool sym = BWD && !cross;
   const int r0 = 16 * s + 4 * (l >> 4), c0 = 4 * (l & 15) + 2 * hf;  // elem's row and column
-  f4 dfin[2];
   float dscale = 1.f;
-  dfin[0] = acc[0];
-  dfin[1] = acc[1];
   const float* const d_final = sym && g.first_s ? g.first_s + edge * 4096 : nullptr;
-  if (sym) {
-    zero2(acc);
-    if (d_final)
+  if (d_final)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) dfin[j] += *reinterpret_cast<const f4*>(d_final + (c0 + j) * 64 + r0);
-  }
-  float* const tr = smem + 2 * NBUF * TILE;  // the transpose tile (backward only)
-  // The state this lane holds (rows r0 + q, columns c0 + j), for dst
-  // (+ 64 q + j); the backward evidence's chunk end states as S + S^T, its
-  // last (the initial-state gradient, `last`) as S.
-  auto state_now = [&](float2 (&out)[4], bool last) {
-    if (sym) {
+    for (int j = 0; j < 2; ++j) acc[j] += *reinterpret_cast<const f4*>(d_final + (c0 + j) * 64 + r0);
+  float* const tr = smem + 2 * NBUF * TILE;  // the transpose tiles (backward only)
+  f4 own[2];        // the part's product,
+  float own_decay;  // and its decay
+  auto add_own = [&](int u) {
+    if (!sym) return;
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float2*>(tr + (r0 + q) * LDT + c0) = float2{acc[0][q], acc[1][q]};
-      __syncthreads();
-      f4 t[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) t[j] = *reinterpret_cast<const f4*>(tr + (c0 + j) * LDT + r0);
-      if (last) {
-        f4 dd[2];
-        zero2(dd);
-        if (d_final)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float2 x = *reinterpret_cast<const float2*>(d_final + elem + 64 * q);
-            dd[0][q] = x.x;
-            dd[1][q] = x.y;
-          }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          out[q] = float2{dscale * dd[0][q] + acc[0][q] + t[0][q],
-                          dscale * dd[1][q] + acc[1][q] + t[1][q]};
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          out[q] = float2{dscale * dfin[0][q] + 2.f * (acc[0][q] + t[0][q]),
-                          dscale * dfin[1][q] + 2.f * (acc[1][q] + t[1][q])};
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) out[q] = float2{acc[0][q], acc[1][q]};
+    for (int j = 0; j < 2; ++j) {
+      own[j] += *reinterpret_cast<const f4*>(tr + u * TILE + (c0 + j) * LDT + r0);
+      acc[j] = fma4(own_decay, acc[j], own[j]);
     }
+    dscale *= own_decay;
+  };
+  // The state this lane holds (rows r0 + q, columns c0 + j), for dst
+  // (+ 64 q + j).
+  auto state_now = [&](float2 (&out)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) out[q] = float2{acc[0][q], acc[1][q]};
   };
   auto store_state = [&](const float2 (&v)[4], float* dst) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) *reinterpret_cast<float2*>(dst + 64 * q) = v[q];
   };
+  // The state after the last step (the backward evidence's initial-state
+  // gradient).
   auto put_state = [&](float* dst) {
+    if (sym) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        f4 anti = f4{0.f, 0.f, 0.f, 0.f};
+        if (d_final) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) anti[q] = d_final[elem + 64 * q + j];
+          anti = 0.5f * (anti - *reinterpret_cast<const f4*>(d_final + (c0 + j) * 64 + r0));
+        }
+        acc[j] = fma4(dscale, anti, 0.5f * acc[j]);
+      }
+    }
     float2 v[4];
-    state_now(v, true);
+    state_now(v);
     store_state(v, dst);
   };
   // A step's start states (one per part), taken before its products and
@@ -624,7 +647,7 @@ __attribute__((amdgpu_waves_per_eu(NBUF == 1 && BWD ? 6 : 1))) void states_kerne
       const float p = wave_inclusive_sum(pg), last = read_lane(p, 63);
       const float mid = cut > 0 ? read_lane(p, cut - 1) : 0.f;  // cut is uniform
       if (BWD) {
-        float c = cross ? 1.f : -0.5f;
+        float c = cross ? 1.f : -1.f;
         if (GATED && cross) c = read_gate(cscale, pb);
         sb[u].wt[0][l] = c * expf(p);
       } else {
@@ -649,16 +672,28 @@ __attribute__((amdgpu_waves_per_eu(NBUF == 1 && BWD ? 6 : 1))) void states_kerne
     const float* tb = smem + 2 * u * TILE;
     const float* ta = own_a ? smem + (2 * u + 1) * TILE : tb;
     held_i = i;
-    auto one_part = [&](int part, float2 (&held)[4]) {
-      state_now(held, false);
-      const float dk = sb[u].decay[part];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[j] *= dk;
-      dscale *= dk;
-      // 16-token blocks that hold the part's tokens; the weights are zero
-      // outside the part.
+    // 16-token blocks that hold a part's tokens; the weights are zero outside
+    // the part (an empty part takes one block of zeros).
+    auto product = [&](int part, f4 (&sum)[2]) {
       const int lo = sb[u].lo[part], hi = lo < sb[u].hi[part] ? sb[u].hi[part] : 0;
-      for (int k0 = lo & ~15; k0 < hi; k0 += 16) weighted_block(acc, ta, tb, sb[u].wt[part], k0, s, hf);
+      const float* wt = sb[u].wt[part];
+      int k0 = lo & ~15;
+      weighted_block<true>(sum, ta, tb, wt, k0, s, hf);
+      for (k0 += 16; k0 < hi; k0 += 16) weighted_block<false>(sum, ta, tb, wt, k0, s, hf);
+    };
+    auto one_part = [&](int part, float2 (&held)[4]) {
+      state_now(held);
+      product(part, own);
+      own_decay = sb[u].decay[part];
+      if (sym) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float2*>(tr + u * TILE + (r0 + q) * LDT + c0) =
+              float2{own[0][q], own[1][q]};
+      } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = fma4(own_decay, acc[j], own[j]);
+      }
     };
     one_part(0, held0);
     if (parts == 2) one_part(1, held1);
@@ -675,6 +710,7 @@ __attribute__((amdgpu_waves_per_eu(NBUF == 1 && BWD ? 6 : 1))) void states_kerne
     for (int k = 0; k < steps; ++k) {
       multiply(k, 0);
       __syncthreads();  // every wave is done with the buffer
+      add_own(0);
       if (k + 1 < steps) stage(R, 0, i0 + (k + 1) * stride);
       store_held();
       fetch(R, i0 + (k + 2) * stride);
@@ -692,6 +728,7 @@ __attribute__((amdgpu_waves_per_eu(NBUF == 1 && BWD ? 6 : 1))) void states_kerne
     auto step = [&](int k, const StepRegs& next, StepRegs& spare) {
       const int i = i0 + k * stride, u = NBUF == 2 ? k & 1 : 0;
       fetch(spare, i + 2 * stride);
+      if (BWD && k > 0) add_own(u ^ 1);
       multiply(k, u);
       if constexpr (NBUF == 2) {
         if (k + 1 < steps) stage(next, u ^ 1, i + stride);
@@ -719,6 +756,7 @@ __attribute__((amdgpu_waves_per_eu(NBUF == 1 && BWD ? 6 : 1))) void states_kerne
     } else {
       step(0, R1, R0);
     }
+    if (BWD) add_own((steps - 1) & 1);
   }
   put_state((cross ? g.last_c : g.last_s) + edge * 4096 + elem);
 }

@@ -120,8 +120,8 @@ def test_mixer_read_matches_separate_path(gpu_lib, monkeypatch, batch, time, hea
     from gpu_helpers import announce, normwise
     from mamba4_amd import SelectiveState
 
-    # The fused op always takes the fused state walk; so does the separate path
-    # here (with one LDS step buffer in the cases with an initial state).
+    # Both paths on the state walk (with one LDS step buffer in the cases with
+    # an initial state).
     monkeypatch.setenv("M4MR_STATE_WALK", "fused")
     monkeypatch.setenv("M4MR_STATE_BUFFERS", "1" if with_initial else "2")
     announce(f"mixer_read vs separate B{batch} T{time} H{heads} P{value_dim} chunk={chunk} "

@@ -378,11 +378,13 @@ def state_walk(request, monkeypatch):
     return request.param[:5]
 
 
-@pytest.mark.parametrize("value_dim,chunk,time", [(5, 4, 21), (64, 64, 90), (128, 48, 100)])
+@pytest.mark.parametrize("value_dim,chunk,time", [(5, 4, 21), (64, 64, 90), (128, 48, 100),
+                                                  (128, 5, 400)])
 def test_state_walks_match_oracle(gpu_lib, state_walk, value_dim, chunk, time):
     """Forward and every gradient through either state path, with an initial
     state and final-state cotangents: ragged last chunks with an empty second
-    sub-chunk (T = 90, 100), P = 128, and chunks without sub-chunks (4)."""
+    sub-chunk (T = 90, 100), P = 128, chunks without sub-chunks (4, 5), and
+    more than 64 steps in the carries (T = 400 in chunks of 5)."""
     from mamba4_amd import _lib
 
     dim = 6 if value_dim == 5 else 64
@@ -421,7 +423,7 @@ def test_state_walks_match_oracle(gpu_lib, state_walk, value_dim, chunk, time):
 
 def test_state_walk_choice_at_full_batch(gpu_lib, monkeypatch):
     """At B*H*(1 + P/64) >= compute units the fused walk is the default, and
-    both walks agree on every output and gradient (summation order only)."""
+    both forms give the same bits in every output and gradient."""
     from mamba4_amd import _lib
 
     batch, heads, time = 32, 8, 70
@@ -448,10 +450,9 @@ def test_state_walk_choice_at_full_batch(gpu_lib, monkeypatch):
         results[mode + "_fused"] = _lib.profile_read("fwd_states")[1]
         _lib.profile_reset()
     assert results["auto_fused"] == 1 and results["split_fused"] == 0
-    # Rounding differences of the two summation orders, amplified by the
-    # solves in the gradients (floor 0.05).
-    for key, ref in results["split"].items():
-        assert normwise(results["auto"][key], ref) <= (1e-4 if key.startswith("d_") else 1e-5), key
+    for key in results["split"]:
+        if not key.endswith("_fused"):
+            np.testing.assert_array_equal(results["auto"][key], results["split"][key], err_msg=key)
     # The final state against a float64 recurrence of the same inputs.
     k, v = data["keys"].astype(np.float64), data["values"].astype(np.float64)
     lam = np.exp(data["log_decay"].astype(np.float64))
@@ -466,14 +467,17 @@ def test_state_walk_choice_at_full_batch(gpu_lib, monkeypatch):
     assert normwise(results["auto"]["cross"], c) <= 1e-5
 
 
+@pytest.mark.parametrize("walk", ["fused", "split"])
 @pytest.mark.parametrize("value_dim,chunk,batch,heads", [(64, 64, 2, 3), (128, 48, 2, 2),
                                                          (64, 64, 32, 8)])
-def test_bf16_inputs_match_the_upcast_path_bit_for_bit(gpu_lib, value_dim, chunk, batch, heads):
+def test_bf16_inputs_match_the_upcast_path_bit_for_bit(gpu_lib, monkeypatch, value_dim, chunk,
+                                                       batch, heads, walk):
     """bfloat16 keys, values and queries go to m4mr_forward_bf16 /
-    m4mr_backward_bf16, which widen them in the kernels; the reference
+    m4mr_backward_bf16_to_bf16, which widen them in the kernels; the reference
     upcasts them first (lm/kernels/mamba4.py:263-265).  Widening is exact,
     so outputs, states and every gradient equal the float32 path on the
-    upcast arrays bit for bit (both state walks: B*H = 6, 4 and 256)."""
+    upcast arrays bit for bit, with the states walked and carried."""
+    monkeypatch.setenv("M4MR_STATE_WALK", walk)
     from mamba4_amd import SelectiveState, _lib, selective_gaussian_memory
 
     data = arrays(time=90, heads=heads, dim=64, value_dim=value_dim, seed=value_dim + batch,
@@ -487,7 +491,7 @@ def test_bf16_inputs_match_the_upcast_path_bit_for_bit(gpu_lib, value_dim, chunk
                          device="cuda:0")
     d_var = torch.tensor(rng.normal(size=data["beta"].shape), dtype=torch.float32,
                          device="cuda:0")
-    announce(f"bf16 inputs P={value_dim} chunk={chunk} B{batch} H{heads} T90")
+    announce(f"bf16 inputs P={value_dim} chunk={chunk} B{batch} H{heads} T90 {walk}")
     results = []
     for dtype in (torch.bfloat16, torch.float32):
         qkv = [torch.tensor(data[n], device="cuda:0").to(torch.bfloat16).to(dtype)
@@ -504,6 +508,9 @@ def test_bf16_inputs_match_the_upcast_path_bit_for_bit(gpu_lib, value_dim, chunk
              + r.state.evidence.sum() + r.state.cross.sum()).backward()
         finally:
             _lib.profile_enable(False)
+        ran = [_lib.profile_read(n)[1] for n in ("fwd_states", "bwd_states", "fwd_stats",
+                                                 "fwd_scan", "bwd_local", "bwd_scan")]
+        assert ran == ([1, 1, 0, 0, 0, 0] if walk == "fused" else [0, 0, 1, 1, 1, 1])
         _lib.profile_reset()
         torch.cuda.synchronize()
         grads = [t.grad.float() for t in qkv + rest + init]
