@@ -4,6 +4,7 @@
 // fixed sequence of kernels on the caller's stream.  Nothing here allocates
 // device memory or synchronises; the only global state is the optional
 // profiling log (mutex-protected) and a per-thread error message.
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -161,13 +162,28 @@ constexpr size_t kBlockLdsMax = sizeof(float) * m4::block_lds_floats(m4::kBlockM
 constexpr size_t kWideLdsMax = sizeof(float) * 3 * m4::kWideMaxDim;
 
 bool configured = false;
-int g_cus = 256;  // compute units of the device (set by configure())
 std::mutex g_cfg_mu;
+
+// Compute units of the device, for the dispatch rules and persistent grids.
+// Read at the first need of any entry, so a rule never depends on which
+// entries ran before.
+int compute_units() {
+  static std::atomic<int> known{0};
+  int cus = known.load(std::memory_order_relaxed);
+  if (cus > 0) return cus;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+      cus <= 0)
+    return 256;  // no device: the launch reports it
+  known.store(cus, std::memory_order_relaxed);
+  return cus;
+}
 
 // Grid of a persistent chunk kernel: `per_cu` resident blocks per compute
 // unit, never more blocks than chunks.
 unsigned persistent_grid(unsigned chunks, int per_cu) {
-  const unsigned cap = (unsigned)(g_cus * per_cu);
+  const unsigned cap = (unsigned)(compute_units() * per_cu);
   return chunks < cap ? chunks : cap;
 }
 
@@ -244,11 +260,6 @@ int configure() {
     if (e != hipSuccess)
       return fail(M4MR_EHIP, std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
   }
-  int device = 0, cus = 0;
-  if (hipGetDevice(&device) == hipSuccess &&
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
-      cus > 0)
-    g_cus = cus;
   configured = true;
   return M4MR_OK;
 }
@@ -294,7 +305,7 @@ bool fused_states(int B, int H, const Dims& d) {
     if (std::strcmp(mode, "split") == 0) return false;
   }
   const double walks = (double)B * H * (1 + d.NV);
-  return walks >= g_cus || 2.0 + 2.2 * d.NC <= 8.0 + 0.0156 * walks * d.NC;
+  return walks >= compute_units() || 2.0 + 2.2 * d.NC <= 8.0 + 0.0156 * walks * d.NC;
 }
 
 // The fused walks with one LDS step buffer (three blocks per CU) when their
@@ -305,7 +316,7 @@ bool states_single_buffer(int B, int H, const Dims& d) {
     if (std::strcmp(n, "1") == 0) return true;
     if (std::strcmp(n, "2") == 0) return false;
   }
-  return (long)B * H * (1 + d.NV) > 2L * g_cus;
+  return (long)B * H * (1 + d.NV) > 2L * compute_units();
 }
 
 // Poll bound of the factor kernel's turn waits: 2^16, or M4MR_TURN_POLLS
@@ -336,7 +347,7 @@ int factor_spans(long tokens, int sub) {
     const int span = (sub + nspan - 1) / nspan, passes = (span + 1) / 2;
     const double catchup = (double)(nspan - 1) * span;  // of the last span; half on average
     const long work = (tokens * nspan + sub - 1) / sub;  // sub-chunks' spans
-    const long pairs = (work + 3) / 4, full = 4L * g_cus, rest = pairs % full;
+    const long pairs = (work + 3) / 4, full = 4L * compute_units(), rest = pairs % full;
     double us = (double)(pairs / full) * (6.0 + 18.0 * passes + 0.5 * catchup);
     if (rest > full / 2)
       us += (0.9 + 0.1 * (2.0 * rest / full - 1.0)) * (6.0 + 18.0 * passes + catchup);
@@ -494,7 +505,7 @@ int forward_impl(const char* entry, const In* keys, const In* values, const In* 
     const int nspan = factor_spans((long)B * H * T, d.sub);
     const unsigned spans = subseqs * nspan;
     const unsigned blocks4 = (spans + 15) / 16;
-    const int pairs = blocks4 % (unsigned)g_cus == 0 ? 4 : 2;
+    const int pairs = blocks4 % (unsigned)compute_units() == 0 ? 4 : 2;
     const dim3 grid((spans + 4 * pairs - 1) / (4 * pairs)), block(128 * pairs);
     const auto kernel = factors ? (pairs == 4 ? m4::fwd_factor_kernel<In, MIX, true, 4>
                                               : m4::fwd_factor_kernel<In, MIX, true, 2>)
@@ -1011,7 +1022,7 @@ namespace {
 // of its own, else per wave: P = 128, 48 states 17.5 against 22.8 us, 1,024
 // 26.9 / 29.8, 1,536 45.4 / 35.3, 16,384 337 / 263.
 bool decode_wide(long N) {
-  return (N + 3) / 4 <= g_cus;
+  return (N + 3) / 4 <= compute_units();
 }
 
 int decode_step(const char* entry, const float* evidence, const float* cross, float* new_evidence,
@@ -1403,7 +1414,7 @@ unsigned order_walk_threads(int T, int W) {
 bool order_walks(int B, int T, int H, int W) {
   const double runs = (T + 31) / 32, waves = order_walk_threads(T, W) / 64;
   const double steps = std::ceil(runs * ((W + 63) / 64) / waves);
-  const double rounds = std::ceil((double)B * H / g_cus);
+  const double rounds = std::ceil((double)B * H / compute_units());
   const double traffic = 2.0 * sizeof(float) * B * T * H * W / 4.5e6;  // us
   return std::fmax(3.0 + 4.2 * steps * rounds, traffic) < 0.8 * (12.0 + 1.5 * traffic);
 }
@@ -1557,7 +1568,7 @@ int m3_groups(int B, int T, int H) {
 // where it is estimated 10% faster.
 bool m3_split_walk(int B, int H, int NC) {
   if (NC > 65535) return false;  // a grid dimension
-  const double blocks = 2.0 * B * H, cus = g_cus;
+  const double blocks = 2.0 * B * H, cus = compute_units();
   const double step = blocks <= cus ? 4.7 : blocks <= 2 * cus ? 6.1 : 8.1;
   const double walk = NC * step * std::ceil(blocks / (3 * cus));
   const double split = 10.0 + 8.0 * ((NC - 1) / 16) + 0.033 * B * H * NC;

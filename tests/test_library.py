@@ -1,12 +1,15 @@
 """Host-only checks of the C ABI and the Python boundary (no GPU needed)."""
 
 import ctypes
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 import torch
 
 from mamba4_amd import _lib
+from mamba4_amd import build
 from mamba4_amd import memory
 
 
@@ -169,3 +172,39 @@ def test_mamba3_shapes_past_the_finish_kernels_32_bit_slabs_are_rejected():
         rc = entry(*([null] * 9), 1, (1 << 22) - 64, 1, 128, 1, 0, *([null] * 4), null)
         assert rc == _lib.EINVAL
         assert "NULL" in lib.m4mr_last_error().decode()
+
+
+_STUB = """
+int hipGetDevice(int* device) { *device = 0; return 0; }
+int hipDeviceGetAttribute(int* value, int attribute, int device) { *value = CUS; return 0; }
+int hipLaunchKernel(void) { return 100; }
+int hipGetLastError(void) { return 100; }
+"""
+_FIRST_CALL = """
+import ctypes, sys
+ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+lib.m4mr_order_workspace_bytes.restype = ctypes.c_size_t
+lib.m4mr_last_error.restype = ctypes.c_char_p
+p, shape = ctypes.c_void_p(4096), (16, 1000, 12, 128, 64)
+need = ctypes.c_size_t(lib.m4mr_order_workspace_bytes(*shape))
+lib.m4mr_order_forward(p, p, None, *shape, p, p, need, None)
+forward = lib.m4mr_last_error().decode().split(":")[0]
+lib.m4mr_order_backward(p, p, None, p, p, *shape, p, p, None, p, need, None)
+print(forward, lib.m4mr_last_error().decode().split(":")[0])
+"""
+
+
+@pytest.mark.parametrize("cus,routes", [(256, ["order_walk", "order_bwd_walk"]),
+                                        (16, ["order_local", "order_bwd_local"])])
+def test_dispatch_reads_the_compute_units_in_the_first_call(tmp_path, cus, routes):
+    """A process's first call takes the route of its device's compute-unit count,
+    not a default's: HIP's queries and launches are stubbed (no launch happens;
+    the failed one's name is in the error)."""
+    source, stub = tmp_path / "stub.c", tmp_path / "libstub.so"
+    source.write_text(_STUB)
+    subprocess.run(["gcc", "-shared", "-fPIC", f"-DCUS={cus}", "-o", stub, source], check=True)
+    done = subprocess.run([sys.executable, "-c", _FIRST_CALL, stub, build.LIBRARY],
+                          capture_output=True, text=True, timeout=120)
+    assert done.returncode == 0, done.stderr
+    assert done.stdout.split() == routes
