@@ -416,8 +416,8 @@ int m4mr_decode_step_to(const float* evidence, const float* cross,
  * consumes: for dim <= 64 the quad-run layout of M4MR_FACTOR_FLOATS (the
  * system padded to 64 with an identity block), above 64 the dense
  * [dim][dim] row-major factor (L below the diagonal, 1/L_ii on it, zero
- * above).  Above width 128 the factorization runs in `factors`, which is
- * then required; N < 2^31 above width 64.
+ * above).  Above width 128 `factors` is required (above 208 the
+ * factorization runs in it; up to there in LDS); N < 2^31 above width 64.
  * Replaces spd_solve and its forward rule (lm/kernels/mamba4.py:190-201,
  * _factor_and_solve :164-187, which take any width); every reference
  * backend ("loop", "blocked", "unrolled", "auto", "fused") solves the same

@@ -1089,8 +1089,7 @@ int m4mr_spd_solve(const float* precision, const float* rhs, long N, int dim, fl
   if (dim > M4MR_KEY_DIM) {
     if (dim > 128 && !factors)
       return fail(M4MR_EINVAL,
-                  "m4mr_spd_solve: above width 128 the factors buffer is required (the "
-                  "factorization runs in it)");
+                  "m4mr_spd_solve: above width 128 the factors buffer is required");
     if (int rc = configure()) return rc;
     if (dim <= m4::kBlockMaxDim) {
       const int waves = m4::block_waves(dim);

@@ -64,7 +64,8 @@ class _FusedScan(torch.autograd.Function):
                 _stream(),
             )
         )
-        # A cotangent that nothing reaches stays None (no zeros filled for it).
+        # A final state's cotangent that nothing reaches stays None (y's, which
+        # the library requires, is filled with zeros).
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(c, b, x, adt, dt, trap, angles, q_bias, k_bias, starts, phases)
         return y, final

@@ -164,8 +164,9 @@ class _MemoryRead(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, keys, values, queries, beta, log_decay, floor, init_s, init_c, chunk):
-        # A cotangent that nothing reaches stays None rather than a tensor of
-        # zeros filled for every call.
+        # A final state's cotangent that nothing reaches stays None and goes to
+        # the library as NULL (the output's and the variance's, which it
+        # requires, are filled with zeros in memread_backward).
         ctx.set_materialize_grads(False)
         ctx.dims = keys.shape[-1], values.shape[-1]
         ctx.has_initial = init_s is not None
@@ -287,7 +288,7 @@ def spd_solve(precision, rhs, backend=None):
     string selects the same HIP solve (the backend changes only the
     arithmetic schedule, never the solved system, lm/kernels/mamba4.py:193-194).
     Widths up to 64 solve four systems per wave; wider ones (up to 4096) one
-    system per 256-thread block.
+    system per block.
     """
     _check_solver(backend)
     precision = torch.as_tensor(precision)

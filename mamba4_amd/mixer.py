@@ -268,7 +268,8 @@ class _MixerRead(torch.autograd.Function):
         ctx.save_for_backward(key, value, query, beta_raw, dt_raw, beta_bias, dt_bias, a_log,
                               floor_raw, previous, confidence_scale, skip, read, variance,
                               beta, log_decay, floor, solved, factors, start_s, start_c)
-        # A cotangent that nothing reaches stays None (no zeros filled for it).
+        # A cotangent that nothing reaches stays None (the output's, which the
+        # library requires, is filled with zeros).
         ctx.set_materialize_grads(False)
         ctx.beta_max, ctx.floor_min, ctx.key_shift, ctx.chunk = (beta_max, floor_min,
                                                                  key_shift, chunk)

@@ -521,3 +521,44 @@ def test_bf16_inputs_match_the_upcast_path_bit_for_bit(gpu_lib, monkeypatch, val
         if 4 <= i < 7:
             want = want.to(torch.bfloat16).float()
         assert torch.equal(got, want), i
+
+
+@pytest.mark.parametrize("dim,value_dim,initial", [(42, 100, True), (33, 63, False), (64, 17, True),
+                                                   (5, 64, False)])
+def test_narrow_bf16_inputs_match_the_upcast_path_bit_for_bit(gpu_lib, dim, value_dim, initial):
+    """bfloat16 keys, values and queries narrower than the kernels' widths are
+    padded, and their bfloat16 gradients cut, two bytes an element: the same
+    bits as the float32 path on the upcast arrays, whose gradients are rounded
+    once."""
+    from mamba4_amd import SelectiveState, selective_gaussian_memory
+
+    batch, time, heads = 2, 71, 3
+    announce(f"narrow bf16 inputs D={dim} P={value_dim} init={initial}")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(dim)
+
+    def normal(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen)
+
+    qkv = [normal(batch, time, heads, n).to(torch.bfloat16) for n in (dim, value_dim, dim)]
+    rest = [torch.sigmoid(normal(batch, time, heads)), -torch.exp(normal(batch, time, heads) - 2.0),
+            normal(heads, dim).abs() + 0.1]
+    if initial:
+        root = normal(batch, heads, dim, 8)
+        rest += [torch.matmul(root, root.transpose(-1, -2).contiguous()) / 8,
+                 normal(batch, heads, value_dim, dim)]
+    cot = [normal(batch, time, heads, value_dim), normal(batch, time, heads),
+           normal(batch, heads, dim, dim), normal(batch, heads, value_dim, dim)]
+    results = []
+    for dtype in (torch.bfloat16, torch.float32):
+        leaves = [t.to(dtype).requires_grad_(True) for t in qkv]
+        leaves += [t.clone().requires_grad_(True) for t in rest]
+        r = selective_gaussian_memory(
+            *leaves[:6], initial=SelectiveState(*leaves[6:]) if initial else None)
+        out = [r.output, r.variance, r.state.evidence, r.state.cross]
+        grads = torch.autograd.grad(out, leaves, cot)
+        torch.cuda.synchronize()
+        assert all(g.dtype == t.dtype and g.shape == t.shape for g, t in zip(grads, leaves))
+        results.append([*out, *grads])
+    for i, (got, want) in enumerate(zip(*results)):
+        assert torch.equal(got, want.to(got.dtype)), i

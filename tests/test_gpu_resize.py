@@ -38,7 +38,13 @@ def test_resize_pads_and_cuts_like_torch(gpu_lib):
     got = _resized((a, None, 64, 0), (b, None, 64, 0), (c, 64, 64, 0), (d, None, 64, 1),
                    (e, None, 1, 0), (f, 100, 48, 0), (empty, None, 64, 0), (None, 64, 64, 0),
                    (a, None, 48, 0))
+    # Two-byte elements cut off: whole quads of columns, a ragged tail, and
+    # rows that start off a quad's alignment.
+    g, h = normal(5, 7, 64, dtype=torch.bfloat16), normal(3, 66, 70, dtype=torch.bfloat16)
+    cut = _resized((g, None, 48, 0), (g, None, 33, 0), (g, None, 1, 0), (h, 65, 63, 0))
     torch.cuda.synchronize()
+    for x, y in zip(cut, (g[..., :48], g[..., :33], g[..., :1], h[:, :65, :63])):
+        assert x.is_contiguous() and x.dtype == y.dtype and torch.equal(x, y)
     want = [F.pad(a, (0, 16)), F.pad(b, (0, 31)), F.pad(c, (0, 51, 0, 44)),
             F.pad(d, (0, 58), value=1.0), e[:, :1], f[..., :100, :48], F.pad(empty, (0, 61))]
     for x, y in zip(got, want):

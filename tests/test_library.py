@@ -106,7 +106,7 @@ def test_spd_solve_arguments_are_checked_before_any_launch():
     assert lib.m4mr_spd_solve(p, p, 0, 6, p, null, null) == _lib.EINVAL
     assert lib.m4mr_spd_solve(p, p, 4, 4097, p, null, null) == _lib.EINVAL
     assert "dim" in lib.m4mr_last_error().decode()
-    # Above width 128 the factorization runs in the factors buffer.
+    # Above width 128 the factors buffer is required.
     assert lib.m4mr_spd_solve(p, p, 4, 129, p, null, null) == _lib.EINVAL
     assert "factors buffer is required" in lib.m4mr_last_error().decode()
     assert lib.m4mr_spd_solve(p, p, 1 << 31, 65, p, p, null) == _lib.EINVAL
