@@ -204,6 +204,14 @@ __device__ __forceinline__ void block_backward(const float* tiles, int nb, float
   }
 }
 
+// The padding's entries, which the forward substitution leaves at 0 times the
+// system's own (not a number where one of those is infinite): none of it may
+// reach the backward substitution.  One wave.
+__device__ __forceinline__ void clear_padding(float* w, int dim, int nb) {
+  const int l = threadIdx.x & 63;
+  if (dim + l < 16 * nb) w[dim + l] = 0.f;
+}
+
 // L w = b likewise (b in `w` on entry), block rows from the first down.
 __device__ __forceinline__ void block_forward(const float* tiles, int nb, float* w) {
   const int l = threadIdx.x & 63, r = l & 15;
@@ -298,6 +306,7 @@ __global__ __launch_bounds__(64 * NW) void spd_block_kernel(const float* __restr
     __syncthreads();
   }
   if (wave == 0) {
+    clear_padding(w, dim, nb);
     block_backward(tiles, nb, w);
     for (int i = l; i < dim; i += 64) solution[n * dim + i] = w[i];
   }
@@ -329,6 +338,7 @@ __global__ __launch_bounds__(64 * NW) void spd_block_backward_kernel(
   __syncthreads();
   if (wave == 0) {
     block_forward(tiles, nb, z);
+    clear_padding(z, dim, nb);
     block_backward(tiles, nb, z);
   }
   __syncthreads();

@@ -170,3 +170,28 @@ def test_wide_non_definite_system_gives_nan(gpu_lib):
     a = -torch.eye(96, device=dev).expand(2, 96, 96).contiguous()
     y = spd_solve(a, torch.ones(2, 96, device=dev))
     assert torch.isnan(y).all()
+
+
+@pytest.mark.parametrize("dim", [65, 79, 96, 113, 161, 207])
+def test_an_infinite_right_hand_side_stays_its_systems_own(gpu_lib, dim):
+    """The last entry of a solution is its right-hand side's scaled: infinite
+    where that is, at widths that are padded too, and the one before it takes
+    the sign of the factor between them.  The other system is untouched, and so
+    is the gradient of the right-hand side, from finite cotangents."""
+    announce(f"spd_solve, infinite rhs, d={dim}")
+    a, stored, rhs = spd(2, dim, seed=dim)
+    cot = np.random.default_rng(dim).normal(size=rhs.shape)
+    want, _, want_rhs = solve_on_gpu(stored, rhs, cot)
+    lower = np.linalg.cholesky(a[0])
+    rhs[0, -1] = np.inf
+    got, _, d_rhs = solve_on_gpu(stored, rhs, cot)
+    assert got[0, -1] == np.inf
+    assert got[0, -2] == -np.sign(lower[-1, -2]) * np.inf
+    np.testing.assert_array_equal(got[1], want[1])
+    np.testing.assert_array_equal(d_rhs, want_rhs)
+    # The same in the backward's substitutions.
+    cot[0, -1] = -np.inf
+    _, _, d_rhs = solve_on_gpu(stored, np.where(np.isinf(rhs), 1.0, rhs), cot)
+    assert d_rhs[0, -1] == -np.inf
+    assert d_rhs[0, -2] == np.sign(lower[-1, -2]) * np.inf
+    np.testing.assert_array_equal(d_rhs[1], want_rhs[1])
