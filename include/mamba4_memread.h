@@ -461,7 +461,8 @@ int m4mr_spd_solve_backward(const float* factors, const float* solution,
  *          1e-30)), state_all_finite (1 / 0), cross_max_abs, floor_min,
  *          floor_max, in the reference's order.
  * The eigenvalues come from a tridiagonalisation and Sturm counts in float64,
- * one 256-thread block per state, rounded to float32; the
+ * one 256-thread block per state, rounded to float32 (coordinates whose
+ * diagonal lies far above the others' split off first); the
  * reference's eigvalsh (LAPACK on the host, or its TPU lowering) has no
  * counterpart to call on the device.
  */

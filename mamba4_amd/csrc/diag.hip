@@ -9,9 +9,12 @@
 // Numerische Mathematik 9 (1967) 386-393): 64 shifts a round, one per lane,
 // so a round narrows the interval 65 times and ten reach float64.  Both steps
 // are backward stable, as eigvalsh's own; the extremes are then rounded to
-// float32.
+// float32.  Rows and columns are taken in descending order of the diagonal's
+// magnitude, so a coordinate far above the others (a large floor) is split off
+// before it can mix with them, and no tolerance is relative to the largest
+// entry: the small eigenvalues of such a precision keep their own precision.
 //
-// Thread (r, w) holds columns 16w..16w+15 of row r in registers.  A
+// Thread (r, w) holds columns 16w..16w+15 of row r of that order in registers.  A
 // reflection takes a product of the matrix with the vector (16 multiply-adds
 // a thread, the four waves' parts meeting in LDS) and a rank-two update (32),
 // two barriers in all.  Bound by that chain of 62 reflections.  A cyclic
@@ -80,13 +83,14 @@ __device__ __forceinline__ double reciprocal(double q) {
 
 // Eigenvalues below x of the tridiagonal with diagonal d and squared
 // off-diagonal e2 (e2[i] between i and i + 1), n rows: the negative pivots of
-// T - x (a pivot under `tiny` counts as -tiny).
-__device__ __forceinline__ int sturm_count(const double* d, const double* e2, int n, double x,
-                                           double tiny) {
+// T - x (a pivot under kTiny counts as -kTiny: below any float32, and float32's
+// squares over it are finite).
+constexpr double kTiny = 0x1p-700;
+__device__ __forceinline__ int sturm_count(const double* d, const double* e2, int n, double x) {
   int count = 0;
   double q = d[0] - x;
   for (int i = 0;; ++i) {
-    if (fabs(q) < tiny) q = -tiny;
+    if (fabs(q) < kTiny) q = -kTiny;
     count += q < 0.0;
     if (i + 1 == n) return count;
     q = (d[i + 1] - x) - e2[i] * reciprocal(q);
@@ -105,25 +109,38 @@ __global__ __launch_bounds__(256) void diag_eigen_kernel(const float* __restrict
   __shared__ double column[2][64];  // the next column to reduce (double buffered)
   __shared__ double part[4][64];
   __shared__ double diagonal[64], off2[64];
-  __shared__ double wave_squares[4];
+  __shared__ int order[64];
   __shared__ float extreme[2], wave_max_cross[4];
   const int bh = blockIdx.x, h = bh % H, r = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float* E = evidence + (long)bh * D * D;
   bool finite = true, prec_finite = true, cross_nan = false;
+  // order[i]: the row with the i-th largest diagonal magnitude (as ordered bits,
+  // ties by row; rows past D last).
+  const float fl = r < D ? floor[h * D + r] : 0.f;
+  const unsigned key = r < D ? __float_as_uint(fabsf(E[r * D + r] + fl)) : 0u;
+  int rank = 0;
+#pragma unroll
+  for (int j = 0; j < 64; ++j) {
+    const unsigned other = (unsigned)__builtin_amdgcn_readlane((int)key, j);
+    rank += other > key || (other == key && j < r);
+  }
+  if (w == 0) order[rank] = r;
+  __syncthreads();
+  const int pr = order[r];  // below D for r < D
+  const float fr = __shfl(fl, pr);
   double a[16];
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const int c = 16 * w + j;
+    const int c = 16 * w + j, pc = order[c];
     a[j] = 0.0;
     if (r < D && c < D) {
-      const float x = E[r * D + c], y = E[c * D + r];
+      const float x = E[pr * D + pc], y = E[pc * D + pr];
       finite = finite && isfinite(x);
       a[j] = 0.5 * ((double)x + (double)y);
       if (c == r) {
-        const float fl = floor[h * D + r];
-        prec_finite = isfinite(fl);
-        a[j] += (double)fl;
+        prec_finite = isfinite(fr);
+        a[j] += (double)fr;
       }
     }
   }
@@ -138,11 +155,6 @@ __global__ __launch_bounds__(256) void diag_eigen_kernel(const float* __restrict
   }
   cmax = wave_max(cmax);
   if (r == 0) wave_max_cross[w] = cmax;
-  double squares = 0.0;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) squares = __builtin_fma(a[j], a[j], squares);
-  squares = wave_sum(squares);
-  if (r == 0) wave_squares[w] = squares;
   if (w == 0) column[0][r] = a[0];
   // Uniform over the block from here on.
   const bool any_bad_precision = __syncthreads_or(!prec_finite);
@@ -153,11 +165,10 @@ __global__ __launch_bounds__(256) void diag_eigen_kernel(const float* __restrict
   // onto row k + 1.  Rows and columns up to k hold stale values afterwards
   // that nothing reads.
   if (!any_bad_precision) {
-    // A column with less than 2^-70 of the matrix's norm below its first
+    // A column of norm below 2^-300 (nothing beside any float32) under its first
     // entry is reduced already: what is left of a rank-deficient matrix
     // would otherwise shrink by 2^-53 a step until its squares underflow.
-    const double negligible =
-        0x1p-140 * (wave_squares[0] + wave_squares[1] + wave_squares[2] + wave_squares[3]);
+    constexpr double negligible = 0x1p-600;
     for (int k = 0; k < D; ++k) {
       const double x = column[k & 1][r];
       if (w == 0 && r == k) diagonal[k] = x;
@@ -204,15 +215,16 @@ __global__ __launch_bounds__(256) void diag_eigen_kernel(const float* __restrict
         lo = fmin(lo, __shfl_xor(lo, o));
         hi = fmax(hi, __shfl_xor(hi, o));
       }
-      const double size = fmax(fabs(lo), fabs(hi));
-      const double tiny = fmax(size * 0x1p-80, 0x1p-960);
-      lo -= size * 0x1p-48 + tiny;
-      hi += size * 0x1p-48 + tiny;
+      lo -= fabs(lo) * 0x1p-48 + kTiny;
+      hi += fabs(hi) * 0x1p-48 + kTiny;
       const int want = w == 0 ? 1 : D;
-      for (int round = 0; round < 14; ++round) {
-        if (hi - lo <= 0x1p-52 * fmax(fabs(lo), fabs(hi))) break;  // uniform
+      // Ten rounds where the extremes are within some orders of magnitude; the
+      // bound covers float32's whole range (an interval below 2^-170 rounds to
+      // zero).
+      for (int round = 0; round < 60; ++round) {
+        if (hi - lo <= fmax(0x1p-52 * fmax(fabs(lo), fabs(hi)), 0x1p-170)) break;  // uniform
         const double step = (hi - lo) * (1.0 / 65.0), x = lo + step * (r + 1);
-        const unsigned long long at = __ballot(sturm_count(diagonal, off2, D, x, tiny) >= want);
+        const unsigned long long at = __ballot(sturm_count(diagonal, off2, D, x) >= want);
         // The counts grow with the shift (up to rounding): the first lane
         // that reaches the count bounds the eigenvalue from above.
         const int first = at ? __builtin_ctzll(at) : 64;

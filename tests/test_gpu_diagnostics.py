@@ -133,6 +133,34 @@ def test_diagnostics_of_degenerate_spectra(gpu_lib, dim):
             assert abs(got[key] - ref) <= 1.2e-7 * abs(ref) + 1e-13 * size, (i, key, got[key], ref)
 
 
+@pytest.mark.parametrize("dim", [2, 3, 17, 64])
+@pytest.mark.parametrize("large", [1e6, 1e15, 1e30, -1e30])
+def test_diagnostics_beside_a_large_coordinate(gpu_lib, dim, large):
+    """One floor entry far above the rest: the extreme of the other coordinates
+    is that of the precision without it, up to its coupling squared over the
+    large entry (that second-order term included for 1e6), not lost in float64
+    rounding of the large one."""
+    evidence, cross, floor = _known_state(dim, 1, 1, dim, 2, low=1e-2, high=50.0)
+    floor[0, dim // 2] = large
+    announce(f"selective_diagnostics beside {large:g} D={dim}")
+    got = _diagnose(evidence, cross, floor)
+    exact = evidence[0, 0].astype(np.float64)
+    exact = 0.5 * (exact + exact.T) + np.diag(floor[0].astype(np.float64))
+    rest = np.arange(dim) != dim // 2
+    coupling, top = exact[rest, dim // 2], exact[dim // 2, dim // 2]
+    others = np.linalg.eigvalsh(exact[np.ix_(rest, rest)] - np.outer(coupling, coupling) / top)
+    small = others[0] if large > 0 else others[-1]
+    # The Schur complement's eigenvalues are off by its own size squared over the
+    # large entry at most.
+    bound = 2e-7 * abs(small) + 50.0 ** 3 / top ** 2 + 1e-12
+    ends = ("precision_min_eigenvalue", "precision_max_eigenvalue")
+    inner, outer = ends if large > 0 else ends[::-1]
+    assert abs(got[inner] - small) <= bound, (got[inner], small)
+    assert got[outer] == pytest.approx(top, rel=2e-7 + 50.0 ** 2 / top ** 2)
+    if large > 0:
+        assert got["precision_max_condition"] == pytest.approx(top / small, rel=1e-6 + bound / small)
+
+
 def test_diagnostics_rejects_wide_states(gpu_lib):
     from mamba4_amd import SelectiveState, selective_diagnostics
 
