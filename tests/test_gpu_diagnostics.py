@@ -161,6 +161,29 @@ def test_diagnostics_beside_a_large_coordinate(gpu_lib, dim, large):
         assert got["precision_max_condition"] == pytest.approx(top / small, rel=1e-6 + bound / small)
 
 
+@pytest.mark.parametrize("low,high", [(-3, 3), (0, 6), (-5, 5)])
+def test_diagnostics_of_graded_precisions(gpu_lib, low, high):
+    """Well-conditioned matrices scaled per coordinate over many orders of
+    magnitude: the smallest eigenvalue (from the inverse, which the scaling makes
+    accurate in float64) to float32 rounding."""
+    rng = np.random.default_rng(high)
+    for dim in (2, 9, 33, 64):
+        x = rng.normal(size=(dim, 2 * dim))
+        scale = 10.0 ** rng.uniform(low, high, size=dim)
+        evidence = (scale[:, None] * (x @ x.T / (2 * dim)) * scale).astype(np.float32)
+        announce(f"selective_diagnostics graded 1e{low}..1e{high} D={dim}")
+        got = _diagnose(evidence[None, None], np.ones((1, 1, 2, dim), np.float32),
+                        np.zeros(dim, np.float32))
+        exact = evidence.astype(np.float64)
+        exact = 0.5 * (exact + exact.T)
+        root = np.sqrt(np.diag(exact))
+        inverse = np.linalg.inv(exact / root[:, None] / root) / root[:, None] / root
+        smallest = 1.0 / np.linalg.eigvalsh(0.5 * (inverse + inverse.T))[-1]
+        assert got["precision_min_eigenvalue"] == pytest.approx(smallest, rel=1.2e-7)
+        assert got["precision_max_eigenvalue"] == pytest.approx(np.linalg.eigvalsh(exact)[-1],
+                                                                rel=1.2e-7)
+
+
 def test_diagnostics_rejects_wide_states(gpu_lib):
     from mamba4_amd import SelectiveState, selective_diagnostics
 
