@@ -143,28 +143,68 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // Runs of a carry whose loads are issued together.
 constexpr int ORDER_CARRY_BATCH = 16;
 
+// The n-th run a carry comes to: from the first one, or from the last.
+template <bool REVERSE>
+__device__ __forceinline__ int carry_run(const OrderDims& d, int n) {
+  return REVERSE ? d.NR - 1 - n : n;
+}
+
+// A batch of runs' own states of one coordinate and decays (past the last
+// run: that run's again).
+template <bool REVERSE>
+struct CarryBatch {
+  float local[ORDER_CARRY_BATCH], decay[ORDER_CARRY_BATCH];
+  __device__ __forceinline__ void load(const OrderDims& d, const float* states,
+                                       const float* totals, int n0) {
+#pragma unroll
+    for (int j = 0; j < ORDER_CARRY_BATCH; ++j) {
+      const int run = carry_run<REVERSE>(d, min(n0 + j, d.NR - 1));
+      local[j] = states[(long)run * d.W];
+      decay[j] = totals[run];
+    }
+  }
+  // Replaces the states of `count` runs from n0 by the carried ones.
+  __device__ __forceinline__ float apply(const OrderDims& d, float* states, int n0, int count,
+                                         float s) const {
+#pragma unroll
+    for (int j = 0; j < ORDER_CARRY_BATCH; ++j)
+      if (j < count) {
+        states[(long)carry_run<REVERSE>(d, n0 + j) * d.W] = s;
+        s = __builtin_fmaf(decay[j], s, local[j]);
+      }
+    return s;
+  }
+};
+
+// Carries one coordinate's state through a sequence's runs, in place.  Bound
+// by the latency of its loads (few blocks, one dependent fma per run), so a
+// batch is loaded while the one before it is carried; the last, which may be
+// short, leaves the loop, so that no wait in it has to allow for fewer stores.
+template <bool REVERSE>
+__device__ __forceinline__ float carry_runs(const OrderDims& d, float* states,
+                                            const float* totals, float s) {
+  constexpr int N = ORDER_CARRY_BATCH;
+  CarryBatch<REVERSE> a, b;
+  a.load(d, states, totals, 0);
+  for (int n0 = 0;; n0 += 2 * N) {
+    b.load(d, states, totals, n0 + N);
+    if (n0 + N > d.NR) return a.apply(d, states, n0, d.NR - n0, s);
+    s = a.apply(d, states, n0, N, s);
+    a.load(d, states, totals, n0 + 2 * N);
+    if (n0 + 2 * N > d.NR) return b.apply(d, states, n0 + N, d.NR - n0 - N, s);
+    s = b.apply(d, states, n0 + N, N, s);
+  }
+}
+
 // Forward pass 2, grid B*H: turns ends into the state each run starts from
 // (in place), starting from `initial`.
 __global__ __launch_bounds__(256) void order_carry_kernel(OrderDims d, const float* initial,
                                                           float* ends, const float* totals) {
-  const int bh = blockIdx.x, c = threadIdx.x;
+  const long bh = blockIdx.x;
+  const int c = threadIdx.x;
   if (c >= d.W) return;
-  float s = initial ? initial[(long)bh * d.W + c] : 0.f;
-  for (int n0 = 0; n0 < d.NR; n0 += ORDER_CARRY_BATCH) {
-    float local[ORDER_CARRY_BATCH], decay[ORDER_CARRY_BATCH];
-#pragma unroll
-    for (int j = 0; j < ORDER_CARRY_BATCH; ++j) {
-      const long slot = (long)bh * d.NR + min(n0 + j, d.NR - 1);
-      local[j] = ends[slot * d.W + c];
-      decay[j] = totals[slot];
-    }
-#pragma unroll
-    for (int j = 0; j < ORDER_CARRY_BATCH; ++j)
-      if (n0 + j < d.NR) {
-        ends[((long)bh * d.NR + n0 + j) * d.W + c] = s;
-        s = __builtin_fmaf(decay[j], s, local[j]);
-      }
-  }
+  carry_runs<false>(d, ends + bh * d.NR * d.W + c, totals + bh * d.NR,
+                    initial ? initial[bh * d.W + c] : 0.f);
 }
 
 // Forward pass 3: each run's scan from its start state.
@@ -238,25 +278,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 __global__ __launch_bounds__(256) void order_bwd_carry_kernel(OrderDims d, float* heads,
                                                               const float* totals,
                                                               float* d_initial) {
-  const int bh = blockIdx.x, c = threadIdx.x;
+  const long bh = blockIdx.x;
+  const int c = threadIdx.x;
   if (c >= d.W) return;
-  float s = 0.f;
-  for (int top = d.NR; top > 0; top -= ORDER_CARRY_BATCH) {
-    float local[ORDER_CARRY_BATCH], decay[ORDER_CARRY_BATCH];
-#pragma unroll
-    for (int j = 0; j < ORDER_CARRY_BATCH; ++j) {
-      const long slot = (long)bh * d.NR + max(top - 1 - j, 0);
-      local[j] = heads[slot * d.W + c];
-      decay[j] = totals[slot];
-    }
-#pragma unroll
-    for (int j = 0; j < ORDER_CARRY_BATCH; ++j)
-      if (top - 1 - j >= 0) {
-        heads[((long)bh * d.NR + top - 1 - j) * d.W + c] = s;
-        s = __builtin_fmaf(decay[j], s, local[j]);
-      }
-  }
-  if (d_initial) d_initial[(long)bh * d.W + c] = s;
+  const float s = carry_runs<true>(d, heads + bh * d.NR * d.W + c, totals + bh * d.NR, 0.f);
+  if (d_initial) d_initial[bh * d.W + c] = s;
 }
 
 constexpr int ORDER_MAX_WAVES = 4;  // W <= 256
