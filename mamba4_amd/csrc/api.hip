@@ -1564,8 +1564,12 @@ int m3_groups(int B, int T, int H) {
 // 0.033 per sequence and chunk.  Forward + backward, walk against split: B1
 // T1000 H24 77 + 77 / 31 + 21 us, B4 T1024 H24 80 + 79 / 67 + 56, B8 T1024 H24
 // 102 + 100 / 118 + 107, B1 T128 H2 13 + 12 / 16 + 13.  The split is taken
-// where it is estimated 10% faster.
+// where it is estimated 10% faster, and from five chunks on: up to four the
+// walk ends within the time the host takes for the call, to which the split
+// adds two launches (forward alone, end to end, B1 H4: T256 31 walked, 36
+// split; T320 35, 36; T512 47, 36).
 bool m3_split_walk(int B, int H, int NC) {
+  if (NC <= 4) return false;
   if (NC > 65535) return false;  // a grid dimension
   const double blocks = 2.0 * B * H, cus = compute_units();
   const double step = blocks <= cus ? 4.7 : blocks <= 2 * cus ? 6.1 : 8.1;

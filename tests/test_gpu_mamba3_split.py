@@ -65,3 +65,32 @@ def test_split_states_match_the_walk(gpu_lib, time, state, width, angles, dtype,
             assert (a - b).norm() <= tolerance * a.norm(), name
         else:
             assert torch.equal(a[row], b[0]), name
+
+
+# A call of up to four chunks is bound by its launches: one walk, not three.
+@pytest.mark.parametrize("time,split", [(1, False), (192, False), (256, False), (257, True)])
+def test_short_sequences_are_walked(gpu_lib, time, split):
+    from mamba4_amd import _lib, mamba3_fused
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(time)
+
+    def normal(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen)
+
+    heads, state, width, angles = 4, 128, 64, 32
+    announce(f"Mamba-3 short sequence T={time}")
+    _lib.profile_reset()
+    _lib.profile_select(None)
+    _lib.profile_enable(True)
+    try:
+        mamba3_fused(normal(1, time, state), normal(1, time, state), normal(1, time, heads * width),
+                     -normal(1, time, heads).abs(), normal(1, time, heads).abs(),
+                     normal(1, time, heads), normal(1, time, angles),
+                     q_bias=normal(heads, 1, state), k_bias=normal(heads, 1, state))
+        torch.cuda.synchronize()
+    finally:
+        _lib.profile_enable(False)
+    launches = [_lib.profile_read(n)[1] for n in ("m3_walk", "m3_local", "m3_carry")]
+    _lib.profile_reset()
+    assert launches == ([0, 1, 1] if split else [1, 0, 0])
