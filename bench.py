@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Memory-read fwd+bwd benchmark on one MI355X (BASELINE.json metric).
+"""Memory-read fwd+bwd benchmark on one MI355X.
 
 A step is one forward (chunk states, per-token factor + solve + factor
 store, reads) and one backward (dy, factored re-solve, reverse carry,
@@ -19,12 +19,12 @@ with vs_baseline against its TPU v4 figure (67.98 ms,
 lm/results/speed-125m/bench-kernels.json:291).
 
 With --workload config4 a step is instead one in-place decode step of
-2048 sequences x 8 heads of resident (S, C) states (BASELINE config 4): the
+2048 sequences x 8 heads of resident (S, C) states: the
 states are the end states of a 1024-token gated recurrence with
 lambda = sigmoid(N(3,1)), built by this library's own forward, and each step
 writes one new token into every state, refactors and reads.
 
-With --workload config3 the step is the same fwd+bwd at BASELINE config 3
+With --workload config3 the step is the same fwd+bwd at a larger batch
 (B=32, L=1024, H=12, slow decay) with bfloat16 keys, values and queries
 read natively by the kernels (m4mr_forward_bf16 / m4mr_backward_bf16).
 
@@ -950,7 +950,7 @@ def oracle_legs(data):
 
 
 def cpu_baseline(data, workload, config0=True):
-    """The CPU baseline of the plan in BASELINE.md: this build's NumPy
+    """The CPU baseline: the oracle's NumPy
     restatement of the reference algorithm (oracle.memread, float32) on this
     host, BLAS on every core, one warm-up then the median of five runs,
     forward and forward+backward.  Config 0 runs in full.  The benchmarked

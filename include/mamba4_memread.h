@@ -350,8 +350,8 @@ int m4mr_backward_bf16_to_bf16(const uint16_t* keys, const uint16_t* values, con
  * runtime-provided scratch either: it takes the backward state walk that
  * spills no registers, whatever the batch size or M4MR_STATE_BUFFERS.
  * Sizes whose m4mr_backward_workspace_bytes exceeds it return M4MR_EINVAL
- * before any launch (128 MiB holds B*T*H = 131072 token-heads at P = 64,
- * BASELINE config 2, with room to spare).  Every call on one GPU shares that
+ * before any launch (128 MiB holds B*T*H = 131072 token-heads at P = 64
+ * with room to spare).  Every call on one GPU shares that
  * GPU's buffer: calls that overlap on one GPU (on different streams, or from
  * different threads without ordering) race and must not be issued.  Every
  * other argument and every result as in m4mr_backward (float32 keys, values

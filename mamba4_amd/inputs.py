@@ -116,7 +116,7 @@ def device_tokens(gen, shape, shift, decay_mean=3.0):
 
 
 def decode_states(batch=2048, heads=8, context=1024, seed=0, slice_rows=128, keep_rows=()):
-    """BASELINE config 4's resident states on cuda:0: the end states (S, C)
+    """Resident decode states on cuda:0: the end states (S, C)
     [batch, heads, 64, 64] of a ``context``-token gated recurrence with
     config-0 distributions and lambda = sigmoid(N(3,1)) (``device_tokens``),
     built slice by slice with this library's forward, which stores no factors

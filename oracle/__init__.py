@@ -1,6 +1,6 @@
 """CPU oracle for the Mamba 4 memory read -- TEST INFRASTRUCTURE ONLY.
 
-This package is the checker for the MI355X HIP implementation in
+This package is the oracle for the MI355X HIP implementation in
 ``mamba4_amd``.  Only ``tests/``, ``__graft_entry__.smoke()`` and the
 ``cpu_baseline`` leg of ``bench.py`` may import it, and only to check or to
 time the CPU restatement.  The product path never calls it; the HIP library

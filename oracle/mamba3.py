@@ -1,7 +1,7 @@
 """Float64 restatement of the FlashMamba Mamba-3 SISO scan.
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, ``__graft_entry__.smoke()`` and
-``bench.py``'s CPU baseline as the checker; the product path never calls it.
+``bench.py``'s CPU baseline as the oracle; the product path never calls it.
 
 The operator is ``mamba3_fused`` (lm/kernels/flashmamba.py:1125-1162) over
 ``fused_scan`` (:901-957): one shared query row c_t and key row b_t per token

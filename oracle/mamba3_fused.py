@@ -2,7 +2,7 @@
 model-dtype rounding of their matrix operands.
 
 TEST INFRASTRUCTURE ONLY: imported by tests/ and ``bench.py``'s CPU
-baseline as the checker; the product path never calls it.
+baseline as the oracle; the product path never calls it.
 
 The reference's fused forward and backward kernels
 (lm/kernels/flashmamba.py:589-660 and :663-786) multiply matrix operands in

@@ -1,7 +1,7 @@
 """NumPy restatement of the Mamba 4 memory read -- TEST INFRASTRUCTURE ONLY.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and ``bench.py``'s
-``cpu_baseline`` leg may import this module, as the checker of the HIP
+``cpu_baseline`` leg may import this module, as the oracle of the HIP
 library; the product path never routes through it.
 
 Operator (per batch row b and head h; D = key width, P = value width)::

@@ -2,7 +2,7 @@
 INFRASTRUCTURE ONLY.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and ``bench.py``'s
-``cpu_baseline`` leg may import this module, as the checker of the HIP
+``cpu_baseline`` leg may import this module, as the oracle of the HIP
 library; the product path never routes through it.
 
 The memory read's caller (``SelectiveMemoryMixer.__call__``,

@@ -2,7 +2,7 @@
 INFRASTRUCTURE ONLY.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and ``bench.py``'s
-``cpu_baseline`` leg may import this module, as the checker of the HIP
+``cpu_baseline`` leg may import this module, as the oracle of the HIP
 library; the product path never routes through it.
 
 The memory mixer's order head (lm/models/mamba4.py:274-289) runs, per batch
@@ -16,7 +16,7 @@ from ``h_(-1) = 0``.  Restated here in float64:
   with inflow ``1 - lam = -expm1(log lam)``, chunk ends combined by the
   decayed carry of lm/kernels/prefix.py:27-44, each chunk's reads taking
   ``exp(prefix)`` times the state it starts from.  ``initial`` (an addition
-  of this build) is the state before the first token; the reference's cached
+  of this framework) is the state before the first token; the reference's cached
   decode step (lm/models/mamba4.py:283-287) is this scan over one token from
   the cached state.
 * ``order_memory_backward``: the closed-form VJP of the chunked scan with

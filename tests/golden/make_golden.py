@@ -1,4 +1,4 @@
-"""Write tests/golden/config0.npz: BASELINE config 0 inputs with float64
+"""Write tests/golden/config0.npz: config 0's inputs with float64
 oracle outputs, final state and every gradient.
 
 Config 0 (B=2, L=256, H=1, D=P=64, seed 0, floor 1e-2, shifted unit keys,

@@ -1,4 +1,4 @@
-"""Full-size BASELINE configurations on the GPU.
+"""The full-size configurations on the GPU.
 
 The HIP path runs the whole workload; the float64 oracle checks a subset of
 batch rows (rows are independent sequences), and size-independent
@@ -12,7 +12,7 @@ properties are checked on every row:
 * a one-row slice run on its own reproduces that row of the full batch
   bit for bit (rows share no state), whichever forms the two batch sizes take.
 Tolerance: normwise max|d| / max|ref| <= 1e-4 on outputs, <= 1e-3 on
-gradients (BASELINE.json north_star).
+gradients.
 """
 
 import numpy as np

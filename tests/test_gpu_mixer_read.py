@@ -3,8 +3,7 @@ into one pass (lm/models/mamba4.py:183-273 without the projections and the
 order head).
 
 The fused op is checked against the composed float64 oracle (oracle.mixer
-around oracle.memread: outputs normwise <= 1e-4, gradients <= 1e-3, the
-north-star tolerances) and against the separate kernels (memory_inputs ->
+around oracle.memread: outputs normwise <= 1e-4, gradients <= 1e-3) and against the separate kernels (memory_inputs ->
 selective_gaussian_memory -> gated_read) on the same state walk: the read
 kernel and the state walk normalise each key and query row with the
 prologue kernel's own arithmetic, the factor kernel sums a row's squares in

@@ -5,7 +5,7 @@ Tolerances (fp32 HIP vs float64 oracle):
   values rtol 3e-5 / atol 3e-6 (lm/tests/test_mamba4.py:43), gradients
   rtol 2e-4 / atol 2e-5 (:103, :404);
 * benchmark configs (floor 1e-2): normwise max|d| / max|ref| <= 1e-4 on
-  outputs and state, <= 1e-3 on gradients (BASELINE.json north_star).
+  outputs and state, <= 1e-3 on gradients.
 """
 
 import ctypes
@@ -214,7 +214,7 @@ def test_nonpositive_floor_propagates_nan(gpu_lib):
 
 def decode_problem(batch=4, heads=8, seed=21, steps=1):
     """Resident states after a 96-token prefill (slow decay, floor 1e-2),
-    then `steps` new tokens, as BASELINE config 4 at a small batch."""
+    then `steps` new tokens, as the decode configuration at a small batch."""
     from mamba4_amd.inputs import synthetic_inputs
 
     pre = synthetic_inputs(batch, 96 + steps, heads, decay_mean=3.0, seed=seed)

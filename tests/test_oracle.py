@@ -1,4 +1,4 @@
-"""Pins the CPU oracle before it is trusted as the checker of the HIP path.
+"""Pins the CPU oracle before it is trusted to check the HIP path.
 
 The reference holds no golden vectors for the memory read; every oracle
 function is pinned here by the reference's own known answers and
